@@ -1109,7 +1109,7 @@ int op_apply_internal(const ck_op* op, int nrhs, const float* X, int64_t ldx, fl
     case CK_OP_WOODBURY_INV:
       return woodbury_apply(op, nrhs, X, ldx, Y, ldy, work, work_bytes, done, s);
     case CK_OP_RBF_F32:
-      return rbf_apply(op, nrhs, X, ldx, Y, ldy, done, s);
+      return rbf_apply(op, nrhs, X, ldx, Y, ldy, work, work_bytes, done, s);
     case CK_OP_KRON_EIG_F32:
       if (!kron64_eligible(op, X, ldx, Y, ldy)) return CK_ERR_UNSUPPORTED;
       return kron64_eig_apply_f32(op, nrhs, X, ldx, Y, ldy, work, work_bytes, done, s);
@@ -1134,6 +1134,8 @@ size_t op_workspace_internal(const ck_op* op, int nrhs) {
         return dense_sym_offset(op->n, nrhs) + sym_scratch_bytes(op->n);
       // room for the p.Ap partials a CG step takes from the matvec epilogue (dense_apply_xy)
       return (nrhs >= 3 && nrhs <= 8) ? dense_xy_bytes(op->n, nrhs) : 0;
+    case CK_OP_RBF_F32:
+      return rbf_workspace_bytes(op, nrhs);
     case CK_OP_CSR_F32:
       // the x.Ax partials of csr_apply_xy (CG's p.Ap, Lanczos's v.Av)
       return csr_xy_bytes(op->n, nrhs);

@@ -55,7 +55,8 @@ inline size_t dense_sym_offset(int64_t n, int nrhs) {
   const size_t a = dense_xy_bytes(n, nrhs), b = wb_fused_bytes(n, nrhs, 64);
   return ((a > b ? a : b) + 255) / 256 * 256;
 }
-int rbf_apply(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, const int* done,
-              hipStream_t s);
+int rbf_apply(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, void* work,
+              size_t work_bytes, const int* done, hipStream_t s);
+size_t rbf_workspace_bytes(const ck_op* op, int nrhs);
 
 }  // namespace ck

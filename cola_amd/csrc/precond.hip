@@ -1,4 +1,4 @@
-// Low-rank (Woodbury) inverse application and the on-the-fly RBF kernel operator.
+// Low-rank (Woodbury) inverse application.
 //
 // Woodbury: (s I + F F^T)^{-1} x = (x - F (s I + F^T F)^{-1} F^T x) / s with the
 // small core inverse precomputed (rank x rank, fp64).  All arithmetic after the
@@ -8,10 +8,6 @@
 // (128 rows at rank 64) in LDS with coalesced loads and serve up to 8 rhs from it:
 // F^T x gives one fp64 partial per tile (added in index order), the core product
 // u = C^-1 t runs once per rhs, and the update re-reads F once more.
-//
-// RBF: S_ij = exp(-|p_i - p_j|^2 / (2 l^2)) is never stored; each block stages
-// 256 points and their x values in LDS and every lane accumulates one row
-// (compute bound: one exp per pair).
 #include "common.hpp"
 #include "ops_internal.hpp"
 
@@ -154,73 +150,6 @@ __global__ __launch_bounds__(256) void wb_apply_tiles(int64_t n, int k, const fl
   }
 }
 
-constexpr int kRbfTile = 256;
-constexpr int kRbfMaxDim = 8;
-constexpr int kRbfNB = 8;
-
-// the stationary kernel k(d2) for d2 = |p_i - p_j|^2: FAMILY 0 exp(-d2 / (2 l^2)) (RBF),
-// 1 exp(-r / l) (Matern 1/2), 2 (1 + a) exp(-a) with a = sqrt(3) r / l (Matern 3/2),
-// 3 (1 + a + a^2 / 3) exp(-a) with a = sqrt(5) r / l (Matern 5/2)
-template <int FAMILY>
-__device__ __forceinline__ float stationary(float d2, float inv2l2, float inv_l) {
-  if (FAMILY == 0) return expf(-d2 * inv2l2);
-  const float r = sqrtf(d2);
-  if (FAMILY == 1) return expf(-r * inv_l);
-  if (FAMILY == 2) {
-    const float a = 1.7320508075688772f * r * inv_l;
-    return (1.f + a) * expf(-a);
-  }
-  const float a = 2.23606797749979f * r * inv_l;
-  return (1.f + a + a * a * (1.f / 3.f)) * expf(-a);
-}
-
-template <int FAMILY>
-__global__ __launch_bounds__(256) void rbf_kernel(int n, int dim, const float* __restrict__ P, int64_t ldp,
-                                                  float inv2l2, float inv_l, const float* __restrict__ X,
-                                                  int64_t ldx, float* __restrict__ Y, int64_t ldy, int nrhs,
-                                                  float scale, float shift, const int* __restrict__ done) {
-  if (done && *done) return;
-  __shared__ float pj[kRbfTile][kRbfMaxDim];
-  __shared__ float xj[kRbfNB][kRbfTile];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int b0 = blockIdx.y * kRbfNB;
-  const int nb = nrhs - b0 < kRbfNB ? nrhs - b0 : kRbfNB;
-  float pi[kRbfMaxDim];
-#pragma unroll
-  for (int d = 0; d < kRbfMaxDim; ++d) pi[d] = (i < n && d < dim) ? P[(int64_t)i * ldp + d] : 0.f;
-  float acc[kRbfNB];
-#pragma unroll
-  for (int b = 0; b < kRbfNB; ++b) acc[b] = 0.f;
-  for (int j0 = 0; j0 < n; j0 += kRbfTile) {
-    __syncthreads();
-    {
-      const int j = j0 + threadIdx.x;
-#pragma unroll
-      for (int d = 0; d < kRbfMaxDim; ++d) pj[threadIdx.x][d] = (j < n && d < dim) ? P[(int64_t)j * ldp + d] : 0.f;
-#pragma unroll
-      for (int b = 0; b < kRbfNB; ++b) xj[b][threadIdx.x] = (j < n && b < nb) ? X[(int64_t)(b0 + b) * ldx + j] : 0.f;
-    }
-    __syncthreads();
-    const int jn = n - j0 < kRbfTile ? n - j0 : kRbfTile;
-    for (int jj = 0; jj < jn; ++jj) {
-      float d2 = 0.f;
-#pragma unroll
-      for (int d = 0; d < kRbfMaxDim; ++d) {
-        const float df = pi[d] - pj[jj][d];
-        d2 = fmaf(df, df, d2);
-      }
-      const float kv = stationary<FAMILY>(d2, inv2l2, inv_l);
-#pragma unroll
-      for (int b = 0; b < kRbfNB; ++b) acc[b] = fmaf(kv, xj[b][jj], acc[b]);
-    }
-  }
-  if (i >= n) return;
-  for (int b = 0; b < nb; ++b) {
-    const float x = X[(int64_t)(b0 + b) * ldx + i];
-    Y[(int64_t)(b0 + b) * ldy + i] = fmaf(shift, x, scale * acc[b]);
-  }
-}
-
 }  // namespace
 
 namespace ck {
@@ -262,36 +191,6 @@ int woodbury_apply(const ck_op* op, int nrhs, const float* X, int64_t ldx, float
   for (int b0 = 0; b0 < nrhs; b0 += kWRhs)
     hipLaunchKernelGGL(wb_apply_tiles, dim3(P), dim3(256), 0, s, n, k, F, op->lda, (const double*)u, X, ldx, Y, ldy,
                        nrhs, b0, (double)op->scale, (double)op->shift, done);
-  CK_CHECK_LAUNCH();
-  return CK_OK;
-}
-
-int rbf_apply(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, const int* done,
-              hipStream_t s) {
-  if (!op->a || op->dim < 1 || op->dim > kRbfMaxDim || op->lda < op->dim || !(op->aux_f > 0.f) || op->rank < 0 ||
-      op->rank > 3)
-    return CK_ERR_BAD_ARG;
-  const float inv2l2 = 1.f / (2.f * op->aux_f * op->aux_f), inv_l = 1.f / op->aux_f;
-  const dim3 grid((unsigned)cdiv(op->n, 256), (unsigned)cdiv(nrhs, kRbfNB));
-  const float* P = static_cast<const float*>(op->a);
-#define CK_RBF(F_)                                                                                               \
-  hipLaunchKernelGGL(rbf_kernel<F_>, grid, dim3(256), 0, s, op->n, op->dim, P, op->lda, inv2l2, inv_l, X, ldx, Y, \
-                     ldy, nrhs, op->scale, op->shift, done)
-  switch (op->rank) {
-    case 0:
-      CK_RBF(0);
-      break;
-    case 1:
-      CK_RBF(1);
-      break;
-    case 2:
-      CK_RBF(2);
-      break;
-    default:
-      CK_RBF(3);
-      break;
-  }
-#undef CK_RBF
   CK_CHECK_LAUNCH();
   return CK_OK;
 }
