@@ -54,6 +54,21 @@ __device__ inline double column_total(const float* __restrict__ part, int P, int
   return wave_sum(acc);
 }
 
+// The same by all 256 threads of a block (thread t adds partials t, t + 256, ...), for consumers that
+// need one column per block: a CSR product leaves up to 2048 partials.  `lds`: four doubles.
+__device__ inline double column_total_block(const float* __restrict__ part, int P, int b, double* lds) {
+  const float* pb = part + (int64_t)b * P;
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < P; i += 2048) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = pb[i + 256 * k < P ? i + 256 * k : P - 1];  // clamped, dropped below
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc += i + 256 * k < P ? (double)v[k] : 0.0;
+  }
+  return block_sum<256>(acc, lds);
+}
+
 // -------------------------------------------------------------- generic partial sums
 // mode 0: sum x*y ; mode 1: sum x*x
 template <int MODE>
@@ -186,24 +201,18 @@ __global__ __launch_bounds__(256) void update_xr_kernel(int64_t n, const float* 
   CgView v = view(state, nrhs);
   if (v.ctrl->done) return;
   __shared__ float red[4];
-  __shared__ float alpha_s;
+  __shared__ double dred[4];
   const int b = blockIdx.y, blk = blockIdx.x;
-  if (threadIdx.x < 64) {
-    const double pap = column_total(part0, np0, b);
-    if (threadIdx.x == 0) {
-      double a = safe_div((double)v.gamma[b], pap);
-      const bool frozen = (double)v.rnorm[b] < kSmall;
-      if (frozen) a = 0.0;  // has_converged (cg.py:143-144,161)
-      alpha_s = (float)a;
-      if (blk == 0) {
-        v.alpha[b] = (float)a;
-        // the reference divides on regardless; the status records it (same value from every writer)
-        if (!frozen && !(pap > 0.0) && v.ctrl->status == CK_OK) v.ctrl->status = CK_ERR_BREAKDOWN;
-      }
-    }
+  const double pap = column_total_block(part0, np0, b, dred);
+  double a = safe_div((double)v.gamma[b], pap);
+  const bool frozen = (double)v.rnorm[b] < kSmall;
+  if (frozen) a = 0.0;  // has_converged (cg.py:143-144,161)
+  const float alpha = (float)a;
+  if (blk == 0 && threadIdx.x == 0) {
+    v.alpha[b] = alpha;
+    // the reference divides on regardless; the status records it (same value from every writer)
+    if (!frozen && !(pap > 0.0) && v.ctrl->status == CK_OK) v.ctrl->status = CK_ERR_BREAKDOWN;
   }
-  __syncthreads();
-  const float alpha = alpha_s;
   const int64_t i0 = blk * per;
   const int64_t i1 = i0 + per < n ? i0 + per : n;
   float* xb = x + b * ld;
@@ -255,18 +264,14 @@ __global__ __launch_bounds__(256) void update_x64_kernel(int64_t n, const float*
                                                          void* state, int nrhs) {
   CgView v = view(state, nrhs);
   const bool stopped = v.ctrl->done != 0;
-  __shared__ float alpha_s;
+  __shared__ double dred[4];
   const int b = blockIdx.y, blk = blockIdx.x;
-  if (!stopped && threadIdx.x < 64) {
-    const double pap = column_total(part0, np0, b);
-    if (threadIdx.x == 0) {
-      double a = safe_div((double)v.gamma[b], pap);
-      if ((double)v.rnorm[b] < kSmall) a = 0.0;
-      alpha_s = (float)a;
-    }
+  float alpha = 0.f;
+  if (!stopped) {  // uniform over the block
+    double a = safe_div((double)v.gamma[b], column_total_block(part0, np0, b, dred));
+    if ((double)v.rnorm[b] < kSmall) a = 0.0;
+    alpha = (float)a;
   }
-  __syncthreads();
-  const float alpha = stopped ? 0.f : alpha_s;
   const float m = v.mult[b];
   const int64_t i0 = blk * per;
   const int64_t i1 = i0 + per < n ? i0 + per : n;
@@ -831,10 +836,10 @@ int cg_iterate(const ck_op* A, const ck_op* P, int32_t nrhs, float* x, float* r,
   const bool dense_xy = !fuse_kron && !fuse_wb && A->kind == CK_OP_DENSE_F32 && nrhs >= 3 && nrhs <= 8 && work &&
                         work_bytes >= dense_xy_bytes(n, nrhs) && n % 4 == 0 && A->lda % 4 == 0 && ld % 4 == 0 &&
                         (reinterpret_cast<uintptr_t>(A->a) & 15) == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
-  // CSR A (rows of at most 32 entries on average): p.Ap partials from the SpMV's epilogue, into
+  // CSR A: p.Ap partials from the SpMV's epilogue, into
   // the head of the workspace like dense_xy
   const bool csr_xy = !fuse_kron && !fuse_wb && !dense_xy && A->kind == CK_OP_CSR_F32 && work &&
-                      work_bytes >= csr_xy_bytes(n, nrhs) && (double)A->nnz <= 32.0 * (double)n;
+                      work_bytes >= csr_xy_bytes(A, nrhs);
   WbFused W{};
   if (fuse_wb) W = wb_fused_carve(work, n, nrhs, P->rank);
   for (int it = 0; it < nsteps; ++it) {
@@ -890,9 +895,9 @@ int cg_iterate(const ck_op* A, const ck_op* P, int32_t nrhs, float* x, float* r,
       st = dense_apply_xy(A, nrhs, p, ld, Ap, ld, done, static_cast<float*>(work), work, work_bytes, s);
       if (st) return st;
     } else if (csr_xy) {
-      np0 = csr_xy_nparts(n);
+      np0 = csr_xy_nparts(A);
       part0 = static_cast<const float*>(work);
-      st = csr_apply_xy(A, nrhs, p, ld, Ap, ld, done, static_cast<float*>(work), s);
+      st = csr_apply_xy(A, nrhs, p, ld, Ap, ld, done, static_cast<float*>(work), work, work_bytes, s);
       if (st) return st;
     } else {
       st = op_apply_internal(A, nrhs, p, ld, Ap, ld, work, work_bytes, done, s);

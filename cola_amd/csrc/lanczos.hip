@@ -1101,17 +1101,17 @@ int ck_lanczos_post(int64_t n, int32_t nb, int32_t max_iters, float* V, int64_t 
 namespace {
 
 // w = A v_i for the nb probes (vector stride ldb); where the operator's kernel has an x . y
-// epilogue (CSR with short rows, 3-factor Kronecker) it also returns the v_i . w partials it
+// epilogue (CSR, 3-factor Kronecker) it also returns the v_i . w partials it
 // wrote (*xy, *pxy per probe) so the step needs no tile_partials pass
 int lz_matvec(const ck_op* A, int nb, const float* vi, float* w, int64_t ldb, void* work, size_t work_bytes,
               const int* done, const LzScratch& sc, const float** xy, int* pxy, hipStream_t s) {
   *xy = nullptr;
   *pxy = 0;
   const int64_t n = A->n;
-  if (A->kind == CK_OP_CSR_F32 && work && work_bytes >= csr_xy_bytes(n, nb) && (double)A->nnz <= 32.0 * (double)n) {
-    if (int st = csr_apply_xy(A, nb, vi, ldb, w, ldb, done, static_cast<float*>(work), s)) return st;
+  if (A->kind == CK_OP_CSR_F32 && work && work_bytes >= csr_xy_bytes(A, nb)) {
+    if (int st = csr_apply_xy(A, nb, vi, ldb, w, ldb, done, static_cast<float*>(work), work, work_bytes, s)) return st;
     *xy = static_cast<const float*>(work);
-    *pxy = csr_xy_nparts(n);
+    *pxy = csr_xy_nparts(A);
     return CK_OK;
   }
   if (A->kind == CK_OP_KRON_F32 && A->nfactors == 3) {

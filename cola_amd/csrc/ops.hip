@@ -699,36 +699,13 @@ int dense_dispatch(const ck_op* op, int nrhs, const float* X, int64_t ldx, float
 }
 
 // ============================================================== CSR
-__global__ __launch_bounds__(256) void csr_wave_per_row(int n, const int32_t* __restrict__ rowptr,
-                                                        const int32_t* __restrict__ colind,
-                                                        const float* __restrict__ val, const float* __restrict__ X,
-                                                        int64_t ldx, float* __restrict__ Y, int64_t ldy, int nrhs,
-                                                        float scale, float shift, const int* __restrict__ done) {
-  if (done && *done) return;
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
-  if (row >= n) return;
-  const int k0 = rowptr[row], k1 = rowptr[row + 1];
-  for (int b = 0; b < nrhs; ++b) {
-    const float* xb = X + b * ldx;
-    float acc = 0.f;
-    for (int k = k0 + lane; k < k1; k += 64) acc = fmaf(val[k], xb[colind[k]], acc);
-    acc = wave_sum(acc);
-    if (lane == 0) {
-      float y = scale * acc;
-      if (shift != 0.f) y = fmaf(shift, xb[row], y);
-      Y[b * ldy + row] = y;
-    }
-  }
-}
-
-// Short rows: one lane per row.  A row of at most kCsrShort nonzeros is loaded into
-// registers in one batch (column indices and values, then the x gathers of NB vectors),
-// so each lane waits for memory twice per NB vectors instead of once per nonzero; the
-// matrix is read once for all vectors.  Longer rows take a plain loop.  Every row is
-// summed k ascending with one fma per nonzero, in both paths, so results do not depend
-// on the path or on the vector count.
-constexpr int kCsrShort = 8;
+// Rows of up to 8 entries on average: one lane per row.  A row of at most eight entries is loaded
+// into registers in one batch (column indices and values, then the x gathers of NB vectors), so
+// each lane waits for memory twice per NB vectors instead of once per nonzero; the matrix is read
+// once for all vectors.  Longer rows go through the same batches NB vectors at a time.  Every row is
+// summed k ascending with one fma per nonzero, in both paths, so results do not depend on the path
+// or on the vector count.
+constexpr int kCsrBatch = 8;
 
 // XY: also xy_part[b * gridDim.x + block] = sum over the block's rows of X[b][row] Y[b][row] (a
 // Krylov step's x . Ax from the matvec itself, instead of a separate pass over both vectors).
@@ -747,20 +724,20 @@ __global__ __launch_bounds__(XY ? 1024 : 256) void csr_lane_per_row(int n, const
   const int rc = row < n ? row : n - 1;  // XY: rows past n compute a copy of row n - 1 and store nothing
   const int k0 = rowptr[rc], k1 = rowptr[rc + 1];
   const int len = k1 - k0;
-  if (len <= kCsrShort) {
-    int c[kCsrShort];
-    float v[kCsrShort];
+  if (len <= kCsrBatch) {
+    int c[kCsrBatch];
+    float v[kCsrBatch];
 #pragma unroll
-    for (int i = 0; i < kCsrShort; ++i) {
+    for (int i = 0; i < kCsrBatch; ++i) {
       c[i] = i < len ? colind[k0 + i] : rc;
       v[i] = i < len ? val[k0 + i] : 0.f;
     }
     for (int b0 = 0; b0 < nrhs; b0 += NB) {
-      float xv[NB][kCsrShort];
+      float xv[NB][kCsrBatch];
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int i = 0; i < kCsrShort; ++i)
+        for (int i = 0; i < kCsrBatch; ++i)
           xv[j][i] = (i < len && b0 + j < nrhs) ? X[(int64_t)(b0 + j) * ldx + c[i]] : 0.f;
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
@@ -768,7 +745,7 @@ __global__ __launch_bounds__(XY ? 1024 : 256) void csr_lane_per_row(int n, const
         if (b >= nrhs) break;
         float acc = 0.f;
 #pragma unroll
-        for (int i = 0; i < kCsrShort; ++i)
+        for (int i = 0; i < kCsrBatch; ++i)
           if (i < len) acc = fmaf(v[i], xv[j][i], acc);
         float y = scale * acc;
         if (shift != 0.f) y = fmaf(shift, X[(int64_t)b * ldx + rc], y);
@@ -776,13 +753,37 @@ __global__ __launch_bounds__(XY ? 1024 : 256) void csr_lane_per_row(int n, const
       }
     }
   } else {
-    for (int b = 0; b < nrhs; ++b) {
-      const float* xb = X + (int64_t)b * ldx;
-      float acc = 0.f;
-      for (int k = k0; k < k1; ++k) acc = fmaf(val[k], xb[colind[k]], acc);
-      float y = scale * acc;
-      if (shift != 0.f) y = fmaf(shift, xb[rc], y);
-      if (!XY || row < n) Y[(int64_t)b * ldy + row] = y;
+    for (int b0 = 0; b0 < nrhs; b0 += NB) {
+      float acc[NB];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[j] = 0.f;
+      for (int kb = k0; kb < k1; kb += kCsrBatch) {
+        int c[kCsrBatch];
+        float v[kCsrBatch], xv[NB][kCsrBatch];
+#pragma unroll
+        for (int i = 0; i < kCsrBatch; ++i) {  // past the row's end: its last entry again, dropped below
+          const int k = kb + i < k1 ? kb + i : k1 - 1;
+          c[i] = colind[k];
+          v[i] = val[k];
+        }
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int i = 0; i < kCsrBatch; ++i)
+            xv[j][i] = X[(int64_t)(b0 + j < nrhs ? b0 + j : b0) * ldx + c[i]];
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int i = 0; i < kCsrBatch; ++i) acc[j] = kb + i < k1 ? fmaf(v[i], xv[j][i], acc[j]) : acc[j];
+      }
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int b = b0 + j;
+        if (b >= nrhs) break;
+        float y = scale * acc[j];
+        if (shift != 0.f) y = fmaf(shift, X[(int64_t)b * ldx + rc], y);
+        if (!XY || row < n) Y[(int64_t)b * ldy + row] = y;
+      }
     }
   }
   if constexpr (XY) {
@@ -795,26 +796,201 @@ __global__ __launch_bounds__(XY ? 1024 : 256) void csr_lane_per_row(int n, const
   }
 }
 
-int csr_dispatch(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, const int* done,
-                 hipStream_t s) {
+// Longer rows: a group of G lanes per row (4, or 8 at eight rhs so that each rhs has a lane to store
+// it; a whole wave for rows of more than 128 entries on average).  Lane l of the group takes the
+// row's entries l, l + G, ... in order, U of them per batch: the batch's column indices and values go
+// out together, then its gathers of x, so a row costs two dependent memory waits per G * U entries.
+// The lanes' sums are added in a fixed tree, whether or not xy_part is asked for.
+// Bound by the gathers, which land on a cache line of their own where the columns are scattered:
+// with several rhs they come from a copy of x with the rhs fastest (csr_interleave, 4-5 us at
+// 300000 x 4), one NB-wide load and one line per entry instead of NB.  Measured, 300000 rows of 14.9
+// entries, a quarter of them anywhere (36 MB): 1 rhs 69 -> 16 us, 4 rhs 246 -> 32 us (57 without
+// the copy), 8 rhs 511 -> 56 us, against one lane per row; 50000 rows of 69 entries, against one
+// wave per row and rhs: 1 rhs 13.6 -> 12.8, 4 rhs 34 -> 21, 8 rhs 62 -> 31 us.  Short regular rows
+// (5-point Laplacian, 631000 rows) stay with one lane per row: 7.6 us against 14.6, 4 rhs 12.7
+// against 19.4.
+template <int G>
+__device__ __forceinline__ float group_sum(float v) {
+  if (G == 64) return wave_sum(v);
+  v += dpp_f32<0xB1>(v);                // quad_perm [1,0,3,2]
+  v += dpp_f32<0x4E>(v);                // quad_perm [2,3,0,1]
+  if (G >= 8) v += dpp_f32<0x141>(v);   // row_half_mirror
+  if (G >= 16) v += dpp_f32<0x140>(v);  // row_mirror
+  return v;
+}
+
+// Xt[i * NB + j] = X[j * ldx + i] for the nbr <= NB rhs of a pass, zero beyond them
+template <int NB>
+__global__ __launch_bounds__(256) void csr_interleave(int n, int nbr, const float* __restrict__ X, int64_t ldx,
+                                                      float* __restrict__ Xt, const int* __restrict__ done) {
+  if (done && *done) return;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  float v[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) v[j] = j < nbr ? X[(int64_t)j * ldx + i] : 0.f;
+  typedef float vec __attribute__((ext_vector_type(NB < 4 ? NB : 4)));
+#pragma unroll
+  for (int q = 0; q < NB; q += (NB < 4 ? NB : 4)) {
+    vec t;
+#pragma unroll
+    for (int j = 0; j < (NB < 4 ? NB : 4); ++j) t[j] = v[q + j];
+    *reinterpret_cast<vec*>(Xt + (int64_t)i * NB + q) = t;
+  }
+}
+
+// One pass of nbr <= NB rhs.  Xt: the interleaved x (unused at NB = 1, where X itself is gathered).
+template <int G, int NB, int U>
+__global__ __launch_bounds__(256) void csr_group_kernel(int n, const int32_t* __restrict__ rowptr,
+                                                        const int32_t* __restrict__ colind,
+                                                        const float* __restrict__ val, const float* __restrict__ X,
+                                                        int64_t ldx, const float* __restrict__ Xt,
+                                                        float* __restrict__ Y, int64_t ldy, int nbr, float scale,
+                                                        float shift, int rows, const int* __restrict__ done,
+                                                        float* __restrict__ xy_part) {
+  static_assert(NB <= G, "one lane of the group stores each rhs");
+  if (done && *done) return;
+  __shared__ float red[256];
+  constexpr int R = 256 / G;  // rows per sweep of the block
+  constexpr int V = NB < 4 ? NB : 4;
+  typedef float vec __attribute__((ext_vector_type(V)));
+  const int l = threadIdx.x % G, g = threadIdx.x / G;
+  const int row0 = blockIdx.x * rows;
+  const bool stores = l < nbr;
+  const int lb = stores ? l : 0;  // the rhs this lane stores
+  float xy = 0.f;
+  for (int r = g; r < rows; r += R) {
+    const int row = row0 + r;
+    const bool in = row < n;
+    const int rc = in ? row : n - 1;
+    const int k0 = rowptr[rc], k1 = in ? rowptr[rc + 1] : k0;
+    const float xr = X[(int64_t)lb * ldx + rc];
+    float acc[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[j] = 0.f;
+    for (int kb = k0; kb < k1; kb += G * U) {
+      int c[U];
+      float v[U], x[U][NB];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {  // past the row's end: its last entry again, dropped below
+        const int k = kb + u * G + l, kk = k < k1 ? k : k1 - 1;
+        c[u] = colind[kk];
+        v[u] = val[kk];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (NB == 1) {
+          x[u][0] = X[c[u]];
+        } else {
+#pragma unroll
+          for (int q = 0; q < NB; q += V) {
+            const vec t = *reinterpret_cast<const vec*>(Xt + (int64_t)c[u] * NB + q);
+#pragma unroll
+            for (int j = 0; j < V; ++j) x[u][q + j] = t[j];
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool on = kb + u * G + l < k1;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[j] = on ? fmaf(v[u], x[u][j], acc[j]) : acc[j];
+      }
+    }
+    float mine = 0.f;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const float s = group_sum<G>(acc[j]);
+      mine = l == j ? s : mine;
+    }
+    float y = scale * mine;
+    if (shift != 0.f) y = fmaf(shift, xr, y);
+    if (stores && in) {
+      Y[(int64_t)lb * ldy + row] = y;
+      xy = fmaf(xr, y, xy);
+    }
+  }
+  if (xy_part) {
+    red[threadIdx.x] = xy;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+      float s = (red[threadIdx.x] + red[threadIdx.x + 64]) + (red[threadIdx.x + 128] + red[threadIdx.x + 192]);
+#pragma unroll
+      for (int o = G; o < 64; o *= 2) s += __shfl_xor(s, o);
+      if ((int)threadIdx.x < nbr) xy_part[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
+    }
+  }
+}
+
+inline int csr_pass(int nrhs) { return nrhs <= 1 ? 1 : nrhs <= 2 ? 2 : nrhs <= 4 ? 4 : 8; }
+inline size_t csr_xt_bytes(int64_t n, int nrhs) {
+  return nrhs > 1 ? (size_t)csr_pass(nrhs) * n * sizeof(float) : 0;
+}
+
+int csr_launch(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, void* work,
+               size_t work_bytes, const int* done, float* xy_part, hipStream_t s) {
   const int n = op->n;
   if (!op->rowptr || !op->colind || !op->values) return CK_ERR_BAD_ARG;
-  const double avg = n > 0 ? (double)op->nnz / n : 0.0;
-  if (avg > 32.0) {
-    const int grid = (n + 3) / 4;
-    hipLaunchKernelGGL(csr_wave_per_row, dim3(grid), dim3(256), 0, s, n, op->rowptr, op->colind, op->values, X, ldx,
-                       Y, ldy, nrhs, op->scale, op->shift, done);
-  } else {
-    const dim3 grid((unsigned)((n + 255) / 256)), blk(256);
+  if (csr_short_rows(op)) {
+    const dim3 grid((unsigned)cdiv(n, xy_part ? 1024 : 256)), blk(xy_part ? 1024 : 256);
+#define CK_CSR(NB_)                                                                                                 \
+  do {                                                                                                              \
+    if (xy_part)                                                                                                    \
+      hipLaunchKernelGGL((csr_lane_per_row<NB_, true>), grid, blk, 0, s, n, op->rowptr, op->colind, op->values, X, \
+                         ldx, Y, ldy, nrhs, op->scale, op->shift, done, xy_part);                                   \
+    else                                                                                                            \
+      hipLaunchKernelGGL((csr_lane_per_row<NB_>), grid, blk, 0, s, n, op->rowptr, op->colind, op->values, X, ldx,  \
+                         Y, ldy, nrhs, op->scale, op->shift, done, xy_part);                                        \
+  } while (0)
     if (nrhs == 1)
-      hipLaunchKernelGGL(csr_lane_per_row<1>, grid, blk, 0, s, n, op->rowptr, op->colind, op->values, X, ldx, Y, ldy,
-                         nrhs, op->scale, op->shift, done, nullptr);
+      CK_CSR(1);
     else if (nrhs == 2)
-      hipLaunchKernelGGL(csr_lane_per_row<2>, grid, blk, 0, s, n, op->rowptr, op->colind, op->values, X, ldx, Y, ldy,
-                         nrhs, op->scale, op->shift, done, nullptr);
+      CK_CSR(2);
     else
-      hipLaunchKernelGGL(csr_lane_per_row<4>, grid, blk, 0, s, n, op->rowptr, op->colind, op->values, X, ldx, Y, ldy,
-                         nrhs, op->scale, op->shift, done, nullptr);
+      CK_CSR(4);
+#undef CK_CSR
+    CK_CHECK_LAUNCH();
+    return CK_OK;
+  }
+  const int rows = csr_rows(op);
+  const dim3 grid((unsigned)csr_xy_nparts(op)), blk(256);
+  // the interleaved x sits past the partials; without room for it the rhs go one at a time
+  const size_t off = csr_xy_bytes(op, nrhs);
+  const bool room = work && work_bytes >= off + csr_xt_bytes(n, nrhs);
+  float* xt = room ? reinterpret_cast<float*>(static_cast<char*>(work) + off) : nullptr;
+  const int step = room ? csr_pass(nrhs) : 1;
+  for (int b0 = 0; b0 < nrhs; b0 += step) {
+    const int nb = nrhs - b0 < step ? nrhs - b0 : step;
+    const float* Xb = X + b0 * ldx;
+    float* Yb = Y + b0 * ldy;
+    float* xyb = xy_part ? xy_part + (size_t)b0 * grid.x : nullptr;
+    const dim3 tg((unsigned)cdiv(n, 256));
+#define CK_CSR(G_, NB_, U_)                                                                                        \
+  do {                                                                                                             \
+    if (NB_ > 1) hipLaunchKernelGGL(csr_interleave<NB_>, tg, blk, 0, s, n, nb, Xb, ldx, xt, done);                  \
+    hipLaunchKernelGGL((csr_group_kernel<G_, NB_, U_>), grid, blk, 0, s, n, op->rowptr, op->colind, op->values,    \
+                       Xb, ldx, (const float*)xt, Yb, ldy, nb, op->scale, op->shift, rows, done, xyb);             \
+  } while (0)
+    if (csr_long_rows(op)) {
+      if (step == 1)
+        CK_CSR(64, 1, 4);
+      else if (step == 2)
+        CK_CSR(64, 2, 4);
+      else if (step == 4)
+        CK_CSR(64, 4, 4);
+      else
+        CK_CSR(64, 8, 2);
+    } else {
+      if (step == 1)
+        CK_CSR(4, 1, 8);
+      else if (step == 2)
+        CK_CSR(4, 2, 4);
+      else if (step == 4)
+        CK_CSR(4, 4, 4);
+      else
+        CK_CSR(8, 8, 4);
+    }
+#undef CK_CSR
   }
   CK_CHECK_LAUNCH();
   return CK_OK;
@@ -825,22 +1001,9 @@ int csr_dispatch(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* 
 namespace ck {
 
 int csr_apply_xy(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, const int* done,
-                 float* xy_part, hipStream_t s) {
-  const int n = op->n;
-  if (op->kind != CK_OP_CSR_F32 || !op->rowptr || !op->colind || !op->values || !xy_part) return CK_ERR_BAD_ARG;
-  if (n > 0 && (double)op->nnz / n > 32.0) return CK_ERR_UNSUPPORTED;  // the wave-per-row kernel has no epilogue
-  const dim3 grid((unsigned)csr_xy_nparts(n)), blk(1024);
-  if (nrhs == 1)
-    hipLaunchKernelGGL((csr_lane_per_row<1, true>), grid, blk, 0, s, n, op->rowptr, op->colind, op->values, X, ldx, Y,
-                       ldy, nrhs, op->scale, op->shift, done, xy_part);
-  else if (nrhs == 2)
-    hipLaunchKernelGGL((csr_lane_per_row<2, true>), grid, blk, 0, s, n, op->rowptr, op->colind, op->values, X, ldx, Y,
-                       ldy, nrhs, op->scale, op->shift, done, xy_part);
-  else
-    hipLaunchKernelGGL((csr_lane_per_row<4, true>), grid, blk, 0, s, n, op->rowptr, op->colind, op->values, X, ldx, Y,
-                       ldy, nrhs, op->scale, op->shift, done, xy_part);
-  CK_CHECK_LAUNCH();
-  return CK_OK;
+                 float* xy_part, void* work, size_t work_bytes, hipStream_t s) {
+  if (op->kind != CK_OP_CSR_F32 || !xy_part) return CK_ERR_BAD_ARG;
+  return csr_launch(op, nrhs, X, ldx, Y, ldy, work, work_bytes, done, xy_part, s);
 }
 
 }  // namespace ck
@@ -1103,7 +1266,7 @@ int op_apply_internal(const ck_op* op, int nrhs, const float* X, int64_t ldx, fl
       return CK_OK;
     }
     case CK_OP_CSR_F32:
-      return csr_dispatch(op, nrhs, X, ldx, Y, ldy, done, s);
+      return csr_launch(op, nrhs, X, ldx, Y, ldy, work, work_bytes, done, nullptr, s);
     case CK_OP_KRON_F32:
       return kron_dispatch(op, nrhs, X, ldx, Y, ldy, work, work_bytes, done, nullptr, 0, s);
     case CK_OP_WOODBURY_INV:
@@ -1137,8 +1300,8 @@ size_t op_workspace_internal(const ck_op* op, int nrhs) {
     case CK_OP_RBF_F32:
       return rbf_workspace_bytes(op, nrhs);
     case CK_OP_CSR_F32:
-      // the x.Ax partials of csr_apply_xy (CG's p.Ap, Lanczos's v.Av)
-      return csr_xy_bytes(op->n, nrhs);
+      // the x.Ax partials of csr_apply_xy (CG's p.Ap, Lanczos's v.Av), then the interleaved x
+      return csr_xy_bytes(op, nrhs) + (csr_short_rows(op) ? 0 : csr_xt_bytes(op->n, nrhs));
     default:
       return 0;
   }

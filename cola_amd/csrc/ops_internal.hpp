@@ -35,12 +35,26 @@ inline size_t dense_xy_bytes(int64_t n, int nrhs) { return ((size_t)4 * nrhs * d
 int dense_apply_xy(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, const int* done,
                    float* xy_part, void* work, size_t work_bytes, hipStream_t s);
 
-// CSR fp32 apply (average row length <= 32) that also writes per-block partial sums of X . Y:
-// csr_xy_nparts(n) partials per rhs; CK_ERR_UNSUPPORTED for longer rows.
-inline int csr_xy_nparts(int64_t n) { return (int)((n + 1023) / 1024); }
-inline size_t csr_xy_bytes(int64_t n, int nrhs) { return ((size_t)4 * nrhs * csr_xy_nparts(n) + 255) / 256 * 256; }
+// CSR fp32 apply that also writes per-block partial sums of X . Y: csr_xy_nparts(op) partials per
+// rhs (every block of the kernel that consumes them reads all of them).  Rows of up to 8 entries on
+// average: one lane per row in blocks of 1024 rows; longer ones: blocks of csr_rows(op) rows, one
+// sweep of the block's lane groups or as many as keep the blocks at 2048.  work: the operator's
+// workspace, the partials at its head.
+inline bool csr_short_rows(const ck_op* op) { return (double)op->nnz <= 8.0 * (double)op->n; }
+inline bool csr_long_rows(const ck_op* op) { return (double)op->nnz > 128.0 * (double)op->n; }
+inline int csr_rows(const ck_op* op) {
+  const int64_t n = op->n, sweep = csr_long_rows(op) ? 4 : 64;
+  return (int)(sweep * ((n + sweep * 2048 - 1) / (sweep * 2048)));
+}
+inline int csr_xy_nparts(const ck_op* op) {
+  const int64_t n = op->n, r = csr_short_rows(op) ? 1024 : csr_rows(op);
+  return (int)((n + r - 1) / r);
+}
+inline size_t csr_xy_bytes(const ck_op* op, int nrhs) {
+  return ((size_t)4 * nrhs * csr_xy_nparts(op) + 255) / 256 * 256;
+}
 int csr_apply_xy(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, const int* done,
-                 float* xy_part, hipStream_t s);
+                 float* xy_part, void* work, size_t work_bytes, hipStream_t s);
 
 int woodbury_apply(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, void* work,
                    size_t work_bytes, const int* done, hipStream_t s);
