@@ -22,6 +22,12 @@ __host__ __device__ inline int stride_of(int nrhs) { return cg_stride_of(nrhs); 
 
 __host__ __device__ inline CgView view(void* state, int nrhs) { return cg_view(state, nrhs); }
 
+// Up to kJoinRhs rhs the state's per-column arrays (rounded up to 64 columns) have as many unused
+// columns as used ones: the beta array's hold, during a step, what each column's beta divides by --
+// gamma before the step, infinity for a column that has converged (written by the x/r update).
+constexpr int kJoinRhs = 32;
+__device__ inline float* step_den(const CgView& v, int nrhs) { return v.beta + kJoinRhs; }
+
 inline int nparts_of(int64_t n) {
   int64_t p = cdiv(n, kChunk);
   if (p < 1) p = 1;
@@ -210,6 +216,7 @@ __global__ __launch_bounds__(256) void update_xr_kernel(int64_t n, const float* 
   const float alpha = (float)a;
   if (blk == 0 && threadIdx.x == 0) {
     v.alpha[b] = alpha;
+    if (nrhs <= kJoinRhs) step_den(v, nrhs)[b] = frozen ? INFINITY : v.gamma[b];
     // the reference divides on regardless; the status records it (same value from every writer)
     if (!frozen && !(pap > 0.0) && v.ctrl->status == CK_OK) v.ctrl->status = CK_ERR_BREAKDOWN;
   }
@@ -335,35 +342,31 @@ __global__ __launch_bounds__(256) void step1_x64_kernel(int64_t n, const float* 
   }
 }
 
-// End of step: rnorm, gamma1, beta, k, errors, loop condition.
-__global__ __launch_bounds__(256) void step_final_kernel(int nrhs, const float* __restrict__ part1,
-                                                         const float* __restrict__ part2, int P, int precond,
-                                                         void* state) {
-  CgView v = view(state, nrhs);
-  if (v.ctrl->done) return;
+// End of step: rnorm, gamma, beta, k, errors, loop condition, by one block of 256 threads.  den: what
+// each column's beta divides by (infinity: frozen), or nullptr for gamma itself.
+__device__ inline void step_scalars(const CgView& v, int nrhs, const float* __restrict__ part1,
+                                    const float* __restrict__ part2, int P, int precond, const float* den) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   __shared__ float newrn[1024];
   for (int b = wave; b < nrhs; b += 4) {
     const double rr = column_total(part1, P, b);
     const double rz = precond ? column_total(part2, P, b) : rr;
     if (lane == 0) {
-      const bool frozen = (double)v.rnorm[b] < kSmall;  // uses ||r0|| of this step
-      double beta = safe_div(rz, (double)v.gamma[b]);
-      if (frozen) beta = 0.0;
-      v.beta[b] = (float)beta;
+      // frozen uses ||r0|| of this step
+      const bool frozen = den ? den[b] == INFINITY : (double)v.rnorm[b] < kSmall;
+      v.beta[b] = frozen ? 0.f : (float)safe_div(rz, (double)(den ? den[b] : v.gamma[b]));
       v.gamma[b] = (float)rz;
       newrn[b & 1023] = (float)sqrt(rr);
     }
   }
   __syncthreads();
   for (int b = threadIdx.x; b < nrhs; b += 256) v.rnorm[b] = newrn[b & 1023];
-  __syncthreads();
   if (threadIdx.x == 0) {
     const int k = v.ctrl->k + 1;
     float mean = 0.f;
     bool any = false;
     for (int b = 0; b < nrhs; ++b) {
-      const float rn = v.rnorm[b];
+      const float rn = newrn[b & 1023];
       mean += rn;
       any = any || (rn > v.tol[b]);
     }
@@ -372,7 +375,7 @@ __global__ __launch_bounds__(256) void step_final_kernel(int nrhs, const float* 
     if (!(any && k < v.ctrl->max_iters)) {
       v.ctrl->done = 1;
       bool finite = true;
-      for (int b = 0; b < nrhs; ++b) finite = finite && isfinite(v.rnorm[b]);
+      for (int b = 0; b < nrhs; ++b) finite = finite && isfinite(newrn[b & 1023]);
       if (!finite)
         v.ctrl->status = CK_ERR_NAN;
       else if (any && v.ctrl->status == CK_OK)
@@ -381,33 +384,62 @@ __global__ __launch_bounds__(256) void step_final_kernel(int nrhs, const float* 
   }
 }
 
-// p = z + beta p
-template <bool V4>
+__global__ __launch_bounds__(256) void step_final_kernel(int nrhs, const float* __restrict__ part1,
+                                                         const float* __restrict__ part2, int P, int precond,
+                                                         void* state) {
+  CgView v = view(state, nrhs);
+  if (v.ctrl->done) return;
+  step_scalars(v, nrhs, part1, part2, P, precond, nullptr);
+}
+
+// p = z + beta p.  JOINED: the end of the step as well, for up to kJoinRhs rhs.  The blocks of
+// row x = 0 are the step's scalars (block (0, 0), all columns); every other block forms its own
+// column's beta from the r.r or r.z partials and the divisor that the x/r update left in step_den.
+// What block (0, 0) writes is read by no other block of the launch except the loop flag: one that
+// already sees it set leaves p alone, which nothing reads once the loop has ended.
+// Latency bound: the two launches took 4.4 + 5.5 us of a step at 144000 x 8, 3.3 + 2.4 us at
+// 2500 x 4 and 4.6 + 4.9 us at 16384 x 8; joined, a step is 3.0, 4.0 and 2.5 us shorter.
+template <bool V4, bool JOINED>
 __global__ __launch_bounds__(256) void update_p_kernel(int64_t n, const float* __restrict__ z, float* __restrict__ p,
-                                                       int64_t ld, void* state, int nrhs) {
+                                                       int64_t ld, const float* __restrict__ part1,
+                                                       const float* __restrict__ part2, int P, int precond,
+                                                       void* state, int nrhs) {
+  CgView v = view(state, nrhs);
+  if (JOINED && blockIdx.x == 0) {
+    if (blockIdx.y == 0 && !v.ctrl->done) step_scalars(v, nrhs, part1, part2, P, precond, step_den(v, nrhs));
+    return;
+  }
   const int b = blockIdx.y;
   const float* zb = z + b * ld;
   float* pb = p + b * ld;
+  const int64_t i = (V4 ? 4 : 1) * ((int64_t)(blockIdx.x - (JOINED ? 1 : 0)) * 256 + threadIdx.x);
+  const int64_t c = i < n ? i : 0;  // clamped: the wave stays whole for the column's total
+  float4 zv, pv;
+  // the vector loads go out before the loop flag, beta and the partials are read
   if (V4) {
-    const int64_t i = 4 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= n) return;
-    // the vector loads go out before the loop flag and beta are read
-    const float4 zv = *reinterpret_cast<const float4*>(zb + i);
-    float4 pv = *reinterpret_cast<float4*>(pb + i);
-    CgView v = view(state, nrhs);
-    if (v.ctrl->done) return;
-    const float beta = v.beta[b];
+    zv = *reinterpret_cast<const float4*>(zb + c);
+    pv = *reinterpret_cast<const float4*>(pb + c);
+  } else {
+    zv.x = zb[c];
+    pv.x = pb[c];
+  }
+  float beta;
+  if (JOINED) {
+    const float den = step_den(v, nrhs)[b];
+    const double rz = column_total(precond ? part2 : part1, P, b);
+    beta = den == INFINITY ? 0.f : (float)safe_div(rz, (double)den);
+  } else {
+    beta = v.beta[b];
+  }
+  if (v.ctrl->done || i >= n) return;
+  if (V4) {
     pv.x = fmaf(beta, pv.x, zv.x);
     pv.y = fmaf(beta, pv.y, zv.y);
     pv.z = fmaf(beta, pv.z, zv.z);
     pv.w = fmaf(beta, pv.w, zv.w);
-    *reinterpret_cast<float4*>(pb + i) = pv;
+    *reinterpret_cast<float4*>(pb + c) = pv;
   } else {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    CgView v = view(state, nrhs);
-    if (v.ctrl->done) return;
-    pb[i] = fmaf(v.beta[b], pb[i], zb[i]);
+    pb[c] = fmaf(beta, pv.x, zv.x);
   }
 }
 
@@ -469,6 +501,24 @@ int step_xr(int64_t n, int nrhs, const float* p, const float* Ap, float* x, floa
   return CK_OK;
 }
 
+void launch_step_p(int64_t n, int nrhs, const float* z, float* p, int64_t ld, const float* rr, const float* rz, int P,
+                   int precond, void* state, hipStream_t s) {
+  const bool v4 = use_v4(n, ld, z, p, nullptr, nullptr), joined = nrhs <= kJoinRhs;
+  if (!joined) hipLaunchKernelGGL(step_final_kernel, dim3(1), dim3(256), 0, s, nrhs, rr, rz, P, precond, state);
+  const dim3 grid((unsigned)cdiv(v4 ? n / 4 : n, 256) + (joined ? 1 : 0), nrhs), blk(256);
+#define CK_STEP_P(V4_, J_) \
+  hipLaunchKernelGGL((update_p_kernel<V4_, J_>), grid, blk, 0, s, n, z, p, ld, rr, rz, P, precond, state, nrhs)
+  if (v4 && joined)
+    CK_STEP_P(true, true);
+  else if (v4)
+    CK_STEP_P(true, false);
+  else if (joined)
+    CK_STEP_P(false, true);
+  else
+    CK_STEP_P(false, false);
+#undef CK_STEP_P
+}
+
 // rz_ready: the preconditioner's last pass already wrote the r.z partials (q.p2)
 int step_p(int64_t n, int nrhs, const float* r, const float* z, float* p, int64_t ld, void* state, const Parts& q,
            hipStream_t s, bool rz_ready = false) {
@@ -478,13 +528,7 @@ int step_p(int64_t n, int nrhs, const float* r, const float* z, float* p, int64_
     int st = launch_partials(0, n, nrhs, r, z, ld, q.p2, q, done, s);
     if (st) return st;
   }
-  hipLaunchKernelGGL(step_final_kernel, dim3(1), dim3(256), 0, s, nrhs, q.p1, q.p2, q.P, precond, state);
-  if (use_v4(n, ld, z, p, nullptr, nullptr))
-    hipLaunchKernelGGL(update_p_kernel<true>, dim3((unsigned)cdiv(n / 4, 256), nrhs), dim3(256), 0, s, n, z, p, ld,
-                       state, nrhs);
-  else
-    hipLaunchKernelGGL(update_p_kernel<false>, dim3((unsigned)cdiv(n, 256), nrhs), dim3(256), 0, s, n, z, p, ld,
-                       state, nrhs);
+  launch_step_p(n, nrhs, z, p, ld, q.p1, q.p2, q.P, precond, state, s);
   CK_CHECK_LAUNCH();
   return CK_OK;
 }
@@ -559,7 +603,7 @@ namespace {
 // For A dense fp32 and P = CK_OP_WOODBURY_INV (rank <= 64, 3..8 rhs) a step runs as
 //   dense matvec (p.Ap partials in its epilogue) -> wbf_xr (alpha, x/r update, r.r and
 //   F^T r tile partials) -> wbf_core (u = C^-1 F^T r) -> wbf_z (z = scale (r - F u) +
-//   shift r, r.z partials) -> step_final -> update_p
+//   shift r, r.z partials) -> step end and p update
 // instead of separate partial, F^T r, core, apply and r.z passes.  The Woodbury arithmetic
 // after the fp32 loads stays FP64 as in the unfused apply.
 struct WbFused {
@@ -641,6 +685,7 @@ __global__ __launch_bounds__(256) void wbf_xr_kernel(int64_t n, int nrhs, const 
       alpha_s[b] = (float)a;
       if (tile == 0) {
         v.alpha[b] = (float)a;
+        if (nrhs <= kJoinRhs) step_den(v, nrhs)[b] = frozen ? INFINITY : v.gamma[b];
         if (!frozen && !(pap_b > 0.0) && v.ctrl->status == CK_OK) v.ctrl->status = CK_ERR_BREAKDOWN;
       }
     }
@@ -869,14 +914,7 @@ int cg_iterate(const ck_op* A, const ck_op* P, int32_t nrhs, float* x, float* r,
                          reinterpret_cast<const double*>(P->aux), W.u, state);
       hipLaunchKernelGGL(wbf_z_kernel, dim3(W.T), dim3(256), 0, s, n, (int)nrhs, (const float*)r, z, ld, F, P->lda, k,
                          (const double*)W.u, (double)P->scale, (double)P->shift, W.rz, W.T, state);
-      hipLaunchKernelGGL(step_final_kernel, dim3(1), dim3(256), 0, s, (int)nrhs, (const float*)W.rr,
-                         (const float*)W.rz, W.T, 1, state);
-      if (use_v4(n, ld, z, p, nullptr, nullptr))
-        hipLaunchKernelGGL(update_p_kernel<true>, dim3((unsigned)cdiv(n / 4, 256), nrhs), dim3(256), 0, s, n, z, p,
-                           ld, state, nrhs);
-      else
-        hipLaunchKernelGGL(update_p_kernel<false>, dim3((unsigned)cdiv(n, 256), nrhs), dim3(256), 0, s, n, z, p, ld,
-                           state, nrhs);
+      launch_step_p(n, nrhs, z, p, ld, W.rr, W.rz, W.T, 1, state, s);
       CK_CHECK_LAUNCH();
       continue;
     }
