@@ -1116,10 +1116,16 @@ int lz_matvec(const ck_op* A, int nb, const float* vi, float* w, int64_t ldb, vo
   }
   if (A->kind == CK_OP_KRON_F32 && A->nfactors == 3) {
     const int np = kron_nparts(A);
-    if (np > 0 && np <= 2 * sc.P) {  // the partials go to dpart (room for nb x 2P)
-      const int st = kron_dispatch(A, nb, vi, ldb, w, ldb, work, work_bytes, done, sc.dpart, np, s);
+    const size_t off = kron_xy_offset(A, nb);
+    // the partials go to the operator's workspace, or (64^3) to dpart (room for nb x 2P)
+    float* part = off ? (work && work_bytes >= kron_workspace_bytes(A, nb)
+                             ? reinterpret_cast<float*>(static_cast<char*>(work) + off)
+                             : nullptr)
+                      : np <= 2 * sc.P ? sc.dpart : nullptr;
+    if (part) {
+      const int st = kron_dispatch(A, nb, vi, ldb, w, ldb, work, work_bytes, done, part, np, s);
       if (st == CK_OK) {
-        *xy = sc.dpart;
+        *xy = part;
         *pxy = np;
         return CK_OK;
       }

@@ -5,10 +5,7 @@
 //   csr    : one lane per row, short rows batched into registers (short rows) or
 //            one wavefront per row (long rows);
 //            int32 column indices; coalesced rowptr/value streams. [HBM bound]
-//   kron   : factors of order <= 64; the last two modes are fused per slab
-//            (U = K2 S K3^T with S the 64x64 slab) and the first mode is a
-//            64-row GEMM over 64-column tiles, both on v_mfma_f32_16x16x4f32 with
-//            LDS-staged, bank-padded factors.                    [MFMA bound]
+//   kron   : factors of order <= 64, in kron.hip (64^3) and kron_any.hip.
 #include "common.hpp"
 #include "ops_internal.hpp"
 
@@ -1024,143 +1021,6 @@ __global__ __launch_bounds__(256) void diag_kernel(int64_t n, int nrhs, const fl
   Y[b * ldy + i] = fmaf(scale * s, x, shift * x);
 }
 
-// ============================================================== Kronecker (MFMA)
-constexpr int KP = 66;  // LDS row pitch (floats): conflict-free 16x4 operand reads
-
-__device__ __forceinline__ floatx4 mfma16x16x4(float a, float b, floatx4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// Load an r x c row-major global matrix (leading dim ld) into LDS [64][KP], zero padded.
-__device__ __forceinline__ void load_pad64(float* __restrict__ dst, const float* __restrict__ src, int r, int c,
-                                           int64_t ld) {
-  for (int idx = threadIdx.x; idx < 64 * 64; idx += blockDim.x) {
-    const int i = idx >> 6, j = idx & 63;
-    dst[i * KP + j] = (i < r && j < c) ? src[(int64_t)i * ld + j] : 0.f;
-  }
-}
-
-// Wave w computes rows [16w, 16w+16) x cols [0,64) of C = A * B^T where A, Bt are
-// LDS [64][KP] (Bt holds B transposed, i.e. Bt[col][k]); k runs over kdim (<= 64).
-__device__ __forceinline__ void wave_gemm_abt(const float* __restrict__ A, const float* __restrict__ Bt, int kdim,
-                                              floatx4 acc[4]) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int ra = (wave * 16 + (lane & 15)) * KP;
-  const int kk = lane >> 4;
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  for (int k = 0; k < kdim; k += 4) {
-    const float a = A[ra + k + kk];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float b = Bt[(t * 16 + (lane & 15)) * KP + k + kk];
-      acc[t] = mfma16x16x4(a, b, acc[t]);
-    }
-  }
-}
-
-// Pass A: for slab (b, i1): U = K2 * S * K3^T, S = X[b][i1] viewed as n2 x n3.
-// LAST: U is the operator output (two-factor case): Y = scale*U + shift*S.
-template <bool LAST>
-__global__ __launch_bounds__(256) void kron_pass_a(int n1, int n2, int n3, const float* __restrict__ K2,
-                                                   const float* __restrict__ K3, const float* __restrict__ X,
-                                                   int64_t ldx, float* __restrict__ Out, int64_t ldo, float scale,
-                                                   float shift, const int* __restrict__ done) {
-  if (done && *done) return;
-  extern __shared__ float lds[];
-  float* S = lds;           // [64][KP] slab
-  float* Kx = S + 64 * KP;  // K3 for the first product, then K2
-  float* Tt = Kx + 64 * KP; // (S K3^T)^T
-  const int i1 = blockIdx.x, b = blockIdx.y;
-  const int64_t slab = (int64_t)b * ldx + (int64_t)i1 * n2 * n3;
-  const int64_t oslab = (int64_t)b * ldo + (int64_t)i1 * n2 * n3;
-  for (int idx = threadIdx.x; idx < 64 * 64; idx += blockDim.x) {
-    const int i = idx >> 6, j = idx & 63;
-    S[i * KP + j] = (i < n2 && j < n3) ? X[slab + i * n3 + j] : 0.f;
-  }
-  load_pad64(Kx, K3, n3, n3, n3);
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  floatx4 acc[4];
-  // T = S * K3^T  (T[r][c] = sum_k S[r][k] K3[c][k]); store transposed.
-  wave_gemm_abt(S, Kx, n3, acc);
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int r = wave * 16 + 4 * (lane >> 4) + it;
-      const int c = t * 16 + (lane & 15);
-      Tt[c * KP + r] = acc[t][it];
-    }
-  __syncthreads();
-  load_pad64(Kx, K2, n2, n2, n2);
-  __syncthreads();
-  // U = K2 * T  (U[r][c] = sum_k K2[r][k] T[k][c] = sum_k K2[r][k] Tt[c][k]).
-  wave_gemm_abt(Kx, Tt, n2, acc);
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int r = wave * 16 + 4 * (lane >> 4) + it;
-      const int c = t * 16 + (lane & 15);
-      if (r < n2 && c < n3) {
-        float u = acc[t][it];
-        if (LAST) {
-          u = scale * u;
-          if (shift != 0.f) u = fmaf(shift, S[r * KP + c], u);
-        }
-        Out[oslab + r * n3 + c] = u;
-      }
-    }
-}
-
-// Pass B: Y[b][j1][c] = scale * sum_k K1[j1][k] U[b][k][c] + shift * X[b][j1][c]
-// for a 64-column tile c in [64*blockIdx.x, +64).  Optionally accumulates the
-// per-block partial sum of X*Y into partials[b * nparts + blockIdx.x].
-__global__ __launch_bounds__(256) void kron_pass_b(int n1, int plane, const float* __restrict__ K1,
-                                                   const float* __restrict__ U, int64_t ldu,
-                                                   const float* __restrict__ X, int64_t ldx, float* __restrict__ Y,
-                                                   int64_t ldy, float scale, float shift, float* __restrict__ partials,
-                                                   int nparts, const int* __restrict__ done) {
-  if (done && *done) return;
-  extern __shared__ float lds[];
-  float* Ka = lds;           // K1 [64][KP]
-  float* Ut = Ka + 64 * KP;  // U tile transposed: Ut[c][k]
-  __shared__ float red[4];
-  const int b = blockIdx.y;
-  const int c0 = blockIdx.x * 64;
-  load_pad64(Ka, K1, n1, n1, n1);
-  for (int idx = threadIdx.x; idx < 64 * 64; idx += blockDim.x) {
-    const int k = idx >> 6, c = idx & 63;
-    Ut[c * KP + k] = (k < n1 && c0 + c < plane) ? U[(int64_t)b * ldu + (int64_t)k * plane + c0 + c] : 0.f;
-  }
-  __syncthreads();
-  floatx4 acc[4];
-  wave_gemm_abt(Ka, Ut, n1, acc);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  float dot = 0.f;
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int r = wave * 16 + 4 * (lane >> 4) + it;
-      const int c = c0 + t * 16 + (lane & 15);
-      if (r < n1 && c < plane) {
-        const int64_t off = (int64_t)r * plane + c;
-        const float x = X[(int64_t)b * ldx + off];
-        float y = scale * acc[t][it];
-        if (shift != 0.f) y = fmaf(shift, x, y);
-        Y[(int64_t)b * ldy + off] = y;
-        dot = fmaf(x, y, dot);
-      }
-    }
-  if (partials) {
-    const float s = block_sum<256>(dot, red);
-    if (threadIdx.x == 0) partials[(int64_t)b * nparts + blockIdx.x] = s;
-  }
-}
-
 }  // namespace
 
 // ============================================================== internal API
@@ -1190,9 +1050,17 @@ int dense_apply_xy(const ck_op* op, int nrhs, const float* X, int64_t ldx, float
   return CK_OK;
 }
 
+// U of the first pass, then (orders other than 64^3) room for the X . Y partials that a Krylov step
+// takes from the second pass's epilogue
 size_t kron_workspace_bytes(const ck_op* op, int nrhs) {
-  if (op->nfactors == 3) return (size_t)nrhs * op->n * sizeof(float);
-  return 0;
+  if (op->nfactors != 3) return 0;
+  const size_t off = kron_xy_offset(op, nrhs);
+  return off == 0 ? (size_t)nrhs * op->n * sizeof(float) : off + (size_t)nrhs * kron_nparts(op) * sizeof(float);
+}
+
+size_t kron_xy_offset(const ck_op* op, int nrhs) {
+  if (op->fdim[0] == 64 && op->fdim[1] == 64 && op->fdim[2] == 64) return 0;
+  return ((size_t)nrhs * op->n * sizeof(float) + 255) / 256 * 256;
 }
 
 int kron_dispatch(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, void* work,
@@ -1205,34 +1073,22 @@ int kron_dispatch(const ck_op* op, int nrhs, const float* X, int64_t ldx, float*
     prod *= op->fdim[i];
   }
   if (prod != op->n) return CK_ERR_BAD_ARG;
-  const size_t ldsA = 3 * 64 * KP * sizeof(float);
-  const size_t ldsB = 2 * 64 * KP * sizeof(float);
   if (d == 2) {
     if (partials) return CK_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL((kron_pass_a<true>), dim3(1, nrhs), dim3(256), ldsA, s, 1, op->fdim[0], op->fdim[1],
-                       op->factor[0], op->factor[1], X, ldx, Y, ldy, op->scale, op->shift, done);
-    CK_CHECK_LAUNCH();
-    return CK_OK;
+    return kron_any_apply(op, nrhs, X, ldx, Y, ldy, nullptr, done, nullptr, 0, s);
   }
-  if (work_bytes < kron_workspace_bytes(op, nrhs) || !work) return CK_ERR_WORKSPACE;
+  if (work_bytes < (size_t)nrhs * op->n * sizeof(float) || !work) return CK_ERR_WORKSPACE;
   if (kron64_eligible(op, X, ldx, Y, ldy))
     return kron64_apply_f32(op, nrhs, X, ldx, Y, ldy, work, work_bytes, done, partials, nparts, s);
-  float* U = static_cast<float*>(work);
-  const int n1 = op->fdim[0], n2 = op->fdim[1], n3 = op->fdim[2];
-  const int plane = n2 * n3;
-  hipLaunchKernelGGL((kron_pass_a<false>), dim3(n1, nrhs), dim3(256), ldsA, s, n1, n2, n3, op->factor[1],
-                     op->factor[2], X, ldx, U, (int64_t)op->n, 1.f, 0.f, done);
-  const int tiles = (plane + 63) / 64;
-  if (partials && nparts != tiles) return CK_ERR_BAD_ARG;
-  hipLaunchKernelGGL(kron_pass_b, dim3(tiles, nrhs), dim3(256), ldsB, s, n1, plane, op->factor[0], U,
-                     (int64_t)op->n, X, ldx, Y, ldy, op->scale, op->shift, partials, nparts, done);
-  CK_CHECK_LAUNCH();
-  return CK_OK;
+  // (64^3 with unaligned vectors or factors: kron_nparts counts kron64_pass_b4's tiles)
+  if (partials && (kron_xy_offset(op, nrhs) == 0 || nparts != kron_nparts(op))) return CK_ERR_UNSUPPORTED;
+  return kron_any_apply(op, nrhs, X, ldx, Y, ldy, static_cast<float*>(work), done, partials, nparts, s);
 }
 
 int kron_nparts(const ck_op* op) {
   if (op->nfactors != 3) return 0;
-  return (op->fdim[1] * op->fdim[2] + 63) / 64;
+  const int plane = op->fdim[1] * op->fdim[2];
+  return kron_xy_offset(op, 1) == 0 ? plane / 64 : kron_any_nparts(plane);
 }
 
 int op_apply_internal(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, void* work,

@@ -18,6 +18,11 @@ int kron_dispatch(const ck_op* op, int nrhs, const float* X, int64_t ldx, float*
                   size_t work_bytes, const int* done, float* partials, int nparts, hipStream_t s);
 int kron_nparts(const ck_op* op);
 size_t kron_workspace_bytes(const ck_op* op, int nrhs);
+// Where the operator's workspace has room for those partials (0: 64^3, which has none).
+size_t kron_xy_offset(const ck_op* op, int nrhs);
+int kron_any_nparts(int plane);
+int kron_any_apply(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, float* U,
+                   const int* done, float* partials, int nparts, hipStream_t s);
 
 bool kron64_eligible(const ck_op* op, const void* X, int64_t ldx, const void* Y, int64_t ldy);
 int kron64_apply_f32(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, void* work,
