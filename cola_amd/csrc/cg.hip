@@ -870,10 +870,9 @@ __global__ __launch_bounds__(256) void wbf_z_kernel(int64_t n, int nrhs, const f
 }
 
 bool wb_fused_ok(const ck_op* A, const ck_op* P, int nrhs, const float* p, int64_t ld, size_t work_bytes) {
-  auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   return P && A->kind == CK_OP_DENSE_F32 && P->kind == CK_OP_WOODBURY_INV && nrhs >= 3 && nrhs <= 8 &&
-         P->rank >= 1 && P->rank <= 64 && P->lda >= P->rank && P->a && P->aux && A->n % 4 == 0 && A->lda % 4 == 0 &&
-         ld % 4 == 0 && al16(A->a) && al16(p) && work_bytes >= wb_fused_bytes(A->n, nrhs, P->rank);
+         P->rank >= 1 && P->rank <= 64 && P->lda >= P->rank && P->a && P->aux &&
+         work_bytes >= wb_fused_bytes(A->n, nrhs, P->rank);
 }
 
 // nsteps steps; with last_partial the final one stops after the x/r update
@@ -902,8 +901,7 @@ int cg_iterate(const ck_op* A, const ck_op* P, int32_t nrhs, float* x, float* r,
   // dense A with a Woodbury P: the fused step (dense_apply_xy, wbf_*) in P's workspace
   const bool fuse_wb = !fuse_kron && wb_fused_ok(A, P, nrhs, p, ld, work_bytes);
   const bool dense_xy = !fuse_kron && !fuse_wb && A->kind == CK_OP_DENSE_F32 && nrhs >= 3 && nrhs <= 8 && work &&
-                        work_bytes >= dense_xy_bytes(n, nrhs) && n % 4 == 0 && A->lda % 4 == 0 && ld % 4 == 0 &&
-                        (reinterpret_cast<uintptr_t>(A->a) & 15) == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
+                        work_bytes >= dense_xy_bytes(n, nrhs);
   // CSR A: p.Ap partials from the SpMV's epilogue, into
   // the head of the workspace like dense_xy
   const bool csr_xy = !fuse_kron && !fuse_wb && !dense_xy && A->kind == CK_OP_CSR_F32 && work &&

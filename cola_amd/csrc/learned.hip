@@ -941,61 +941,17 @@ __global__ __launch_bounds__(256) void rbf_dense_kernel(int n, int dim, const fl
 }
 
 // ------------------------------------------------------- dense apply, fp64 vectors
-constexpr int kF64Rows = 8;  // rows per wave
-constexpr int kF64NB = 8;    // rhs per pass
+constexpr int kF64NB = 8;  // rhs per pass
 
-__global__ __launch_bounds__(256) void dense_f64acc_kernel(int n, const float* __restrict__ A, int64_t lda,
-                                                           const double* __restrict__ X, int64_t ldx,
-                                                           double* __restrict__ Y, int64_t ldy, int nb, double scale,
-                                                           double shift) {
-  __shared__ double xs[kF64NB][256];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row0 = blockIdx.x * (4 * kF64Rows) + wave * kF64Rows;
-  double acc[kF64Rows][kF64NB];
-#pragma unroll
-  for (int r = 0; r < kF64Rows; ++r)
-#pragma unroll
-    for (int b = 0; b < kF64NB; ++b) acc[r][b] = 0.0;
-  for (int j0 = 0; j0 < n; j0 += 256) {
-    __syncthreads();
-    for (int e = threadIdx.x; e < kF64NB * 256; e += 256) {
-      const int b = e / 256, jj = e % 256;
-      xs[b][jj] = (b < nb && j0 + jj < n) ? X[(int64_t)b * ldx + j0 + jj] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kF64Rows; ++r) {
-      const int row = row0 + r;
-      if (row >= n) break;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int jj = q * 64 + lane;
-        const int j = j0 + jj;
-        const double a = j < n ? (double)A[(int64_t)row * lda + j] : 0.0;
-#pragma unroll
-        for (int b = 0; b < kF64NB; ++b) acc[r][b] = fma(a, xs[b][jj], acc[r][b]);
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < kF64Rows; ++r) {
-#pragma unroll
-    for (int b = 0; b < kF64NB; ++b) {
-      const double s = wave_sum(acc[r][b]);
-      const int row = row0 + r;
-      if (lane == 0 && row < n && b < nb) Y[(int64_t)b * ldy + row] = scale * s + shift * X[(int64_t)b * ldx + row];
-    }
-  }
-}
-
-// The same product with every load unconditional (rows and columns clamped, the extra terms
-// multiplied by zero) and the x chunk staged once per block for all of its rows: eight waves of
-// four rows share one FP64 copy of X[:, c0:c0+512) in LDS; A is streamed with non-temporal
-// float4 loads.  Requires n % 4 == 0, 16-byte aligned rows of A and X, lda % 4 == 0 and
-// ldx % 2 == 0 (the entry point keeps dense_f64acc_kernel for the rest).
+// Every load is unconditional (rows and columns clamped, the extra terms multiplied by zero) and
+// the x chunk staged once per block for all of its rows: eight waves of four rows share one FP64 copy
+// of X[:, c0:c0+512) in LDS; A is streamed with non-temporal 16-byte loads, which need dword
+// alignment only, so odd orders and leading dimensions take the same path (12289 x 8: 1616 -> 164 us against one column per lane); the
+// last n % 4 columns are added one per lane.
 constexpr int kF64Chunk = 512;
 constexpr int kF64Waves = 8;
-typedef float f64acc_f4 __attribute__((ext_vector_type(4)));
+typedef float f64acc_f4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef double f64acc_d2 __attribute__((ext_vector_type(2), aligned(8)));
 
 __global__ __launch_bounds__(64 * kF64Waves) __attribute__((amdgpu_waves_per_eu(4))) void dense_f64acc_lds_kernel(int n, const float* __restrict__ A,
                                                                          int64_t lda, const double* __restrict__ X,
@@ -1019,13 +975,15 @@ __global__ __launch_bounds__(64 * kF64Waves) __attribute__((amdgpu_waves_per_eu(
     arow[r] = A + (int64_t)row * lda;
     rmask[r] = row0 + r < n ? 1.f : 0.f;
   }
-  for (int c0 = 0; c0 < n; c0 += kF64Chunk) {
-    const int cn = n - c0 < kF64Chunk ? n - c0 : kF64Chunk;  // a multiple of 4
+  const int n4 = n & ~3;
+  for (int c0 = 0; c0 < n4; c0 += kF64Chunk) {
+    const int cn = n4 - c0 < kF64Chunk ? n4 - c0 : kF64Chunk;  // a multiple of 4
     __syncthreads();
     for (int e = threadIdx.x; e < kF64NB * (kF64Chunk / 2); e += 64 * kF64Waves) {
       const int b = e / (kF64Chunk / 2), j2 = e % (kF64Chunk / 2);
-      xs[b][j2] = (b < nb && 2 * j2 < cn) ? *reinterpret_cast<const double2*>(X + (int64_t)b * ldx + c0 + 2 * j2)
-                                          : make_double2(0.0, 0.0);
+      f64acc_d2 v = {0.0, 0.0};
+      if (b < nb && 2 * j2 < cn) v = *reinterpret_cast<const f64acc_d2*>(X + (int64_t)b * ldx + c0 + 2 * j2);
+      xs[b][j2] = make_double2(v.x, v.y);
     }
     __syncthreads();
 #pragma unroll
@@ -1052,6 +1010,14 @@ __global__ __launch_bounds__(64 * kF64Waves) __attribute__((amdgpu_waves_per_eu(
           acc[r][b] = t;
         }
       }
+    }
+  }
+  if (lane < n - n4) {
+#pragma unroll
+    for (int b = 0; b < kF64NB; ++b) {
+      const double xv = X[(int64_t)(b < nb ? b : 0) * ldx + n4 + lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r][b] = fma((double)arow[r][n4 + lane], xv, acc[r][b]);
     }
   }
 #pragma unroll
@@ -1224,18 +1190,10 @@ int ck_dense_apply_f64acc(int64_t n, const float* A, int64_t lda, double scale, 
                           const double* X, int64_t ldx, double* Y, int64_t ldy, void* stream) {
   if (n < 1 || n > 0x7FFFFFFF || !A || lda < n || nrhs < 1 || !X || !Y || ldx < n || ldy < n) return CK_ERR_BAD_ARG;
   hipStream_t s = (hipStream_t)stream;
-  auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-  const bool vec = n % 4 == 0 && lda % 4 == 0 && ldx % 2 == 0 && al16(A) && al16(X);
-  const unsigned grid = (unsigned)cdiv(n, 4 * kF64Rows);
-  const unsigned grid_lds = (unsigned)cdiv(n, 4 * kF64Waves);
   for (int b0 = 0; b0 < nrhs; b0 += kF64NB) {
     const int nb = nrhs - b0 < kF64NB ? nrhs - b0 : kF64NB;
-    if (vec)
-      hipLaunchKernelGGL(dense_f64acc_lds_kernel, dim3(grid_lds), dim3(64 * kF64Waves), 0, s, (int)n, A, lda,
-                         X + (int64_t)b0 * ldx, ldx, Y + (int64_t)b0 * ldy, ldy, nb, scale, shift);
-    else
-      hipLaunchKernelGGL(dense_f64acc_kernel, dim3(grid), dim3(256), 0, s, (int)n, A, lda, X + (int64_t)b0 * ldx,
-                         ldx, Y + (int64_t)b0 * ldy, ldy, nb, scale, shift);
+    hipLaunchKernelGGL(dense_f64acc_lds_kernel, dim3((unsigned)cdiv(n, 4 * kF64Waves)), dim3(64 * kF64Waves), 0, s,
+                       (int)n, A, lda, X + (int64_t)b0 * ldx, ldx, Y + (int64_t)b0 * ldy, ldy, nb, scale, shift);
   }
   CK_CHECK_LAUNCH();
   return CK_OK;

@@ -16,11 +16,17 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 namespace {
 
 // ============================================================== dense fp32
+// Rows and vectors start at any multiple of four bytes: the hardware takes dword-aligned 16-byte
+// loads, so an odd order or leading dimension costs one more cache line per kilobyte of row, not
+// four times the load instructions.  The last n % 4 columns are added one per lane.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// One or two rhs: x stays in the caches and every wave reads it for itself.
 template <int NB, int ROWS>
 __global__ __launch_bounds__(256) void dense_f32_kernel(int n, const float* __restrict__ A, int64_t lda,
                                                         const float* __restrict__ X, int64_t ldx, float* __restrict__ Y,
                                                         int64_t ldy, int nbr, float scale, float shift,
-                                                        const int* __restrict__ done, bool vec) {
+                                                        const int* __restrict__ done) {
   if (done && *done) return;
   const int lane = threadIdx.x & 63;
   const int wave = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
@@ -31,41 +37,30 @@ __global__ __launch_bounds__(256) void dense_f32_kernel(int n, const float* __re
   for (int r = 0; r < ROWS; ++r)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[r][b] = 0.f;
-
-  if (vec) {
-    for (int j = lane * 4; j < n; j += 256) {
-      float4 xv[NB];
+  const int n4 = n & ~3;
+  for (int j = lane * 4; j < n4; j += 256) {
+    f4u xv[NB];
 #pragma unroll
-      for (int b = 0; b < NB; ++b)
-        xv[b] = (b < nbr) ? *reinterpret_cast<const float4*>(X + b * ldx + j) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int b = 0; b < NB; ++b) xv[b] = *reinterpret_cast<const f4u*>(X + (b < nbr ? b : 0) * ldx + j);
 #pragma unroll
-      for (int r = 0; r < ROWS; ++r) {
-        if (row0 + r < n) {
-          const float4 a = *reinterpret_cast<const float4*>(A + (int64_t)(row0 + r) * lda + j);
+    for (int r = 0; r < ROWS; ++r) {
+      if (row0 + r < n) {
+        const f4u a = *reinterpret_cast<const f4u*>(A + (int64_t)(row0 + r) * lda + j);
 #pragma unroll
-          for (int b = 0; b < NB; ++b) {
-            acc[r][b] = fmaf(a.x, xv[b].x, acc[r][b]);
-            acc[r][b] = fmaf(a.y, xv[b].y, acc[r][b]);
-            acc[r][b] = fmaf(a.z, xv[b].z, acc[r][b]);
-            acc[r][b] = fmaf(a.w, xv[b].w, acc[r][b]);
-          }
-        }
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[r][b] = fmaf(a[e], xv[b][e], acc[r][b]);
       }
     }
-  } else {
-    for (int j = lane; j < n; j += 64) {
-      float xv[NB];
+  }
+  if (lane < n - n4) {
 #pragma unroll
-      for (int b = 0; b < NB; ++b) xv[b] = (b < nbr) ? X[b * ldx + j] : 0.f;
+    for (int r = 0; r < ROWS; ++r)
+      if (row0 + r < n) {
+        const float a = A[(int64_t)(row0 + r) * lda + n4 + lane];
 #pragma unroll
-      for (int r = 0; r < ROWS; ++r) {
-        if (row0 + r < n) {
-          const float a = A[(int64_t)(row0 + r) * lda + j];
-#pragma unroll
-          for (int b = 0; b < NB; ++b) acc[r][b] = fmaf(a, xv[b], acc[r][b]);
-        }
+        for (int b = 0; b < NB; ++b) acc[r][b] = fmaf(a, X[(b < nbr ? b : 0) * ldx + n4 + lane], acc[r][b]);
       }
-    }
   }
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
@@ -80,6 +75,169 @@ __global__ __launch_bounds__(256) void dense_f32_kernel(int n, const float* __re
       }
     }
   }
+}
+
+// Three and more rhs: the eight waves of a block share one copy of X[:, c0 : c0 + 1024) in LDS instead
+// of each wave re-reading it from L2, so per block and chunk the traffic is 8 * ROWS rows of A from HBM
+// against one NB x 1024 slice of X.  A is streamed with non-temporal loads (it is read once per product
+// and would otherwise evict X and the vectors of the surrounding solver from the caches).  The pieces
+// of A and of X that a wave holds are replaced by the next chunk's as soon as they are used, so a
+// whole chunk of rows is always in flight.  HBM bound at large n; at small n a launch is latency
+// and needs blocks: dense_rows(n) rows each, 8, 16 or 32.
+// Measured (before -> now): 20001^2, 4 / 8 / 16 rhs 537 -> 270, 580 -> 292, 947 -> 357 us (odd orders took
+// 4-byte loads and re-read x per wave); 16384^2 x 8 167 -> 165 us (6.5 TB/s), x 16 251 -> 219 us;
+// 2500^2 x 4 15.2 -> 6.6 us, 8192^2 x 8 62 -> 49 us.
+constexpr int kDenseChunk = 1024;
+constexpr int kDenseWaves = 8;
+
+// With astride != 0 the launch is batched over blockIdx.y: block row b multiplies its own
+// matrix (A + b * astride elements) with its own vectors (X + b * xbs, Y + b * ybs).
+template <int NB, int ROWS>
+__global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_eu(4))) void dense_f32_lds_kernel(int n, const float* __restrict__ A,
+                                                                         int64_t lda, const float* __restrict__ X,
+                                                                         int64_t ldx, float* __restrict__ Y,
+                                                                         int64_t ldy, int nbr, float scale,
+                                                                         float shift, const int* __restrict__ done,
+                                                                         int64_t astride, int64_t xbs, int64_t ybs,
+                                                                         float* __restrict__ xy_part = nullptr) {
+  if (done && *done) return;
+  A += blockIdx.y * astride;
+  X += blockIdx.y * xbs;
+  Y += blockIdx.y * ybs;
+  constexpr int Q = kDenseChunk / 256;                               // pieces of a row per lane and chunk
+  constexpr int XQ = (NB * (kDenseChunk / 4) + 64 * kDenseWaves - 1) / (64 * kDenseWaves);  // of X per thread
+  __shared__ float4 xs[NB][kDenseChunk / 4];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // rows and their pointers stay scalar
+  const int row0 = blockIdx.x * (kDenseWaves * ROWS) + wave * ROWS;
+  const int n4 = n & ~3;
+  const float* arow[ROWS];  // rows past the last: its copy, never stored
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) arow[r] = A + (int64_t)(row0 + r < n ? row0 + r : n - 1) * lda;
+  float acc[ROWS][NB];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[r][b] = 0.f;
+  f4u a[Q][ROWS], xn[XQ];
+  auto fetch_a = [&](int c0, int q) {
+    const int j = c0 + q * 256 + lane * 4, c = j < n4 ? j : n4 - 4;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) a[q][r] = __builtin_nontemporal_load(reinterpret_cast<const f4u*>(arow[r] + c));
+  };
+  auto fetch_x = [&](int c0) {
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) {
+      const int e = threadIdx.x + 64 * kDenseWaves * q, b = e / (kDenseChunk / 4), j = c0 + 4 * (e % (kDenseChunk / 4));
+      xn[q] = *reinterpret_cast<const f4u*>(X + (int64_t)(b < nbr ? b : 0) * ldx + (j < n4 ? j : n4 - 4));
+    }
+  };
+  // 4 rows x 8 rhs have no registers left to hold the next slice of X: it is loaded where it is stored
+  constexpr bool XP = ROWS * NB < 32;
+  if (n4 > 0) {
+    if (XP) fetch_x(0);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) fetch_a(0, q);
+  }
+  for (int c0 = 0; c0 < n4; c0 += kDenseChunk) {
+    if (!XP) fetch_x(c0);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) {
+      const int e = threadIdx.x + 64 * kDenseWaves * q;
+      if (e < NB * (kDenseChunk / 4))
+        xs[e / (kDenseChunk / 4)][e % (kDenseChunk / 4)] = make_float4(xn[q][0], xn[q][1], xn[q][2], xn[q][3]);
+    }
+    __syncthreads();
+    const bool more = c0 + kDenseChunk < n4;
+    if (XP && more) fetch_x(c0 + kDenseChunk);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      if (c0 + q * 256 + lane * 4 < n4) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const float4 xv = xs[b][q * 64 + lane];
+#pragma unroll
+          for (int r = 0; r < ROWS; ++r) {
+            float t = acc[r][b];
+            t = fmaf(a[q][r][0], xv.x, t);
+            t = fmaf(a[q][r][1], xv.y, t);
+            t = fmaf(a[q][r][2], xv.z, t);
+            t = fmaf(a[q][r][3], xv.w, t);
+            acc[r][b] = t;
+          }
+        }
+      }
+      if (more) fetch_a(c0 + kDenseChunk, q);
+    }
+  }
+  if (lane < n - n4) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const float xv = X[(int64_t)(b < nbr ? b : 0) * ldx + n4 + lane];
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) acc[r][b] = fmaf(arow[r][n4 + lane], xv, acc[r][b]);
+    }
+  }
+  // lane L < ROWS * NB owns (row0 + L / NB, rhs L % NB): the wave-wide sums give it Y
+  const int my_r = lane / NB, my_b = lane % NB;
+  const bool mine = lane < ROWS * NB && my_b < nbr && row0 + my_r < n;
+  const bool need_x = shift != 0.f || xy_part != nullptr;
+  const float my_x = mine && need_x ? X[(int64_t)my_b * ldx + row0 + my_r] : 0.f;
+  float my_y = 0.f;
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const float sum = wave_sum(acc[r][b]);
+      my_y = lane == r * NB + b ? sum : my_y;
+    }
+  }
+  my_y *= scale;
+  if (shift != 0.f) my_y = fmaf(shift, my_x, my_y);
+  if (mine) Y[(int64_t)my_b * ldy + row0 + my_r] = my_y;
+  if (xy_part) {
+    // per-block partial sums of X . Y (the CG step's p.Ap), rows then waves in index order
+    __shared__ float xys[kDenseWaves][ROWS * NB];
+    if (lane < ROWS * NB) xys[wave][lane] = mine ? my_x * my_y : 0.f;
+    __syncthreads();
+    if (threadIdx.x < nbr) {
+      float t = 0.f;
+      for (int w = 0; w < kDenseWaves; ++w)
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) t += xys[w][r * NB + threadIdx.x];
+      xy_part[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = t;
+    }
+  }
+}
+
+// One launch of up to 8 rhs (16 without partials): dense_rows(n) rows per block, half of them at 16.
+void dense_f32_lds(int n, const float* A, int64_t lda, const float* X, int64_t ldx, float* Y, int64_t ldy, int nb,
+                   float scale, float shift, const int* done, float* xy_part, hipStream_t s) {
+  const int rows = dense_rows(n) / kDenseWaves;
+#define CK_DENSE(NB_, ROWS_)                                                                                        \
+  hipLaunchKernelGGL((dense_f32_lds_kernel<NB_, ROWS_>), dim3((unsigned)cdiv(n, kDenseWaves * (ROWS_))),            \
+                     dim3(64 * kDenseWaves), 0, s, n, A, lda, X, ldx, Y, ldy, nb, scale, shift, done, (int64_t)0,   \
+                     (int64_t)0, (int64_t)0, xy_part)
+#define CK_DENSE_ROWS(NB_)  \
+  do {                      \
+    if (rows == 1)          \
+      CK_DENSE(NB_, 1);     \
+    else if (rows == 2)     \
+      CK_DENSE(NB_, 2);     \
+    else                    \
+      CK_DENSE(NB_, 4);     \
+  } while (0)
+  if (nb <= 4)
+    CK_DENSE_ROWS(4);
+  else if (nb <= 8)
+    CK_DENSE_ROWS(8);
+  else if (rows == 1)
+    CK_DENSE(16, 1);
+  else
+    CK_DENSE(16, 2);
+#undef CK_DENSE_ROWS
+#undef CK_DENSE
 }
 
 // bf16 stored matrix, fp32 vectors and accumulation (vector path; the MFMA
@@ -151,39 +309,19 @@ __global__ __launch_bounds__(256) void dense_bf16_kernel(int n, const uint16_t* 
   }
 }
 
-// Multi-rhs dense product with the vector chunk staged in LDS: the eight waves of a
-// block share one copy of X[:, c0:c0+1024) instead of each wave re-reading it from
-// L2, so per block and chunk the traffic is 8*ROWS rows of A from HBM against one
-// NB x 1024 slice of X.  A is streamed with non-temporal loads (it is read once per
-// product and would otherwise evict X and the vectors of the surrounding solver from
-// the caches); measured on MI355X at 16384^2 x 8 rhs: 6.3 TB/s with 8 waves x 4 rows
-// and non-temporal loads, 4.6 TB/s with 4 waves x 8 rows and ordinary loads.
-// Requires n % 4 == 0 (fp32) or n % 8 == 0 (bf16) and 16-byte aligned rows; lanes take
-// 4 (fp32) or 8 (bf16) consecutive columns.
-constexpr int kDenseChunk = 1024;
-constexpr int kDenseWaves = 8;
-typedef float f32x4_nt __attribute__((ext_vector_type(4)));
+// Multi-rhs product of a bf16 matrix, the vector chunk staged in LDS as in dense_f32_lds_kernel.
+// Requires n % 8 == 0 and 16-byte aligned rows; lanes take 8 consecutive columns.
 typedef float f32x2_nt __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4_nt __attribute__((ext_vector_type(4)));
 
-// With astride != 0 the launch is batched over blockIdx.y: block row b multiplies its own
-// matrix (A + b * astride elements) with its own vectors (X + b * xbs, Y + b * ybs).
-template <int NB, int ROWS, bool BF>
-__global__ __launch_bounds__(64 * kDenseWaves) void dense_lds_kernel(int n, const void* __restrict__ Av, int64_t lda,
-                                                                     const float* __restrict__ X, int64_t ldx,
-                                                                     float* __restrict__ Y, int64_t ldy, int nbr,
-                                                                     float scale, float shift,
-                                                                     const int* __restrict__ done, int64_t astride,
-                                                                     int64_t xbs, int64_t ybs,
-                                                                     float* __restrict__ xy_part = nullptr) {
+template <int NB, int ROWS>
+__global__ __launch_bounds__(64 * kDenseWaves) void dense_bf16_lds_kernel(int n, const uint16_t* __restrict__ A,
+                                                                          int64_t lda, const float* __restrict__ X,
+                                                                          int64_t ldx, float* __restrict__ Y,
+                                                                          int64_t ldy, int nbr, float scale,
+                                                                          float shift,
+                                                                          const int* __restrict__ done) {
   if (done && *done) return;
-  {
-    const int64_t pb = blockIdx.y;
-    Av = BF ? static_cast<const void*>(static_cast<const uint16_t*>(Av) + pb * astride)
-            : static_cast<const void*>(static_cast<const float*>(Av) + pb * astride);
-    X += pb * xbs;
-    Y += pb * ybs;
-  }
   __shared__ float4 xs[NB][kDenseChunk / 4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row0 = blockIdx.x * (kDenseWaves * ROWS) + wave * ROWS;
@@ -193,7 +331,7 @@ __global__ __launch_bounds__(64 * kDenseWaves) void dense_lds_kernel(int n, cons
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[r][b] = 0.f;
   for (int c0 = 0; c0 < n; c0 += kDenseChunk) {
-    const int cn = n - c0 < kDenseChunk ? n - c0 : kDenseChunk;  // multiple of 4
+    const int cn = n - c0 < kDenseChunk ? n - c0 : kDenseChunk;  // multiple of 8
     __syncthreads();
     for (int e = threadIdx.x; e < NB * (kDenseChunk / 4); e += 64 * kDenseWaves) {
       const int b = e / (kDenseChunk / 4), j4 = e % (kDenseChunk / 4);
@@ -201,107 +339,52 @@ __global__ __launch_bounds__(64 * kDenseWaves) void dense_lds_kernel(int n, cons
                                             : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     __syncthreads();
-    if (BF) {
-      const uint16_t* A = static_cast<const uint16_t*>(Av);
 #pragma unroll
-      for (int q = 0; q < kDenseChunk / 512; ++q) {
-        const int j = q * 512 + lane * 8;
-        if (j < cn) {
-          uint4 w[ROWS];
+    for (int q = 0; q < kDenseChunk / 512; ++q) {
+      const int j = q * 512 + lane * 8;
+      if (j < cn) {
+        uint4 w[ROWS];
 #pragma unroll
-          for (int r = 0; r < ROWS; ++r) {
-            if (row0 + r < n) {
-              const u32x4_nt v = __builtin_nontemporal_load(
-                  reinterpret_cast<const u32x4_nt*>(A + (int64_t)(row0 + r) * lda + c0 + j));
-              w[r] = make_uint4(v.x, v.y, v.z, v.w);
-            } else {
-              w[r] = make_uint4(0u, 0u, 0u, 0u);
-            }
-          }
-#pragma unroll
-          for (int b = 0; b < NB; ++b) {
-            const float4 x0 = xs[b][j / 4], x1 = xs[b][j / 4 + 1];
-#pragma unroll
-            for (int r = 0; r < ROWS; ++r) {
-              float t = acc[r][b];
-              t = fmaf(__uint_as_float(w[r].x << 16), x0.x, t);
-              t = fmaf(__uint_as_float(w[r].x & 0xFFFF0000u), x0.y, t);
-              t = fmaf(__uint_as_float(w[r].y << 16), x0.z, t);
-              t = fmaf(__uint_as_float(w[r].y & 0xFFFF0000u), x0.w, t);
-              t = fmaf(__uint_as_float(w[r].z << 16), x1.x, t);
-              t = fmaf(__uint_as_float(w[r].z & 0xFFFF0000u), x1.y, t);
-              t = fmaf(__uint_as_float(w[r].w << 16), x1.z, t);
-              t = fmaf(__uint_as_float(w[r].w & 0xFFFF0000u), x1.w, t);
-              acc[r][b] = t;
-            }
+        for (int r = 0; r < ROWS; ++r) {
+          if (row0 + r < n) {
+            const u32x4_nt v = __builtin_nontemporal_load(
+                reinterpret_cast<const u32x4_nt*>(A + (int64_t)(row0 + r) * lda + c0 + j));
+            w[r] = make_uint4(v.x, v.y, v.z, v.w);
+          } else {
+            w[r] = make_uint4(0u, 0u, 0u, 0u);
           }
         }
-      }
-    } else {
-      const float* A = static_cast<const float*>(Av);
 #pragma unroll
-      for (int q = 0; q < kDenseChunk / 256; ++q) {
-        const int j = q * 256 + lane * 4;
-        if (j < cn) {
-          float4 a[ROWS];
+        for (int b = 0; b < NB; ++b) {
+          const float4 x0 = xs[b][j / 4], x1 = xs[b][j / 4 + 1];
 #pragma unroll
           for (int r = 0; r < ROWS; ++r) {
-            if (row0 + r < n) {
-              const f32x4_nt v = __builtin_nontemporal_load(
-                  reinterpret_cast<const f32x4_nt*>(A + (int64_t)(row0 + r) * lda + c0 + j));
-              a[r] = make_float4(v.x, v.y, v.z, v.w);
-            } else {
-              a[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-          }
-#pragma unroll
-          for (int b = 0; b < NB; ++b) {
-            const float4 xv = xs[b][j / 4];
-#pragma unroll
-            for (int r = 0; r < ROWS; ++r) {
-              float t = acc[r][b];
-              t = fmaf(a[r].x, xv.x, t);
-              t = fmaf(a[r].y, xv.y, t);
-              t = fmaf(a[r].z, xv.z, t);
-              t = fmaf(a[r].w, xv.w, t);
-              acc[r][b] = t;
-            }
+            float t = acc[r][b];
+            t = fmaf(__uint_as_float(w[r].x << 16), x0.x, t);
+            t = fmaf(__uint_as_float(w[r].x & 0xFFFF0000u), x0.y, t);
+            t = fmaf(__uint_as_float(w[r].y << 16), x0.z, t);
+            t = fmaf(__uint_as_float(w[r].y & 0xFFFF0000u), x0.w, t);
+            t = fmaf(__uint_as_float(w[r].z << 16), x1.x, t);
+            t = fmaf(__uint_as_float(w[r].z & 0xFFFF0000u), x1.y, t);
+            t = fmaf(__uint_as_float(w[r].w << 16), x1.z, t);
+            t = fmaf(__uint_as_float(w[r].w & 0xFFFF0000u), x1.w, t);
+            acc[r][b] = t;
           }
         }
       }
     }
   }
-  // X . Y partials: lane L < ROWS * NB owns (row0 + L / NB, rhs L % NB) and loads its X value
-  // once; the wave-wide sums give it Y
-  const int my_r = lane / NB, my_b = lane % NB;
-  const bool mine = xy_part && lane < ROWS * NB && my_b < nbr && row0 + my_r < n;
-  const float my_x = mine ? X[(int64_t)my_b * ldx + row0 + my_r] : 0.f;
-  float my_y = 0.f;
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const float sum = wave_sum(acc[r][b]);
       const int row = row0 + r;
-      float y = scale * sum;
       if (lane == 0 && b < nbr && row < n) {
+        float y = scale * sum;
         if (shift != 0.f) y = fmaf(shift, X[(int64_t)b * ldx + row], y);
         Y[(int64_t)b * ldy + row] = y;
       }
-      if (lane == r * NB + b) my_y = shift != 0.f ? fmaf(shift, my_x, scale * sum) : y;
-    }
-  }
-  if (xy_part) {
-    // per-block partial sums of X . Y (the CG step's p.Ap), rows then waves in index order
-    __shared__ float xys[kDenseWaves][ROWS * NB];
-    if (lane < ROWS * NB) xys[wave][lane] = mine ? my_x * my_y : 0.f;
-    __syncthreads();
-    if (threadIdx.x < nbr) {
-      float t = 0.f;
-      for (int w = 0; w < kDenseWaves; ++w)
-#pragma unroll
-        for (int r = 0; r < ROWS; ++r) t += xys[w][r * NB + threadIdx.x];
-      xy_part[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = t;
     }
   }
 }
@@ -556,7 +639,7 @@ __global__ __launch_bounds__(64 * kSymRedWaves) void dense_sym_reduce(int n, con
     if (shift != 0.f) y = fmaf(shift, x, y);
     Y[(int64_t)b * ldy + row] = y;
     if (xy_part) {
-      // two partials of 32 rows each, as the full product's epilogue writes them
+      // two partials of 32 rows each
       float v = x * y;
       v += dpp_f32<0xB1>(v);
       v += dpp_f32<0x4E>(v);
@@ -566,8 +649,12 @@ __global__ __launch_bounds__(64 * kSymRedWaves) void dense_sym_reduce(int n, con
       const float h0 = readlane_f32(v, 0) + readlane_f32(v, 16);
       const float h1 = readlane_f32(v, 32) + readlane_f32(v, 48);
       if (il == 0) {
-        xy_part[(int64_t)b * (n / 32) + 2 * s] = h0;
-        xy_part[(int64_t)b * (n / 32) + 2 * s + 1] = h1;
+        // dense_xy_nparts(n) slots, 64 / dense_rows(n) of them per block: what is left over is zero
+        const int per = 64 / dense_rows(n);
+        float* dst = xy_part + ((int64_t)b * (n / 64) + s) * per;
+        dst[0] = h0;
+        dst[1] = h1;
+        for (int k = 2; k < per; ++k) dst[k] = 0.f;
       }
     }
   }
@@ -632,63 +719,49 @@ int dense_dispatch(const ck_op* op, int nrhs, const float* X, int64_t ldx, float
   if (work && work_bytes > off && sym_eligible(op, X, ldx, work_bytes - off))
     return dense_sym_apply(op, nrhs, X, ldx, Y, ldy, done, static_cast<char*>(work) + off, nullptr, s);
   const int n = op->n;
-  const bool bf16 = op->kind == CK_OP_DENSE_BF16;
+  if (op->kind == CK_OP_DENSE_F32) {
+    const float* A = static_cast<const float*>(op->a);
+    for (int b0 = 0; b0 < nrhs; b0 += 16) {
+      const int nb = nrhs - b0 < 16 ? nrhs - b0 : 16;
+      const float* Xb = X + b0 * ldx;
+      float* Yb = Y + b0 * ldy;
+      if (nb == 1)
+        hipLaunchKernelGGL((dense_f32_kernel<1, 1>), dim3((n + 3) / 4), dim3(256), 0, s, n, A, op->lda, Xb, ldx, Yb, ldy,
+                           nb, op->scale, op->shift, done);
+      else if (nb == 2)
+        hipLaunchKernelGGL((dense_f32_kernel<2, 2>), dim3((n + 7) / 8), dim3(256), 0, s, n, A, op->lda, Xb, ldx, Yb, ldy,
+                           nb, op->scale, op->shift, done);
+      else
+        dense_f32_lds(n, A, op->lda, Xb, ldx, Yb, ldy, nb, op->scale, op->shift, done, nullptr, s);
+    }
+    CK_CHECK_LAUNCH();
+    return CK_OK;
+  }
+  const uint16_t* A = static_cast<const uint16_t*>(op->a);
   auto aligned16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-  // float4 / uint4 loads need 16-byte aligned rows and vector starts
-  const bool vec = (n % 4 == 0) && (op->lda % 4 == 0) && (ldx % 4 == 0) && aligned16(op->a) && aligned16(X);
-  if (bf16 && ((n % 8) || (op->lda % 8) || (ldx % 4) || !aligned16(op->a) || !aligned16(X)))
-    return CK_ERR_UNSUPPORTED;
-  // LDS-staged path for 3+ rhs when rows and vectors allow 16-byte loads
-  const bool lds_ok = vec && (!bf16 || n % 8 == 0) && (ldx % 4 == 0) && nrhs >= 3;
+  // uint4 / float4 loads need 16-byte aligned rows and vector starts
+  if ((n % 8) || (op->lda % 8) || (ldx % 4) || !aligned16(op->a) || !aligned16(X)) return CK_ERR_UNSUPPORTED;
   for (int b0 = 0; b0 < nrhs; b0 += 16) {
     const int nb = nrhs - b0 < 16 ? nrhs - b0 : 16;
     const float* Xb = X + b0 * ldx;
     float* Yb = Y + b0 * ldy;
-    if (lds_ok && nb >= 3) {
 #define CK_DENSE_LDS(NB_, ROWS_)                                                                                  \
-  do {                                                                                                            \
-    const int grid = (n + kDenseWaves * (ROWS_)-1) / (kDenseWaves * (ROWS_));                                     \
-    if (bf16)                                                                                                     \
-      hipLaunchKernelGGL((dense_lds_kernel<NB_, ROWS_, true>), dim3(grid), dim3(64 * kDenseWaves), 0, s, n,      \
-                         op->a, op->lda, Xb, ldx, Yb, ldy, nb, op->scale, op->shift, done, (int64_t)0, (int64_t)0, \
-                         (int64_t)0);                                                                             \
-    else                                                                                                          \
-      hipLaunchKernelGGL((dense_lds_kernel<NB_, ROWS_, false>), dim3(grid), dim3(64 * kDenseWaves), 0, s, n,     \
-                         op->a, op->lda, Xb, ldx, Yb, ldy, nb, op->scale, op->shift, done, (int64_t)0, (int64_t)0, \
-                         (int64_t)0);                                                                             \
-  } while (0)
-      if (nb <= 4)
-        CK_DENSE_LDS(4, 4);
-      else if (nb <= 8)
-        CK_DENSE_LDS(8, 4);
-      else
-        CK_DENSE_LDS(16, 2);
-#undef CK_DENSE_LDS
-      continue;
-    }
-    // ROWS rows per wave: more rows reuse each loaded x chunk more often.
-    constexpr int WAVES = 4;
-#define CK_DENSE_LAUNCH(NB_, ROWS_)                                                                               \
-  do {                                                                                                            \
-    const int nwaves = (n + (ROWS_)-1) / (ROWS_);                                                                 \
-    const int grid = (nwaves + WAVES - 1) / WAVES;                                                                \
-    if (bf16)                                                                                                     \
-      hipLaunchKernelGGL((dense_bf16_kernel<NB_, ROWS_>), dim3(grid), dim3(64 * WAVES), 0, s, n,                  \
-                         (const uint16_t*)op->a, op->lda, Xb, ldx, Yb, ldy, nb, op->scale, op->shift, done);      \
-    else                                                                                                          \
-      hipLaunchKernelGGL((dense_f32_kernel<NB_, ROWS_>), dim3(grid), dim3(64 * WAVES), 0, s, n,                   \
-                         (const float*)op->a, op->lda, Xb, ldx, Yb, ldy, nb, op->scale, op->shift, done, vec);    \
-  } while (0)
+  hipLaunchKernelGGL((dense_bf16_lds_kernel<NB_, ROWS_>), dim3((unsigned)cdiv(n, kDenseWaves * (ROWS_))),         \
+                     dim3(64 * kDenseWaves), 0, s, n, A, op->lda, Xb, ldx, Yb, ldy, nb, op->scale, op->shift, done)
+#define CK_DENSE_LAUNCH(NB_, ROWS_)                                                                              \
+  hipLaunchKernelGGL((dense_bf16_kernel<NB_, ROWS_>), dim3((unsigned)cdiv(n, 4 * (ROWS_))), dim3(256), 0, s, n, A, \
+                     op->lda, Xb, ldx, Yb, ldy, nb, op->scale, op->shift, done)
     if (nb == 1)
       CK_DENSE_LAUNCH(1, 1);
     else if (nb == 2)
       CK_DENSE_LAUNCH(2, 2);
     else if (nb <= 4)
-      CK_DENSE_LAUNCH(4, 4);
+      CK_DENSE_LDS(4, 4);
     else if (nb <= 8)
-      CK_DENSE_LAUNCH(8, 4);
+      CK_DENSE_LDS(8, 4);
     else
-      CK_DENSE_LAUNCH(16, 2);
+      CK_DENSE_LDS(16, 2);
+#undef CK_DENSE_LDS
 #undef CK_DENSE_LAUNCH
   }
   CK_CHECK_LAUNCH();
@@ -1031,21 +1104,13 @@ namespace ck {
 // rhs); returns CK_ERR_UNSUPPORTED when the shapes fall outside that kernel
 int dense_apply_xy(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, int64_t ldy, const int* done,
                    float* xy_part, void* work, size_t work_bytes, hipStream_t s) {
-  auto aligned16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   const int n = op->n;
   const size_t off = dense_sym_offset(n, nrhs);
   if (work && work_bytes > off && nrhs >= 1 && nrhs <= 8 && sym_eligible(op, X, ldx, work_bytes - off))
     return dense_sym_apply(op, nrhs, X, ldx, Y, ldy, done, static_cast<char*>(work) + off, xy_part, s);
-  if (op->kind != CK_OP_DENSE_F32 || nrhs < 3 || nrhs > 8 || n % 4 || op->lda % 4 || ldx % 4 || !aligned16(op->a) ||
-      !aligned16(X))
-    return CK_ERR_UNSUPPORTED;
-  const int grid = dense_xy_nparts(n);
-  if (nrhs <= 4)
-    hipLaunchKernelGGL((dense_lds_kernel<4, 4, false>), dim3(grid), dim3(64 * kDenseWaves), 0, s, n, op->a, op->lda, X,
-                       ldx, Y, ldy, nrhs, op->scale, op->shift, done, (int64_t)0, (int64_t)0, (int64_t)0, xy_part);
-  else
-    hipLaunchKernelGGL((dense_lds_kernel<8, 4, false>), dim3(grid), dim3(64 * kDenseWaves), 0, s, n, op->a, op->lda, X,
-                       ldx, Y, ldy, nrhs, op->scale, op->shift, done, (int64_t)0, (int64_t)0, (int64_t)0, xy_part);
+  if (op->kind != CK_OP_DENSE_F32 || nrhs < 3 || nrhs > 8) return CK_ERR_UNSUPPORTED;
+  dense_f32_lds(n, static_cast<const float*>(op->a), op->lda, X, ldx, Y, ldy, nrhs, op->scale, op->shift, done, xy_part,
+                s);
   CK_CHECK_LAUNCH();
   return CK_OK;
 }
@@ -1116,8 +1181,9 @@ int op_apply_internal(const ck_op* op, int nrhs, const float* X, int64_t ldx, fl
       if (op->n % 4 || op->lda % 4 || op->nnz % 4 || ldx % 4 || ldy % 4 || !aligned16(op->a) || !aligned16(X))
         return CK_ERR_UNSUPPORTED;
       const int grid = (op->n + kDenseWaves * 4 - 1) / (kDenseWaves * 4);
-      hipLaunchKernelGGL((dense_lds_kernel<1, 4, false>), dim3(grid, nrhs), dim3(64 * kDenseWaves), 0, s, op->n,
-                         op->a, op->lda, X, ldx, Y, ldy, 1, op->scale, op->shift, done, op->nnz, ldx, ldy);
+      hipLaunchKernelGGL((dense_f32_lds_kernel<1, 4>), dim3(grid, nrhs), dim3(64 * kDenseWaves), 0, s, op->n,
+                         static_cast<const float*>(op->a), op->lda, X, ldx, Y, ldy, 1, op->scale, op->shift, done,
+                         op->nnz, ldx, ldy, nullptr);
       CK_CHECK_LAUNCH();
       return CK_OK;
     }
