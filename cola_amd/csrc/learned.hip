@@ -3,11 +3,11 @@
 // Woodbury factor; plus the rank-r pivoted Cholesky comparator and the dense RBF
 // kernel-matrix builder.
 //
-//   mlp_fwd      one block = 64 points; the three layers run back to back with the
-//                hidden activations in LDS (bank-padded pitch 129), optional
-//                pre-activation save for the backward pass    [VALU, ~50k flop/point]
-//   mlp_bwd      one block = 64 points; per-block partial parameter gradients in the
-//                flat parameter layout, summed over blocks in index order (FP64)
+//   mlp_fwd      one block = 16 points; the three layers run back to back on MFMA with the
+//                hidden activations in LDS, optional pre-activation save for the
+//                backward pass                                [latency, ~50k flop/point]
+//   mlp_bwd      64 points per chunk on MFMA; per-chunk partial parameter gradients in the
+//                flat parameter layout, summed over chunks in index order (FP64)
 //   gram         C = X^T Y for tall-skinny X, Y (FP64 accumulation, fixed order)
 //   rows_gemm    Y = alpha X W + beta Y for tall-skinny X and a small W (LDS-staged)
 //   spd_inv      batched Cholesky of small SPD matrices (k <= 64) with jitter,
@@ -30,7 +30,6 @@ constexpr int kH = 128;     // hidden width
 constexpr int kMaxIn = 8;   // input dimension limit
 constexpr int kMaxOut = 128;
 constexpr int kRows = 64;   // points per block
-constexpr int kPitch = kH + 1;
 
 struct MlpLayout {
   int64_t w1, b1, w2, b2, w3, b3, total;
@@ -56,338 +55,332 @@ __device__ __forceinline__ float gelu_grad(float z) {
   return fmaf(z, pdf, cdf);
 }
 
-// xs[r][d] = X[(64 b + r) ldx + d] for the block's points, zero past n and din; the
-// loads are unconditional (indexes clamped) so they issue together
-__device__ __forceinline__ void load_points(float (*xs)[kMaxIn], const float* __restrict__ X, int64_t ldx, int n,
-                                            int din, int t) {
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ floatx4 mfma(float a, float b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// entries p[0 .. 3], those from index `left` on replaced by the last valid one
+__device__ __forceinline__ floatx4 load4(const float* __restrict__ p, int left) {
+  if (left >= 4) return *reinterpret_cast<const f4u*>(p);
+  floatx4 v;
 #pragma unroll
-  for (int k = 0; k < kRows * kMaxIn / 256; ++k) {
-    const int e = t + 256 * k, rr = e / kMaxIn, d = e % kMaxIn;
-    const int64_t i = (int64_t)blockIdx.x * kRows + rr;
-    const float v = X[min(i, (int64_t)n - 1) * ldx + min(d, din - 1)];
-    xs[rr][d] = (i < n && d < din) ? v : 0.f;
-  }
+  for (int e = 0; e < 4; ++e) v[e] = p[min(e, left - 1)];
+  return v;
 }
 
 // ------------------------------------------------------------------ MLP forward
-// Weights of layers 2 and 3 are staged in LDS once per block and read back as
-// wave-wide broadcasts; layer 1 (din <= 8 rows) reads W1 through scalar loads.
-// Summation order per output is the input index order.
-// One launch runs a few blocks once each, so its instruction cache starts cold: the
-// activation epilogues are rolled loops over LDS and layer 3 runs in 8-column chunks,
-// which keeps the code small (its size, not the arithmetic, set the time of an
-// unrolled form).
+// One block: 16 points, four waves of 32 hidden units; all three layers on
+// v_mfma_f32_16x16x4f32.  Step (c, e) of a sum takes k = 16 c + 4 g + e in lane group g = lane / 16, so a
+// lane's operand of the activations is a float4 of its row in LDS; the weights come straight from
+// memory, every one of them issued before the first layer runs.  The accumulator holds four
+// consecutive points of one unit: the saved pre-activations, stored by unit, are 16-byte stores.
+// Latency bound at the training size (1024 points): 16 points per block make 64 blocks there, where
+// 64 made 16, and with 64 points on the matrix units larger sets run no faster either (16384 points 22.6
+// against 27.0 us, 131072 123 against 124: the weights a block reads come from L2).  The activations are
+// rolled loops over LDS: a launch runs its code once, from cold instruction caches.  1024 points: 40.4
+// us with 64 points per block on the vector units, now 8.8; 16384: 46.8 -> 22.6 us.
+constexpr int kFwdRows = 16;
+
 template <bool SAVE>
 __global__ __launch_bounds__(256) void mlp_fwd_kernel(int n, int din, int dout, const float* __restrict__ X,
                                                       int64_t ldx, const float* __restrict__ prm,
                                                       float* __restrict__ G, int64_t gsr, int64_t gsc,
                                                       float* __restrict__ Z1, float* __restrict__ Z2, int64_t ldz) {
-  __shared__ float xs[kRows][kMaxIn];
-  __shared__ float h1[kRows][kPitch];
-  __shared__ float h2[kRows][kPitch];
-  __shared__ __align__(16) float ws[kH * kMaxOut];  // W2 (kH x kH), then W3 (kH x dout), row-major
+  constexpr int kP = kH + 4;  // row pitch: 16-byte aligned, rows four banks apart
+  __shared__ __align__(16) float h[2][kFwdRows][kP];
   const MlpLayout L = mlp_layout(din, dout);
-  const int t = threadIdx.x;
-  // g is the wave index: made wave-uniform (an SGPR), so the W1 loads below, whose
-  // addresses depend only on g and the loop counters, become scalar loads
-  const int r = t & 63, g = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int64_t row = (int64_t)blockIdx.x * kRows + r;
-  const bool valid = row < n;
-  // W2 and W3 start at multiples of kH floats (16-byte aligned); kH x dout is a
-  // multiple of 4 floats
-  constexpr int kQ = kH * kH / 4 / 256;  // float4 per thread for W2
-  const float4* w2g = reinterpret_cast<const float4*>(prm + L.w2);
-  const float4* w3g = reinterpret_cast<const float4*>(prm + L.w3);
-  float4* ws4 = reinterpret_cast<float4*>(ws);
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), g = lane >> 4, li = lane & 15;
+  const int p0 = blockIdx.x * kFwdRows;
+  const int u0 = 32 * w + li;  // this lane's unit of the wave's first tile, the second's is u0 + 16
+  // layer 1 (din <= 8: k = 4 s + g), biases, W2, the wave's first tile of W3
+  float x1[2], w1[2][2], b1[2], b2[2];
 #pragma unroll
-  for (int q = 0; q < kQ; ++q) ws4[t + 256 * q] = w2g[t + 256 * q];
-  load_points(xs, X, ldx, n, din, t);
-  __syncthreads();
-  const int c0 = g * 32;  // each wave owns 32 hidden units
-  {
-    float acc[32];
+  for (int s = 0; s < 2; ++s) {
+    const int d = 4 * s + g, dc = min(d, din - 1);
+    x1[s] = X[(int64_t)min(p0 + li, n - 1) * ldx + dc];
 #pragma unroll
-    for (int cc = 0; cc < 32; ++cc) acc[cc] = prm[L.b1 + c0 + cc];
-    for (int d = 0; d < din; ++d) {
-      const float xv = xs[r][d];
-      const float* w = prm + L.w1 + (int64_t)d * kH + c0;
+    for (int u = 0; u < 2; ++u) w1[u][s] = prm[L.w1 + dc * kH + u0 + 16 * u];
+  }
 #pragma unroll
-      for (int cc = 0; cc < 32; ++cc) acc[cc] = fmaf(xv, w[cc], acc[cc]);
+  for (int u = 0; u < 2; ++u) {
+    b1[u] = prm[L.b1 + u0 + 16 * u];
+    b2[u] = prm[L.b2 + u0 + 16 * u];
+  }
+  float w2[2][32], w3[32];
+  const float* w2p = prm + L.w2 + 4 * g * kH + u0;
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) w2[u][4 * c + e] = w2p[(16 * c + e) * kH + 16 * u];
+  int o = 16 * w + li;  // this lane's output
+  auto load_w3 = [&]() {
+    const float* w3p = prm + L.w3 + (int64_t)4 * g * dout + min(o, dout - 1);
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w3[4 * c + e] = w3p[(16 * c + e) * dout];
+  };
+  load_w3();
+  __builtin_amdgcn_sched_barrier(0);
+  // z: pre-activations of the wave's 32 units; saved, activated in place in LDS
+  auto activate = [&](const floatx4 (&z)[2], const float (&bias)[2], float* __restrict__ Z, int buf) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const floatx4 v = z[u] + bias[u];
+      if (SAVE) {
+        float* d = Z + (int64_t)(u0 + 16 * u) * ldz + p0 + 4 * g;
+        const int left = n - (p0 + 4 * g);
+        if (left >= 4)
+          *reinterpret_cast<f4u*>(d) = v;
+        else
+          for (int q = 0; q < left; ++q) d[q] = q == 0 ? v[0] : q == 1 ? v[1] : v[2];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) h[buf][4 * g + q][u0 + 16 * u] = v[q];
     }
-#pragma unroll
-    for (int cc = 0; cc < 32; ++cc) h1[r][c0 + cc] = acc[cc];
-  }
-  // each lane activates its own row's 32 entries: no barrier needed
+    // each lane activates the entries it wrote: no barrier
 #pragma unroll 1
-  for (int cc = 0; cc < 32; ++cc) {
-    const float z = h1[r][c0 + cc];
-    if (SAVE && valid) Z1[(int64_t)(c0 + cc) * ldz + row] = z;
-    h1[r][c0 + cc] = gelu(z);
-  }
+    for (int i = 0; i < 8; ++i) {
+      float* q = &h[buf][4 * g + (i & 3)][u0 + 4 * (i & 4)];
+      *q = gelu(*q);
+    }
+  };
+  floatx4 z[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const bool in = 4 * s + g < din;
+      z[u] = mfma(in ? x1[s] : 0.f, in ? w1[u][s] : 0.f, z[u]);
+    }
+  activate(z, b1, Z1, 0);
   __syncthreads();
-  {
-    float acc[32];
+  z[0] = z[1] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int cc = 0; cc < 32; ++cc) acc[cc] = prm[L.b2 + c0 + cc];
-    for (int j = 0; j < kH; ++j) {
-      const float hv = h1[r][j];
-      const float4* w = reinterpret_cast<const float4*>(ws + j * kH + c0);
+  for (int c = 0; c < 8; ++c) {
+    const floatx4 a = *reinterpret_cast<const floatx4*>(&h[0][li][16 * c + 4 * g]);
 #pragma unroll
-      for (int c4 = 0; c4 < 8; ++c4) {
-        const float4 wv = w[c4];
-        acc[4 * c4 + 0] = fmaf(hv, wv.x, acc[4 * c4 + 0]);
-        acc[4 * c4 + 1] = fmaf(hv, wv.y, acc[4 * c4 + 1]);
-        acc[4 * c4 + 2] = fmaf(hv, wv.z, acc[4 * c4 + 2]);
-        acc[4 * c4 + 3] = fmaf(hv, wv.w, acc[4 * c4 + 3]);
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) z[u] = mfma(a[e], w2[u][4 * c + e], z[u]);
+  }
+  activate(z, b2, Z2, 1);
+  __syncthreads();
+#pragma unroll 1
+  for (; o - li < dout; o += 64) {
+    floatx4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const floatx4 a = *reinterpret_cast<const floatx4*>(&h[1][li][16 * c + 4 * g]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y = mfma(a[e], w3[4 * c + e], y);
+    }
+    if (o < dout) {
+      const float b3 = prm[L.b3 + o];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t row = p0 + 4 * g + q;
+        if (row < n) G[row * gsr + (int64_t)o * gsc] = y[q] + b3;
       }
     }
-#pragma unroll
-    for (int cc = 0; cc < 32; ++cc) h2[r][c0 + cc] = acc[cc];
-  }
-#pragma unroll 1
-  for (int cc = 0; cc < 32; ++cc) {
-    const float z = h2[r][c0 + cc];
-    if (SAVE && valid) Z2[(int64_t)(c0 + cc) * ldz + row] = z;
-    h2[r][c0 + cc] = gelu(z);
-  }
-  __syncthreads();  // W2 reads done, h2 complete
-  const int n3 = kH * dout / 4;  // float4 of W3, <= 256 kQ
-#pragma unroll
-  for (int q = 0; q < kQ; ++q)
-    if (t + 256 * q < n3) ws4[t + 256 * q] = w3g[t + 256 * q];
-  __syncthreads();
-  // layer 3: wave g owns outputs o0 .. o0 + per - 1, in chunks of 8. A chunk's tail
-  // past its owned range reads other LDS words (within ws: o0 + c8 + 7 <= 4 per + 6
-  // and row 127 ends at 128 dout) into accumulators that are never stored.
-  const int per = (dout + 3) / 4;  // <= 32 outputs per wave
-  const int o0 = g * per;
-#pragma unroll 1
-  for (int c8 = 0; c8 < per; c8 += 8) {
-    float acc[8];
-#pragma unroll
-    for (int cc = 0; cc < 8; ++cc)
-      acc[cc] = (c8 + cc < per && o0 + c8 + cc < dout) ? prm[L.b3 + o0 + c8 + cc] : 0.f;
-    for (int j = 0; j < kH; ++j) {
-      const float hv = h2[r][j];
-      const float* w = ws + j * dout + o0 + c8;
-#pragma unroll
-      for (int cc = 0; cc < 8; ++cc) acc[cc] = fmaf(hv, w[cc], acc[cc]);
-    }
-    if (valid) {
-#pragma unroll
-      for (int cc = 0; cc < 8; ++cc)
-        if (c8 + cc < per && o0 + c8 + cc < dout) G[row * gsr + (int64_t)(o0 + c8 + cc) * gsc] = acc[cc];
+    if (o - li + 64 < dout) {
+      o += 64;
+      load_w3();
+      o -= 64;
     }
   }
 }
 
 // ----------------------------------------------------------------- MLP backward
-// Given dL/dG for a block of 64 points, writes that block's contribution to every
-// parameter gradient (flat layout) into part[blockIdx.x * total + ...].
-// W3 (row pitch dout rounded up to 4, zero-padded) and then W2 are staged in LDS;
-// dZ2 and dZ1 are accumulated in registers over 4 columns at a time, with the weight
-// rows read as wave-wide float4 broadcasts. dG and dZ2 share one LDS array (dG is
-// dead once dZ2 is in registers). The saved pre-activations are loaded into
-// registers up front (one latency); GELU and its derivative run in rolled loops over
-// LDS so the code stays small. Summation order per output is the index order.
-__global__ __launch_bounds__(256) void mlp_bwd_kernel(int n, int din, int dout, const float* __restrict__ X,
+// Given dL/dG for a chunk of 64 points, writes that chunk's contribution to every parameter gradient
+// (flat layout) into part[blockIdx.x * total + ...].  Eight waves; the five products
+//   dH2 = dG W3^T, dW3 = h2^T dG, dH1 = dZ2 W2^T, dW2 = h1^T dZ2 (and dW1 = X^T dZ1 on the vector units)
+// run on v_mfma_f32_16x16x4f32 with the operand order of the forward pass: every operand is a float4
+// along the sum, so dG and dZ2 are kept both by point and by column.  dZ2 is formed whole; everything
+// that follows is done for 32 hidden units at a time, quarter blockIdx.y, + gridDim.y, ... -- few chunks
+// are spread over up to four blocks each.  Latency bound at the training size (1024 points): 119.4 us
+// with a chunk per block on the vector units, now 22 us; 16384 points, the sum over chunks included: 184 -> 109 us.
+constexpr int kBP = kH + 4;     // pitch of rows by point
+constexpr int kBT = kRows + 4;  // pitch of rows by column
+constexpr int kBQ = 32;         // hidden units per quarter
+
+__global__ __launch_bounds__(512) void mlp_bwd_kernel(int n, int din, int dout, const float* __restrict__ X,
                                                       int64_t ldx, const float* __restrict__ prm,
                                                       const float* __restrict__ Z1, const float* __restrict__ Z2,
                                                       int64_t ldz, const float* __restrict__ dG, int64_t dsr,
                                                       int64_t dsc, float* __restrict__ part) {
-  __shared__ float xs[kRows][kMaxIn];
-  __shared__ float a[kRows][kPitch];   // Z2 -> h2; Z2; Z1 -> h1; dZ1
-  __shared__ float dd[kRows][kPitch];  // dG (columns up to dp, zero beyond dout); dZ2; Z1
-  __shared__ __align__(16) float ws[kH * kMaxOut];  // W3 (kH x dp), then W2 (kH x kH)
+  __shared__ __align__(16) float Dg[kRows][kBP], DgT[kH][kBT];  // dG, zero past dout and past n
+  __shared__ __align__(16) float Dz[kRows][kBP], DzT[kH][kBT];  // dZ2
+  __shared__ __align__(16) float Hq[kBQ][kBT], Eq[kBQ][kBT];    // the quarter's h2, then h1; its dZ1
+  __shared__ float xs[kRows][kMaxIn + 1];                       // the points, and 1 for the bias
   const MlpLayout L = mlp_layout(din, dout);
   float* out = part + (int64_t)blockIdx.x * L.total;
-  const int t = threadIdx.x;
-  const int r = t & 63, g = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int64_t row = (int64_t)blockIdx.x * kRows + r;
-  const bool valid = row < n;
-  const int dp = (dout + 3) & ~3;
-  const int c0 = g * 32;  // this wave's 32 hidden units
-  constexpr int kQ = kH * kH / 4 / 256;  // float4 of W2 (and at most of W3) per thread
-  // every global load below is unconditional (row and column indexes clamped into
-  // range, the value selected afterwards), so each group is issued back to back and
-  // waited for once
-  const int64_t rowc = valid ? row : (int64_t)n - 1;
-  float z2[32], z1[32], gv[32];
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), g = lane >> 4, li = lane & 15;
+  const int p0 = blockIdx.x * kRows, left = n - p0;  // points of this chunk
+  const int nc = (dout + 15) / 16;
+  // Z2 at this lane's unit and four points of each row tile: the accumulator's layout
+  const int u = 16 * w + li;
+  floatx4 z2[4];
 #pragma unroll
-  for (int jj = 0; jj < 32; ++jj) {
-    const float v2 = Z2[(int64_t)(c0 + jj) * ldz + rowc], v1 = Z1[(int64_t)(c0 + jj) * ldz + rowc];
-    z2[jj] = valid ? v2 : 0.f;
-    z1[jj] = valid ? v1 : 0.f;
+  for (int r = 0; r < 4; ++r) {
+    const int p = min(16 * r + 4 * g, left - 1);
+    z2[r] = load4(Z2 + (int64_t)u * ldz + p0 + p, left - p);
   }
+  float w3[8][4];
 #pragma unroll
-  for (int i = 0; i < 32; ++i) {  // dG columns c = g + 4 i
-    const int c = g + 4 * i;
-    const float v = dG[rowc * dsr + (int64_t)min(c, dout - 1) * dsc];
-    gv[i] = (valid && c < dout) ? v : 0.f;
-  }
-  load_points(xs, X, ldx, n, din, t);
-  if (dp == dout) {  // W3 rows are 16-byte aligned in both layouts: straight float4 copy
-    const float4* w3g = reinterpret_cast<const float4*>(prm + L.w3);
-    float4* ws4 = reinterpret_cast<float4*>(ws);
-    const int n3 = kH * dout / 4;
+  for (int c = 0; c < 8; ++c)
+    if (c < nc) {
 #pragma unroll
-    for (int q = 0; q < kQ; ++q)
-      if (t + 256 * q < n3) ws4[t + 256 * q] = w3g[t + 256 * q];
-  } else {
-    // lane r copies columns r and r + 64 of rows g, g + 4, ...; zero padding to dp
-#pragma unroll 1
-    for (int j0 = 0; j0 < kH; j0 += 32) {
-      float v0[8], v1[8];
+      for (int e = 0; e < 4; ++e) w3[c][e] = prm[L.w3 + (int64_t)u * dout + min(16 * c + 4 * g + e, dout - 1)];
+    }
+  for (int e0 = 0; e0 < 16 * nc; e0 += 64) {  // dG: lanes along the points, eight columns per thread
+    float v[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float* w = prm + L.w3 + (int64_t)(j0 + 4 * i + g) * dout;
-        const float u0 = w[min(r, dout - 1)], u1 = w[min(r + 64, dout - 1)];
-        v0[i] = r < dout ? u0 : 0.f;
-        v1[i] = r + 64 < dout ? u1 : 0.f;
-      }
+    for (int q = 0; q < 8; ++q)
+      v[q] = dG[(int64_t)(p0 + min(lane, left - 1)) * dsr + (int64_t)min(e0 + w + 8 * q, dout - 1) * dsc];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        float* w = ws + (j0 + 4 * i + g) * dp;
-        if (r < dp) w[r] = v0[i];
-        if (r + 64 < dp) w[r + 64] = v1[i];
-      }
+    for (int q = 0; q < 8; ++q) {
+      const int c = e0 + w + 8 * q;
+      const float d = c < dout && lane < left ? v[q] : 0.f;
+      Dg[lane][c] = d;
+      DgT[c][lane] = d;
     }
   }
-  // columns g + 4 i reach 127 < kPitch; those past dp receive zeros and are never read
-  // before dd is rewritten, so the stores need no test
-#pragma unroll
-  for (int i = 0; i < 32; ++i) dd[r][g + 4 * i] = gv[i];
-#pragma unroll
-  for (int jj = 0; jj < 32; ++jj) a[r][c0 + jj] = z2[jj];
-#pragma unroll 1
-  for (int jj = 0; jj < 32; ++jj) a[r][c0 + jj] = gelu(a[r][c0 + jj]);  // own row: no barrier
-  __syncthreads();
-
-  // dW3[j][c] = sum_r h2[r][j] dG[r][c]; db3[c] = sum_r dG[r][c]
   {
-    const int j = t & 127, par = t >> 7;
-    const int nq = (dout - par + 1) / 2;  // columns c = par + 2 q
-#pragma unroll 1
-    for (int q0 = 0; q0 < nq; q0 += 16) {
-      float acc[16];
-#pragma unroll
-      for (int qq = 0; qq < 16; ++qq) acc[qq] = 0.f;
-      // columns past dout are clamped to the pad column kH; those sums are not stored
-      for (int rr = 0; rr < kRows; ++rr) {
-        const float av = a[rr][j];
-#pragma unroll
-        for (int qq = 0; qq < 16; ++qq) acc[qq] = fmaf(av, dd[rr][min(par + 2 * (q0 + qq), kH)], acc[qq]);
-      }
-#pragma unroll
-      for (int qq = 0; qq < 16; ++qq)
-        if (q0 + qq < nq) out[L.w3 + (int64_t)j * dout + par + 2 * (q0 + qq)] = acc[qq];
-    }
-    for (int c = t; c < dout; c += 256) {
-      float s = 0.f;
-      for (int rr = 0; rr < kRows; ++rr) s += dd[rr][c];
-      out[L.b3 + c] = s;
-    }
-  }
-  // dZ2[r][j] = (sum_c dG[r][c] W3[j][c]) * gelu'(Z2[r][j]), j = c0 + jj
-  float acc[32];
-#pragma unroll
-  for (int jj = 0; jj < 32; ++jj) acc[jj] = 0.f;
-  for (int c = 0; c < dp; c += 4) {
-    const float x0 = dd[r][c], x1 = dd[r][c + 1], x2 = dd[r][c + 2], x3 = dd[r][c + 3];
-#pragma unroll
-    for (int jj = 0; jj < 32; ++jj) {
-      const float4 w = *reinterpret_cast<const float4*>(ws + (c0 + jj) * dp + c);
-      acc[jj] = fmaf(x0, w.x, acc[jj]);
-      acc[jj] = fmaf(x1, w.y, acc[jj]);
-      acc[jj] = fmaf(x2, w.z, acc[jj]);
-      acc[jj] = fmaf(x3, w.w, acc[jj]);
-    }
-  }
-  __syncthreads();  // dG, h2 and W3 reads done
-  {  // W2 starts 16-byte aligned
-    const float4* w2g = reinterpret_cast<const float4*>(prm + L.w2);
-    float4* ws4 = reinterpret_cast<float4*>(ws);
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) ws4[t + 256 * q] = w2g[t + 256 * q];
-  }
-#pragma unroll
-  for (int jj = 0; jj < 32; ++jj) {
-    dd[r][c0 + jj] = acc[jj];
-    a[r][c0 + jj] = z2[jj];
-  }
-#pragma unroll 1
-  for (int jj = 0; jj < 32; ++jj) {
-    const float v = dd[r][c0 + jj];
-    dd[r][c0 + jj] = valid ? v * gelu_grad(a[r][c0 + jj]) : 0.f;
-  }
-#pragma unroll
-  for (int jj = 0; jj < 32; ++jj) a[r][c0 + jj] = z1[jj];
-#pragma unroll 1
-  for (int jj = 0; jj < 32; ++jj) a[r][c0 + jj] = gelu(a[r][c0 + jj]);
-  __syncthreads();
-  // dW2[j][k] = sum_r h1[r][j] dZ2[r][k]; db2[k] = sum_r dZ2[r][k]
-  {
-    const int j = t & 127, par = t >> 7;
-#pragma unroll 1
-    for (int q0 = 0; q0 < kH / 2; q0 += 16) {
-      float acc2[16];
-#pragma unroll
-      for (int qq = 0; qq < 16; ++qq) acc2[qq] = 0.f;
-      for (int rr = 0; rr < kRows; ++rr) {
-        const float av = a[rr][j];
-#pragma unroll
-        for (int qq = 0; qq < 16; ++qq) acc2[qq] = fmaf(av, dd[rr][par + 2 * (q0 + qq)], acc2[qq]);
-      }
-#pragma unroll
-      for (int qq = 0; qq < 16; ++qq) out[L.w2 + (int64_t)j * kH + par + 2 * (q0 + qq)] = acc2[qq];
-    }
-    for (int k = t; k < kH; k += 256) {
-      float s = 0.f;
-      for (int rr = 0; rr < kRows; ++rr) s += dd[rr][k];
-      out[L.b2 + k] = s;
-    }
-  }
-  // dZ1[r][j] = (sum_k dZ2[r][k] W2[j][k]) * gelu'(Z1[r][j]), j = c0 + jj
-#pragma unroll
-  for (int jj = 0; jj < 32; ++jj) acc[jj] = 0.f;
-  for (int k = 0; k < kH; k += 4) {
-    const float x0 = dd[r][k], x1 = dd[r][k + 1], x2 = dd[r][k + 2], x3 = dd[r][k + 3];
-#pragma unroll
-    for (int jj = 0; jj < 32; ++jj) {
-      const float4 w = *reinterpret_cast<const float4*>(ws + (c0 + jj) * kH + k);
-      acc[jj] = fmaf(x0, w.x, acc[jj]);
-      acc[jj] = fmaf(x1, w.y, acc[jj]);
-      acc[jj] = fmaf(x2, w.z, acc[jj]);
-      acc[jj] = fmaf(x3, w.w, acc[jj]);
-    }
-  }
-  __syncthreads();  // h1 and dZ2 reads done
-#pragma unroll
-  for (int jj = 0; jj < 32; ++jj) {
-    a[r][c0 + jj] = acc[jj];
-    dd[r][c0 + jj] = z1[jj];
-  }
-#pragma unroll 1
-  for (int jj = 0; jj < 32; ++jj) {
-    const float v = a[r][c0 + jj];
-    a[r][c0 + jj] = valid ? v * gelu_grad(dd[r][c0 + jj]) : 0.f;
+    const int d = w;  // kMaxIn == 8 waves
+    const float v = X[(int64_t)(p0 + min(lane, left - 1)) * ldx + min(d, din - 1)];
+    xs[lane][d] = d < din && lane < left ? v : 0.f;
+    if (w == 0) xs[lane][kMaxIn] = 1.f;
   }
   __syncthreads();
-  // dW1[d][j] = sum_r x[r][d] dZ1[r][j]; db1[j] = sum_r dZ1[r][j]
+  // dZ2 = (dG W3^T) * gelu'(Z2), all 128 units: wave w takes units 16 w .., four row tiles
   {
-    const int j = t & 127, par = t >> 7;
-    for (int d = par; d < din; d += 2) {
-      float s = 0.f;
-      for (int rr = 0; rr < kRows; ++rr) s = fmaf(xs[rr][d], a[rr][j], s);
-      out[L.w1 + (int64_t)d * kH + j] = s;
+    floatx4 a[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) a[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      if (c < nc) {
+        floatx4 d[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d[r] = *reinterpret_cast<const floatx4*>(&Dg[16 * r + li][16 * c + 4 * g]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) a[r] = mfma(d[r][e], w3[c][e], a[r]);
+      }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      *reinterpret_cast<floatx4*>(&DzT[u][16 * r + 4 * g]) = a[r];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) Dz[16 * r + 4 * g + q][u] = z2[r][q];
     }
-    if (t < kH) {
-      float s = 0.f;
-      for (int rr = 0; rr < kRows; ++rr) s += a[rr][t];
-      out[L.b1 + t] = s;
+#pragma unroll 1
+    for (int i = 0; i < 16; ++i) {  // the entries this lane wrote
+      const int p = 16 * (i >> 2) + 4 * g + (i & 3);
+      const float v = DzT[u][p] * gelu_grad(Dz[p][u]);
+      DzT[u][p] = v;
+      Dz[p][u] = v;
     }
+  }
+#pragma unroll 1
+  for (int y = blockIdx.y; y < kH / kBQ; y += gridDim.y) {
+    const int j0 = kBQ * y;
+    // W2 rows of the wave's dH1 tile (row tile w & 3, units j0 + 16 (w >> 2) ..) and Z1 there
+    const int j = j0 + 16 * (w >> 2) + li, rt = w & 3, p = min(16 * rt + 4 * g, left - 1);
+    floatx4 w2[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) w2[c] = *reinterpret_cast<const floatx4*>(prm + L.w2 + (int64_t)j * kH + 16 * c + 4 * g);
+    const floatx4 z1 = load4(Z1 + (int64_t)j * ldz + p0 + p, left - p);
+    // h2 of the quarter
+    {
+      float v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = Z2[(int64_t)(j0 + w + 8 * q) * ldz + p0 + min(lane, left - 1)];
+      __syncthreads();  // the previous quarter's Hq and Eq are read
+#pragma unroll
+      for (int q = 0; q < 4; ++q) Hq[w + 8 * q][lane] = v[q];
+#pragma unroll 1
+      for (int q = 0; q < 4; ++q) Hq[w + 8 * q][lane] = gelu(Hq[w + 8 * q][lane]);
+    }
+    __syncthreads();  // Hq, and (first quarter) Dz, DzT
+    // dW3[j][c] = sum_p h2[p][j] dG[p][c]
+    for (int tile = w; tile < 2 * nc; tile += 8) {
+      const int jt = tile & 1, ct = tile >> 1;
+      floatx4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const floatx4 hv = *reinterpret_cast<const floatx4*>(&Hq[16 * jt + li][16 * c + 4 * g]);
+        const floatx4 dv = *reinterpret_cast<const floatx4*>(&DgT[16 * ct + li][16 * c + 4 * g]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a = mfma(hv[e], dv[e], a);
+      }
+      const int col = 16 * ct + li;
+      if (col < dout) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) out[L.w3 + (int64_t)(j0 + 16 * jt + 4 * g + q) * dout + col] = a[q];
+      }
+    }
+    // db3 (first quarter) and db2 of the quarter: one row of 64 points per thread
+    const int nb = kBQ + (y == 0 ? dout : 0);
+    if (t < nb) {
+      const float* row = t < kBQ ? DzT[j0 + t] : DgT[t - kBQ];
+      float s = 0.f;
+#pragma unroll 4
+      for (int q = 0; q < kRows; ++q) s += row[q];
+      out[t < kBQ ? L.b2 + j0 + t : L.b3 + t - kBQ] = s;
+    }
+    // dH1 tile
+    floatx4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const floatx4 d = *reinterpret_cast<const floatx4*>(&Dz[16 * rt + li][16 * c + 4 * g]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a = mfma(d[e], w2[c][e], a);
+    }
+    __syncthreads();  // h2 is read
+    const int jl = 16 * (w >> 2) + li;
+    *reinterpret_cast<floatx4*>(&Eq[jl][16 * rt + 4 * g]) = a;
+    *reinterpret_cast<floatx4*>(&Hq[jl][16 * rt + 4 * g]) = z1;
+#pragma unroll 1
+    for (int q = 0; q < 4; ++q) {  // the entries this lane wrote: dZ1 and h1
+      const float z = Hq[jl][16 * rt + 4 * g + q];
+      Eq[jl][16 * rt + 4 * g + q] *= gelu_grad(z);
+      Hq[jl][16 * rt + 4 * g + q] = gelu(z);
+    }
+    __syncthreads();
+    // dW1[d][j] and db1[j] (the point's constant 1): thread (j, d)
+    for (int o = t; o < kBQ * (din + 1); o += 512) {
+      const int q = o & (kBQ - 1), d = o / kBQ, dc = d < din ? d : kMaxIn;
+      float s = 0.f;
+#pragma unroll 4
+      for (int r = 0; r < kRows; ++r) s = fmaf(xs[r][dc], Eq[q][r], s);
+      out[d < din ? L.w1 + (int64_t)d * kH + j0 + q : L.b1 + j0 + q] = s;
+    }
+    // dW2[j][k] = sum_p h1[p][j] dZ2[p][k]: wave w takes k = 16 w .., both unit tiles
+    floatx4 b[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const floatx4 dv = *reinterpret_cast<const floatx4*>(&DzT[u][16 * c + 4 * g]);
+#pragma unroll
+      for (int jt = 0; jt < 2; ++jt) {
+        const floatx4 hv = *reinterpret_cast<const floatx4*>(&Hq[16 * jt + li][16 * c + 4 * g]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) b[jt] = mfma(hv[e], dv[e], b[jt]);
+      }
+    }
+#pragma unroll
+    for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) out[L.w2 + (int64_t)(j0 + 16 * jt + 4 * g + q) * kH + u] = b[jt][q];
   }
 }
+
 
 // grad[p] = scale * sum_b part[b][p] (blocks in index order, FP64)
 __global__ __launch_bounds__(256) void grad_reduce_kernel(int nblk, int64_t total, const float* __restrict__ part,
@@ -470,213 +463,246 @@ __global__ __launch_bounds__(256) void gram_reduce(int nchunks, int64_t count, c
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= count) return;
   double acc = 0.0;
-  for (int c = 0; c < nchunks; ++c) acc += part[(int64_t)c * count + idx];
+  for (int c0 = 0; c0 < nchunks; c0 += 16) {
+    double v[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) v[c] = part[(int64_t)min(c0 + c, nchunks - 1) * count + idx];  // in flight together
+#pragma unroll
+    for (int c = 0; c < 16; ++c) acc += c0 + c < nchunks ? v[c] : 0.0;
+  }
   C[idx] = acc;
 }
 
 // --------------------------------------------------------- rows GEMM Y = a X W + b Y
 constexpr int kGemmMax = 128;
 
+// One block: 64 rows x 32 columns, thread (row, 8 columns); the rows of X and the columns of W it needs
+// are staged in LDS 64 of the sum at a time.  1024 x 64 x 64: 16.3 us with a row of 32 columns per
+// thread and X from global memory (8 blocks), now 8.8 us.
 __global__ __launch_bounds__(256) void rows_gemm_kernel(int64_t n, int kin, int kout, const float* __restrict__ X,
                                                         int64_t xsr, int64_t xsc, const float* __restrict__ W,
                                                         float alpha, float beta, float* __restrict__ Y, int64_t ysr,
                                                         int64_t ysc) {
-  __shared__ float ws[kGemmMax * 32];
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  __shared__ float xs[64][65];
+  __shared__ __align__(16) float ws[64][32];
+  const int t = threadIdx.x, r = t & 63, cg = (t >> 6) * 8;
+  const int64_t i0 = (int64_t)blockIdx.x * 64, i = i0 + r;
   const int c0 = blockIdx.y * 32;
-  const int nc = kout - c0 < 32 ? kout - c0 : 32;
-  // W's column slab in groups of eight loads per thread (indexes clamped, so a group
-  // issues together)
-  for (int e0 = 0; e0 < kin * 32; e0 += 2048) {
-    float v[8];
+  float acc[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int e = min(e0 + (int)threadIdx.x + 256 * q, kin * 32 - 1), j = e / 32, cc = e % 32;
-      v[q] = W[(int64_t)j * kout + c0 + min(cc, nc - 1)];
+  for (int q = 0; q < 8; ++q) acc[q] = 0.f;
+  for (int j0 = 0; j0 < kin; j0 += 64) {
+    float xv[16], wv[8];  // clamped indexes: both groups issue together
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int e = t + 256 * q;
+      // consecutive threads along the operand's contiguous direction
+      const int rr = xsr == 1 ? e & 63 : e >> 6, jj = xsr == 1 ? e >> 6 : e & 63;
+      const int64_t row = i0 + rr < n ? i0 + rr : n - 1;
+      xv[q] = X[row * xsr + (int64_t)min(j0 + jj, kin - 1) * xsc];
     }
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      const int e = e0 + threadIdx.x + 256 * q;
-      if (e < kin * 32) ws[e] = e % 32 < nc ? v[q] : 0.f;
+      const int e = t + 256 * q, jj = e >> 5, cc = e & 31;
+      wv[q] = W[(int64_t)min(j0 + jj, kin - 1) * kout + min(c0 + cc, kout - 1)];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int e = t + 256 * q;
+      const int rr = xsr == 1 ? e & 63 : e >> 6, jj = xsr == 1 ? e >> 6 : e & 63;
+      xs[rr][jj] = xv[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int e = t + 256 * q;
+      ws[e >> 5][e & 31] = wv[q];
+    }
+    __syncthreads();
+    const int jn = kin - j0 < 64 ? kin - j0 : 64;
+#pragma unroll 4
+    for (int j = 0; j < jn; ++j) {
+      const float x = xs[r][j];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[q] = fmaf(x, ws[j][cg + q], acc[q]);
     }
   }
-  __syncthreads();
   if (i >= n) return;
-  float acc[32];
 #pragma unroll
-  for (int cc = 0; cc < 32; ++cc) acc[cc] = 0.f;
-  // X row entries eight at a time so their loads are in flight together
-  int j = 0;
-  for (; j + 8 <= kin; j += 8) {
-    float xv[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) xv[u] = X[i * xsr + (int64_t)(j + u) * xsc];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-#pragma unroll
-      for (int cc = 0; cc < 32; ++cc) acc[cc] = fmaf(xv[u], ws[(j + u) * 32 + cc], acc[cc]);
-  }
-  for (; j < kin; ++j) {
-    const float xv = X[i * xsr + (int64_t)j * xsc];
-#pragma unroll
-    for (int cc = 0; cc < 32; ++cc) acc[cc] = fmaf(xv, ws[j * 32 + cc], acc[cc]);
-  }
-#pragma unroll
-  for (int cc = 0; cc < 32; ++cc) {
-    if (cc < nc) {
-      float* y = Y + i * ysr + (int64_t)(c0 + cc) * ysc;
-      *y = beta == 0.f ? alpha * acc[cc] : fmaf(beta, *y, alpha * acc[cc]);
+  for (int q = 0; q < 8; ++q) {
+    if (c0 + cg + q < kout) {
+      float* y = Y + i * ysr + (int64_t)(c0 + cg + q) * ysc;
+      *y = beta == 0.f ? alpha * acc[q] : fmaf(beta, *y, alpha * acc[q]);
     }
   }
 }
 
 // ------------------------------------------------------ small SPD: chol, L^-1, A^-1
 constexpr int kSpdMax = 64;
-constexpr int kPack = kSpdMax * (kSpdMax + 1) / 2;  // packed lower triangle
+constexpr int kSpdPitch = kSpdMax + 2;  // LDS row pitch in doubles: 16-byte aligned pairs, two banks apart
 
-__device__ __forceinline__ int pk(int i, int j) { return i * (i + 1) / 2 + j; }  // i >= j
+// 1 / p to within a unit in the last place: the hardware's estimate (good to about 2^-26) and two
+// Newton steps; the library's division where the estimate could overflow or flush.
+__device__ __forceinline__ double rcp_f64(double p) {
+  if (!(fabs(p) > 1e-290 && fabs(p) < 1e290)) return 1.0 / p;
+  double r = __builtin_amdgcn_rcp(p);
+  r = fma(r, fma(-p, r, 1.0), r);
+  return fma(r, fma(-p, r, 1.0), r);
+}
 
-// One block per matrix, everything in LDS (packed lower triangles of L and X = L^-1):
-// A + (jitter_abs + jitter_rel * trace(A) / k) I = L L^T.
+// One block per matrix: A + (jitter_abs + jitter_rel * trace(A) / k) I = L L^T.
 // linv (required, k x k row-major lower) = L^-1; inv64 / inv32 = A^-1; linvT32 = L^-T.
 // status[b] = 0, or j + 1 when the j-th pivot is not positive.
+// Latency bound: k dependent pivots.  The factorization runs as L D L^T (L unit lower) and is applied
+// to the identity in the same steps, two pivots to a step: columns j, j + 1 of what is left of A and rows
+// j, j + 1 of Y = L^-1 are read from a double-buffered LDS row (one barrier, one LDS round trip per
+// step), every thread updates its 4 x 4 pieces of A and Y in registers, and the owners of the next two
+// columns and rows publish them.  D^-1/2 (the square roots) scales Y's rows once at the end.
+// k = 64: 110.8 us with a column per step, two barriers, a square root and a division each; 42.5 us
+// with one pivot per step; now 33 us.
 __global__ __launch_bounds__(256) void spd_inv_kernel(int k, const double* __restrict__ A, int64_t lda, int64_t sa,
                                                       double jitter_rel, double jitter_abs, double* __restrict__ linv,
                                                       double* __restrict__ inv64, float* __restrict__ inv32,
                                                       float* __restrict__ linvT32, int* __restrict__ status) {
-  __shared__ double Ls[kPack];
-  __shared__ double Xs[kPack];
-  __shared__ double dgl[kSpdMax];  // Cholesky diagonal, kept apart until the factorization ends
-  __shared__ double shift;
-  const int b = blockIdx.x, t = threadIdx.x;
-  const int kk = k * k;
+  __shared__ __align__(16) double Xs[kSpdMax * kSpdPitch];
+  __shared__ double2 acol[2][kSpdMax];  // [row i]: A's entries (i, j) and (i, j + 1)
+  __shared__ double2 yrow[2][kSpdMax];  // [column c]: Y's entries (j, c) and (j + 1, c)
+  __shared__ double piv[kSpdMax];
+  __shared__ double red[4];
+  const int b = blockIdx.x, t = threadIdx.x, ti = t >> 4, tj = t & 15;
+  const int64_t kk = (int64_t)k * k;
   const double* Ab = A + (int64_t)b * sa;
-  // lower triangle in; loads are unconditional (index clamped) so each group of eight
-  // issues together
-  for (int e0 = 0; e0 < kk; e0 += 2048) {
-    double v[8];
+  // piece (u, v): row at(ti, u), column at(tj, v) of the symmetric matrix, neighbouring pairs 32 apart,
+  // read from its lower triangle; loads are unconditional (indexes clamped) and issue together
+  auto at = [](int q, int u) { return 2 * q + (u & 1) + 32 * (u >> 1); };
+  double av[4][4], yv[4][4];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int e = min(e0 + t + 256 * q, kk - 1), i = e / k, j = e % k;
-      v[q] = Ab[(int64_t)i * lda + j];
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = at(ti, u), c = at(tj, v), hi = min(max(i, c), k - 1), lo = min(min(i, c), k - 1);
+      av[u][v] = Ab[(int64_t)hi * lda + lo];
     }
+  double tr = 0.0;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int e = e0 + t + 256 * q, i = e / k, j = e % k;
-      if (e < kk && j <= i) Ls[pk(i, j)] = v[q];
+  for (int u = 0; u < 4; ++u)
+    if (ti == tj && at(ti, u) < k) tr += av[u][u];
+  tr = block_sum<256>(tr, red);
+  const double shift = jitter_abs + jitter_rel * tr / k;
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const bool diag = ti == tj && u == v;
+      // past the order: the identity, which factors to itself
+      const bool in = at(ti, u) < k && at(tj, v) < k;
+      yv[u][v] = diag ? 1.0 : 0.0;
+      av[u][v] = in ? av[u][v] + (diag ? shift : 0.0) : yv[u][v];
     }
-  }
-  for (int e = t; e < k * (k + 1) / 2; e += 256) Xs[e] = 0.0;
-  __syncthreads();
-  if (t == 0) {
-    double tr = 0.0;
-    for (int i = 0; i < k; ++i) tr += Ls[pk(i, i)];
-    shift = jitter_abs + jitter_rel * tr / k;
-  }
-  __syncthreads();
-  if (t < k) Ls[pk(t, t)] += shift;
-  // this thread's entries of the packed lower triangle, e = t + 256 m, as (row, column);
-  // the per-step updates below touch only these, unrolled so their LDS accesses issue
-  // back to back
-  constexpr int kM = (kPack + 255) / 256;
-  const int np = k * (k + 1) / 2;
-  int er[kM], ec[kM], rb[kM], cb[kM];  // row, column, and the packed offsets of their rows
+  auto publish = [&](int buf, int j) {  // columns and rows j, j + 1 (j even)
+    const int q = (j >> 1) & 15;
+    const bool hi = j >= 32;
+    if (tj == q) {
 #pragma unroll
-  for (int m = 0; m < kM; ++m) {
-    const int e = t + 256 * m;
-    int i = (int)((sqrtf(8.f * (float)e + 1.f) - 1.f) * 0.5f);
-    while (i * (i + 1) / 2 > e) --i;
-    while ((i + 1) * (i + 2) / 2 <= e) ++i;
-    er[m] = e < np ? i : -1;
-    ec[m] = e < np ? e - i * (i + 1) / 2 : kSpdMax;
-    rb[m] = e < np ? i * (i + 1) / 2 : 0;
-    cb[m] = e < np ? ec[m] * (ec[m] + 1) / 2 : 0;
-  }
-  // right-looking Cholesky, two barriers per column: every thread reads the pivot
-  // and takes its square root itself (the same value everywhere, so the break on a
-  // non-positive pivot is block-uniform); thread 0 records it in dgl
+      for (int u = 0; u < 4; ++u)
+        acol[buf][at(ti, u)] = hi ? make_double2(av[u][2], av[u][3]) : make_double2(av[u][0], av[u][1]);
+    }
+    if (ti == q) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        yrow[buf][at(tj, v)] = hi ? make_double2(yv[2][v], yv[3][v]) : make_double2(yv[0][v], yv[1][v]);
+    }
+  };
+  publish(0, 0);
   int bad = 0;
-  for (int j = 0; j < k; ++j) {
+#pragma unroll 1
+  for (int j = 0; j < k; j += 2) {
+    const int cur = (j >> 1) & 1;
     __syncthreads();
-    const double v = Ls[pk(j, j)];
-    if (!(v > 0.0)) {
+    const double2 c0 = acol[cur][j], c1 = acol[cur][j + 1];  // (a_jj, .), (a_j+1,j, a_j+1,j+1)
+    double2 ai[4], ac[4], y[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      ai[u] = acol[cur][at(ti, u)];
+      ac[u] = acol[cur][at(tj, u)];
+      y[u] = yrow[cur][at(tj, u)];
+    }
+    const double p0 = c0.x, r0 = rcp_f64(p0), l = c1.x * r0, p1 = fma(-l, c1.x, c1.y);
+    // uniform: every thread reads the same two pivots
+    if (!(p0 > 0.0)) {
       bad = j + 1;
       break;
     }
-    const double djj = sqrt(v);
-    if (t == 0) dgl[j] = djj;
-    for (int i = j + 1 + t; i < k; i += 256) Ls[pk(i, j)] /= djj;
-    __syncthreads();
-    // trailing update of the lower triangle: entries (i, l) with j < l <= i. It reads
-    // column j and writes only columns > j, so all reads go first (unconditional: the
-    // offsets stay inside the triangle) and the writes after
-    double lv[kM], rv[kM], ov[kM];
+    if (!(p1 > 0.0)) {
+      bad = j + 2;
+      break;
+    }
+    if (t == 0) {
+      piv[j] = p0;
+      piv[j + 1] = p1;
+    }
+    const double r1 = rcp_f64(p1);
+    double b1[4], y1[4];  // column j + 1 and row j + 1 after pivot j
 #pragma unroll
-    for (int m = 0; m < kM; ++m) {
-      lv[m] = Ls[rb[m] + min(j, er[m] < 0 ? 0 : er[m])];
-      rv[m] = Ls[cb[m] + (ec[m] < kSpdMax ? min(j, ec[m]) : 0)];
-      ov[m] = Ls[min(t + 256 * m, kPack - 1)];
+    for (int v = 0; v < 4; ++v) {
+      b1[v] = fma(-l, ac[v].x, ac[v].y);
+      y1[v] = fma(-l, y[v].x, y[v].y);
     }
 #pragma unroll
-    for (int m = 0; m < kM; ++m)
-      if (ec[m] > j && ec[m] < kSpdMax) Ls[t + 256 * m] = ov[m] - lv[m] * rv[m];
+    for (int u = 0; u < 4; ++u) {
+      const int i = at(ti, u);
+      const double f0 = i > j ? -ai[u].x * r0 : 0.0;                           // rows up to j are final
+      const double f1 = i > j + 1 ? -fma(-l, ai[u].x, ai[u].y) * r1 : 0.0;  // ... up to j + 1
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        av[u][v] = fma(f1, b1[v], fma(f0, ac[v].x, av[u][v]));
+        yv[u][v] = fma(f1, y1[v], fma(f0, y[v].x, yv[u][v]));
+      }
+    }
+    if (j + 2 < k) publish(cur ^ 1, j + 2);
   }
   if (t == 0) status[b] = bad;
   if (bad) return;
   __syncthreads();
-  if (t < k) Ls[pk(t, t)] = dgl[t];
-  // X = L^-1, one row per step: row q is final once the steps before it have added
-  // their terms, X[q][c] = -(sum_{c<=p<q} L[q][p] X[p][c]) / L[q][q]; the step then adds
-  // L[i][q] X[q][c] to every later row i. Each sum takes its terms in increasing p,
-  // the order of a column-by-column forward substitution.
-  for (int q = 0; q < k; ++q) {
-    __syncthreads();
-    if (t <= q) Xs[pk(q, t)] = t == q ? 1.0 / Ls[pk(q, q)] : -Xs[pk(q, t)] / Ls[pk(q, q)];
-    __syncthreads();
-    // rows > q are written, row q and L are read: reads first, then writes
-    const int qb = q * (q + 1) / 2;
-    double lv[kM], xv[kM], ov[kM];
+  // X = L^-1 = D^-1/2 Y
 #pragma unroll
-    for (int m = 0; m < kM; ++m) {
-      lv[m] = Ls[rb[m] + min(q, er[m] < 0 ? 0 : er[m])];
-      xv[m] = Xs[qb + min(ec[m], q)];
-      ov[m] = Xs[min(t + 256 * m, kPack - 1)];
+  for (int u = 0; u < 4; ++u) {
+    const int i = at(ti, u);
+    const double d = i < k ? 1.0 / sqrt(piv[i]) : 0.0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int c = at(tj, v);
+      Xs[i * kSpdPitch + c] = c <= i && i < k ? yv[u][v] * d : 0.0;
     }
-#pragma unroll
-    for (int m = 0; m < kM; ++m)
-      if (er[m] > q && ec[m] <= q) Xs[t + 256 * m] = fma(lv[m], xv[m], ov[m]);
   }
   __syncthreads();
   double* Li = linv + (int64_t)b * kk;
-  for (int e = t; e < kk; e += 256) {
+  for (int e = t; e < k * k; e += 256) {
     const int r = e / k, cc = e % k;
-    Li[e] = cc <= r ? Xs[pk(r, cc)] : 0.0;
-    if (linvT32) linvT32[(int64_t)b * kk + e] = r <= cc ? (float)Xs[pk(cc, r)] : 0.f;
+    Li[e] = Xs[r * kSpdPitch + cc];
+    if (linvT32) linvT32[(int64_t)b * kk + e] = (float)Xs[cc * kSpdPitch + r];
   }
   if (inv64 || inv32) {
-    // S^-1 = X^T X: thread owns the 4 x 4 block at rows r0.., columns c0..; entry (r, c)
-    // sums X[q][r] X[q][c] over q >= max(r, c) in increasing q (the block's earlier q
-    // add exact zeros, as X[q][r] = 0 for r > q)
-    const int r0 = 4 * (t >> 4), c0 = 4 * (t & 15);
+    // S^-1 = X^T X: thread owns the 4 x 4 block at rows r0.., columns c0..; rows q below the block's
+    // first nonzero add exact zeros and are skipped
+    const int r0 = 4 * ti, c0 = 4 * tj;
     if (r0 < k && c0 < k) {
       double acc[4][4];
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
         for (int w = 0; w < 4; ++w) acc[u][w] = 0.0;
-#pragma unroll 2
+#pragma unroll 4
       for (int q = r0 > c0 ? r0 : c0; q < k; ++q) {
-        double xr[4], xc[4];
-        const int base = q * (q + 1) / 2;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          xr[u] = r0 + u <= q ? Xs[base + r0 + u] : 0.0;
-          xc[u] = c0 + u <= q ? Xs[base + c0 + u] : 0.0;
-        }
+        const double* xr = Xs + q * kSpdPitch + r0;
+        const double* xc = Xs + q * kSpdPitch + c0;
+        const double2 ra = *reinterpret_cast<const double2*>(xr), rb = *reinterpret_cast<const double2*>(xr + 2);
+        const double2 ca = *reinterpret_cast<const double2*>(xc), cb = *reinterpret_cast<const double2*>(xc + 2);
+        const double rv[4] = {ra.x, ra.y, rb.x, rb.y}, cv[4] = {ca.x, ca.y, cb.x, cb.y};
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-          for (int w = 0; w < 4; ++w) acc[u][w] = fma(xr[u], xc[w], acc[u][w]);
+          for (int w = 0; w < 4; ++w) acc[u][w] = fma(rv[u], cv[w], acc[u][w]);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u)
@@ -696,99 +722,102 @@ __global__ __launch_bounds__(256) void spd_inv_kernel(int k, const double* __res
 //   f  = sum_i w_i sum_a P[i][a] T[i][a] / sum w      (= tr(S^-1 G^T U W U^T G) / sum w)
 //   C1 = -(2 / sum w) diag(w) P          (m x k)  so that  dL/dG = U C1 + G C2
 //   C2 =  (2 / sum w) P^T diag(w) P      (k x k)  for the loss L = 1 - f
-// T and the lower triangle of S^-1 live in LDS; P overwrites T once every thread has
-// read its row.
+// One block: two 64^3 products in FP64 from zero-padded LDS tiles, T transposed, each thread a 4 x 4
+// block, so a step of the sum is four 16-byte broadcasts against sixteen fmas.  P overwrites S^-1
+// once every thread has read it.  k = m = 64: 48.8 us with scalar LDS reads whose rows shared a bank,
+// now 13.3 us.
 __global__ __launch_bounds__(256) void energy_kernel(int k, int m, const double* __restrict__ Sinv,
                                                      const double* __restrict__ T, const double* __restrict__ w,
                                                      float* __restrict__ C1, float* __restrict__ C2,
                                                      double* __restrict__ loss) {
-  __shared__ double Ts[kSpdMax * kSpdMax];
-  __shared__ double Ss[kSpdMax * kSpdMax];  // S^-1 rebuilt symmetric from its lower triangle
+  __shared__ __align__(16) double Tt[kSpdMax * kSpdPitch];  // T^T: [q][i]
+  __shared__ __align__(16) double Ss[kSpdMax * kSpdPitch];  // S^-1 rebuilt symmetric from its lower triangle; P
   __shared__ double ws[kSpdMax];
   __shared__ double red[4];
-  const int t = threadIdx.x;
-  // loads in groups of eight per thread, indexes clamped so each group issues together
-  for (int e0 = 0; e0 < kSpdMax * kSpdMax; e0 += 2048) {
-    double vt[8], vs[8];
+  const int t = threadIdx.x, ti = t >> 4, tj = t & 15;
+  {
+    double vt[16], vs[16];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int e = e0 + t + 256 * q;
-      const int et = min(e, m * k - 1), es = min(e, k * k - 1), i = es / k, j = es % k;
-      vt[q] = T[et];
-      vs[q] = Sinv[i >= j ? es : j * k + i];
+    for (int q = 0; q < 16; ++q) {
+      const int e = t + 256 * q, i = e >> 6, j = e & 63;
+      const int hi = min(max(i, j), k - 1), lo = min(min(i, j), k - 1);
+      vt[q] = T[min(i, m - 1) * k + min(j, k - 1)];
+      vs[q] = Sinv[hi * k + lo];
     }
+    const double wv = w[min(t, m - 1)];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int e = e0 + t + 256 * q;
-      if (e < m * k) Ts[e] = vt[q];
-      if (e < k * k) Ss[e] = vs[q];
+    for (int q = 0; q < 16; ++q) {
+      const int e = t + 256 * q, i = e >> 6, j = e & 63;
+      Tt[j * kSpdPitch + i] = i < m && j < k ? vt[q] : 0.0;
+      Ss[i * kSpdPitch + j] = i < k && j < k ? vs[q] : 0.0;
     }
+    if (t < kSpdMax) ws[t] = t < m ? wv : 0.0;
   }
-  if (t < m) ws[t] = w[t];
   __syncthreads();
-  double wsum = 0.0;
-  for (int i = 0; i < m; ++i) wsum += ws[i];
+  const double wsum = block_sum<256>(t < m ? ws[t] : 0.0, red);
   const double c = 2.0 / wsum;
-  // P[i][a] = sum_q T[i][q] S^-1[q][a] for a = g + 4 u: sixteen independent sums per
-  // thread, each over q in increasing order
-  const int i = t >> 2, g = t & 3;
-  double pv[kSpdMax / 4];
+  auto load4 = [](const double* p, double (&o)[4]) {
+    const double2 x = *reinterpret_cast<const double2*>(p), y = *reinterpret_cast<const double2*>(p + 2);
+    o[0] = x.x;
+    o[1] = x.y;
+    o[2] = y.x;
+    o[3] = y.y;
+  };
+  const int i0 = 4 * ti, a0 = 4 * tj;
+  double pv[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) pv[u][v] = 0.0;
+#pragma unroll 4
+  for (int q = 0; q < k; ++q) {
+    double tv[4], sv[4];
+    load4(Tt + q * kSpdPitch + i0, tv);
+    load4(Ss + q * kSpdPitch + a0, sv);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) pv[u][v] = fma(tv[u], sv[v], pv[u][v]);
+  }
   double f = 0.0;
-  if (i < m) {
 #pragma unroll
-    for (int u = 0; u < kSpdMax / 4; ++u) pv[u] = 0.0;
-    for (int q = 0; q < k; ++q) {
-      const double tq = Ts[i * k + q];
-      const double* srow = Ss + q * k;
+  for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int u = 0; u < kSpdMax / 4; ++u)
-        if (g + 4 * u < k) pv[u] = fma(tq, srow[g + 4 * u], pv[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < kSpdMax / 4; ++u) {
-      const int a = g + 4 * u;
-      if (a < k) {
-        C1[i * k + a] = (float)(-c * ws[i] * pv[u]);
-        f = fma(ws[i] * pv[u], Ts[i * k + a], f);
+    for (int v = 0; v < 4; ++v) {
+      const int i = i0 + u, a = a0 + v;
+      if (i < m && a < k) {
+        C1[i * k + a] = (float)(-c * ws[i] * pv[u][v]);
+        f = fma(ws[i] * pv[u][v], Tt[a * kSpdPitch + i], f);
       }
     }
-  }
-  f = block_sum<256>(f, red);  // its barriers also order every read of Ts before the writes below
-  if (i < m) {
+  f = block_sum<256>(f, red);  // its barriers also order every read of Ss before the writes below
 #pragma unroll
-    for (int u = 0; u < kSpdMax / 4; ++u) {
-      const int a = g + 4 * u;
-      if (a < k) Ts[i * k + a] = pv[u];
-    }
-  }
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) Ss[(i0 + u) * kSpdPitch + a0 + v] = pv[u][v];
   __syncthreads();
-  // C2[a][b] = c sum_r (w_r P[r][a]) P[r][b]: thread owns the 4 x 4 block at (a0, b0)
-  const int a0 = 4 * (t >> 4), b0 = 4 * (t & 15);
-  if (a0 < k && b0 < k) {
-    double acc[4][4];
+  // C2[a][b] = c sum_r (w_r P[r][a]) P[r][b]: thread owns the 4 x 4 block at (i0, a0)
+  double acc[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[u][v] = 0.0;
+#pragma unroll 4
+  for (int r = 0; r < m; ++r) {
+    double pa[4], pb[4];
+    load4(Ss + r * kSpdPitch + i0, pa);
+    load4(Ss + r * kSpdPitch + a0, pb);
+    const double wr = ws[r];
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) acc[u][v] = 0.0;
-    for (int r = 0; r < m; ++r) {
-      const double* prow = Ts + r * k;
-      double wa[4], pb[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        wa[u] = ws[r] * prow[min(a0 + u, k - 1)];
-        pb[u] = prow[min(b0 + u, k - 1)];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] = fma(wa[u], pb[v], acc[u][v]);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (a0 + u < k && b0 + v < k) C2[(a0 + u) * k + b0 + v] = (float)(c * acc[u][v]);
+      for (int v = 0; v < 4; ++v) acc[u][v] = fma(wr * pa[u], pb[v], acc[u][v]);
   }
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (i0 + u < k && a0 + v < k) C2[(i0 + u) * k + a0 + v] = (float)(c * acc[u][v]);
   if (t == 0) loss[0] = 1.0 - f / wsum;
 }
 
@@ -1053,14 +1082,14 @@ int ck_mlp_forward(int64_t n, int32_t din, int32_t dout, const float* X, int64_t
     return CK_ERR_BAD_ARG;
   if ((Z1 == nullptr) != (Z2 == nullptr) || (Z1 && ldz < n)) return CK_ERR_BAD_ARG;
   if (reinterpret_cast<uintptr_t>(params) % 16) return CK_ERR_BAD_ARG;  // weights are staged as float4
-  const unsigned grid = (unsigned)cdiv(n, kRows);
   hipStream_t s = (hipStream_t)stream;
+  const dim3 grid((unsigned)cdiv(n, kFwdRows));
   if (Z1)
-    hipLaunchKernelGGL(mlp_fwd_kernel<true>, dim3(grid), dim3(256), 0, s, (int)n, din, dout, X, ldx, params, G, gsr,
-                       gsc, Z1, Z2, ldz);
+    hipLaunchKernelGGL(mlp_fwd_kernel<true>, grid, dim3(256), 0, s, (int)n, din, dout, X, ldx, params, G, gsr, gsc, Z1,
+                       Z2, ldz);
   else
-    hipLaunchKernelGGL(mlp_fwd_kernel<false>, dim3(grid), dim3(256), 0, s, (int)n, din, dout, X, ldx, params, G, gsr,
-                       gsc, Z1, Z2, ldz);
+    hipLaunchKernelGGL(mlp_fwd_kernel<false>, grid, dim3(256), 0, s, (int)n, din, dout, X, ldx, params, G, gsr, gsc, Z1,
+                       Z2, ldz);
   CK_CHECK_LAUNCH();
   return CK_OK;
 }
@@ -1077,8 +1106,9 @@ int ck_mlp_backward(int64_t n, int32_t din, int32_t dout, const float* X, int64_
   const int64_t total = mlp_layout(din, dout).total;
   hipStream_t s = (hipStream_t)stream;
   float* part = static_cast<float*>(work);
-  hipLaunchKernelGGL(mlp_bwd_kernel, dim3(nblk), dim3(256), 0, s, (int)n, din, dout, X, ldx, params, Z1, Z2, ldz, dG,
-                     dsr, dsc, part);
+  const unsigned split = nblk <= 64 ? 4 : nblk <= 128 ? 2 : 1;  // blocks per chunk until they fill the chip
+  hipLaunchKernelGGL(mlp_bwd_kernel, dim3(nblk, split), dim3(512), 0, s, (int)n, din, dout, X, ldx, params, Z1, Z2, ldz,
+                     dG, dsr, dsc, part);
   hipLaunchKernelGGL(grad_reduce_kernel, dim3((unsigned)cdiv(total, 256)), dim3(256), 0, s, nblk, total,
                      (const float*)part, grad_scale, grad);
   CK_CHECK_LAUNCH();
@@ -1121,7 +1151,7 @@ int ck_gram_f64(int64_t n, int32_t ka, int32_t kb, const float* X, int64_t xsr, 
 int ck_rows_gemm_f32(int64_t n, int32_t kin, int32_t kout, const float* X, int64_t xsr, int64_t xsc, const float* W,
                      float alpha, float beta, float* Y, int64_t ysr, int64_t ysc, void* stream) {
   if (n < 1 || kin < 1 || kin > kGemmMax || kout < 1 || !X || !W || !Y) return CK_ERR_BAD_ARG;
-  hipLaunchKernelGGL(rows_gemm_kernel, dim3((unsigned)cdiv(n, 256), (unsigned)cdiv(kout, 32)), dim3(256), 0,
+  hipLaunchKernelGGL(rows_gemm_kernel, dim3((unsigned)cdiv(n, 64), (unsigned)cdiv(kout, 32)), dim3(256), 0,
                      (hipStream_t)stream, n, kin, kout, X, xsr, xsc, W, alpha, beta, Y, ysr, ysc);
   CK_CHECK_LAUNCH();
   return CK_OK;
