@@ -174,16 +174,6 @@ __device__ __forceinline__ float4 load4_masked(const float* __restrict__ p, int6
   return r;
 }
 
-// elements idx..idx+3 of p: a plain 16-byte load when the caller knows they are all below n
-// (every tile but a vector's last), so no load sits behind a bounds branch that would make
-// the compiler wait for the loads before it.  (The two-sweep kernels keep the masked loads:
-// there the plain form measured 11-17% slower on the 1024^2 Laplacian basis.)
-template <bool FULL>
-__device__ __forceinline__ float4 load4(const float* __restrict__ p, int64_t idx, int64_t n) {
-  if constexpr (FULL) return *reinterpret_cast<const float4*>(p + idx);
-  else return load4_masked(p, idx, n);
-}
-
 // hpart[j * P + blk] = V[:, j]^T w over this block's 1024-element tile, j0 <= j <= j1, with
 // the tile of w staged in wl.  Each lane owns 4 consecutive elements of each 256-element
 // quarter; two basis vectors (j, j+4) per pass keep eight 16-byte loads in flight per lane.
@@ -428,95 +418,90 @@ __global__ __launch_bounds__(256) void lz_apply_project(int64_t n, float* __rest
   project_tile_vec<true>(Vb, ldv, n, i0, j0, j1, wl, hpart + (int64_t)b * M2 * P, P, blk);
 }
 
-// RPL consecutive elements idx.. of p (zero past n): one 16-, 8- or 4-byte load
-template <int RPL, bool FULL>
-__device__ __forceinline__ void load_rows(const float* __restrict__ p, int64_t idx, int64_t n, float (&r)[RPL]) {
-  if constexpr (RPL == 4) {
-    const float4 v = load4<FULL>(p, idx, n);
-    r[0] = v.x, r[1] = v.y, r[2] = v.z, r[3] = v.w;
-  } else if constexpr (RPL == 2) {
-    if (FULL || idx + 1 < n) {
-      const float2 v = *reinterpret_cast<const float2*>(p + idx);
-      r[0] = v.x, r[1] = v.y;
-    } else {
-      r[0] = idx < n ? p[idx] : 0.f;
-      r[1] = 0.f;
-    }
-  } else {
-    r[0] = (FULL || idx < n) ? p[idx] : 0.f;
-  }
-}
-
 // The same two passes as lz_apply_project with one read of the basis: the block's 1024-row
-// tile is walked in sub-tiles of SR rows; each wave takes the columns j0 + wave + 4c
-// (c < 4 JW, so up to 16 JW columns; 32 KB of LDS for the staged rows), adds their share of
-// V h for its lane's RPL = SR / 64 rows and keeps the loaded rows in LDS; after one barrier
-// every wave forms the updated w for its lane's rows (the four shares in wave order), wave 0
-// stores it, and each wave accumulates its columns' dot products from the LDS copy.  The
-// per-lane sums run across the sub-tiles; one wave sum per column at the end gives the
-// tile's partial.  The tiles below n (all but a vector's last) load without bounds masks.
-template <int SR, int JW, bool FULL>
-__device__ __forceinline__ void apply_project_tile(int64_t n, const float* __restrict__ Vb, int64_t ldv,
-                                                   float* __restrict__ w, int64_t i0, int j0, int j1,
-                                                   const float* hs, float (*Vs)[SR], float (*red)[SR],
-                                                   float* __restrict__ hp, int P, int blk) {
-  constexpr int RPL = SR / 64;
-  constexpr int NC = 4 * JW;  // column slots per wave
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+// tile is walked in sub-tiles of SR = 64 RPL rows; each wave takes the columns j0 + wave + 4c
+// (c < NC), adds their share of V h for its lane's RPL rows and keeps what it loaded in registers
+// (NC * RPL of them); after one barrier every wave forms the updated w for its lane's rows (the
+// four shares in wave order), wave 0 stores it, and each wave accumulates its columns' dot products
+// from its registers.  The per-lane sums run across the sub-tiles; one wave sum per column at
+// the end gives the tile's partial.  MASK (a vector's last tile): rows from `left` on count as zero
+// and are not stored; their 16-byte pieces end inside ldv, which is a multiple of four.  A column's
+// base is the same in every lane and the lane offset 32 bits, so a column costs no vector address.
+template <int RPL, int NC, bool MASK>
+__device__ __forceinline__ void apply_project_tile(int left, const float* __restrict__ Vb, int64_t ldv,
+                                                   float* __restrict__ w, int64_t i0, int j0, int j1, const float* hs,
+                                                   float (*red)[4][64 * RPL], float* __restrict__ hp, int P,
+                                                   int blk) {
+  typedef float vec __attribute__((ext_vector_type(RPL)));
+  constexpr int SR = 64 * RPL;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // columns of this wave: j0 + wv + 4 c for c < nc
   const int nc = j0 + wv > j1 ? 0 : (j1 - j0 - wv) / 4 + 1;
+  const float* base = Vb + i0;
+  float* wb = w + i0;
   float acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = 0.f;
+#pragma unroll 1
   for (int st = 0; st < kTile / SR; ++st) {
-    const int64_t idx = i0 + st * SR + RPL * lane;
-    float wr[RPL], part[RPL];
-    load_rows<RPL, FULL>(w, idx, n, wr);
-#pragma unroll
-    for (int q = 0; q < RPL; ++q) part[q] = 0.f;
-    // four columns per batch, loads clamped to the last column and issued together
+    const uint32_t off = st * SR + RPL * lane, offc = MASK && (int)off >= left ? 0 : off;
+    vec part = {}, v[NC];
+    // loads clamped to the last column, all issued together
 #pragma unroll
     for (int c0 = 0; c0 < NC; c0 += 4) {
       if (c0 >= nc) break;
-      float v[4][RPL];
 #pragma unroll
       for (int u = 0; u < 4; ++u)
-        load_rows<RPL, FULL>(Vb + (int64_t)min(j0 + wv + 4 * (c0 + u), j1) * ldv, idx, n, v[u]);
+        v[c0 + u] = *reinterpret_cast<const vec*>(base + (int64_t)min(j0 + wv + 4 * (c0 + u), j1) * ldv + offc);
+    }
+    vec wr = *reinterpret_cast<const vec*>(wb + offc);
+    if (MASK) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        float* dst = &Vs[wv * NC + c0 + u][RPL * lane];
+      for (int q = 0; q < RPL; ++q) {
+        const bool in = (int)off + q < left;
+        wr[q] = in ? wr[q] : 0.f;
 #pragma unroll
-        for (int q = 0; q < RPL; ++q) dst[q] = v[u][q];
-        const float hv = hs[min(j0 + wv + 4 * (c0 + u), j1)];
-        const float hj = c0 + u < nc ? hv : 0.f;
-#pragma unroll
-        for (int q = 0; q < RPL; ++q) part[q] = fmaf(v[u][q], hj, part[q]);
+        for (int c = 0; c < NC; ++c) v[c][q] = in ? v[c][q] : 0.f;
       }
     }
 #pragma unroll
-    for (int q = 0; q < RPL; ++q) red[wv][RPL * lane + q] = part[q];
+    for (int c0 = 0; c0 < NC; c0 += 4) {
+      if (c0 >= nc) break;
+      // hs[wave][c]: zero past this wave's columns
+      const float4 h4 = *reinterpret_cast<const float4*>(hs + wv * NC + c0);
+      const float hj[4] = {h4.x, h4.y, h4.z, h4.w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int q = 0; q < RPL; ++q) part[q] = fmaf(v[c0 + u][q], hj[u], part[q]);
+    }
+    float (*rd)[SR] = red[st & 1];  // two buffers: one barrier per sub-tile
+    *reinterpret_cast<vec*>(&rd[wv][RPL * lane]) = part;
     __syncthreads();
-    float w1[RPL];
+    vec sum4[4];
 #pragma unroll
-    for (int q = 0; q < RPL; ++q) {
-      const int r = RPL * lane + q;
-      w1[q] = wr[q] - (((red[0][r] + red[1][r]) + red[2][r]) + red[3][r]);
-    }
+    for (int k = 0; k < 4; ++k) sum4[k] = *reinterpret_cast<const vec*>(&rd[k][RPL * lane]);
+    const vec w1 = wr - (((sum4[0] + sum4[1]) + sum4[2]) + sum4[3]);
     if (wv == 0) {
+      if (!MASK || (int)off + RPL <= left) {
+        *reinterpret_cast<vec*>(wb + off) = w1;
+      } else {
 #pragma unroll
-      for (int q = 0; q < RPL; ++q)
-        if (FULL || idx + q < n) w[idx + q] = w1[q];
+        for (int q = 0; q < RPL; ++q)
+          if ((int)off + q < left) wb[off + q] = w1[q];
+      }
     }
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      if (c >= nc) break;
-      const float* src = &Vs[wv * NC + c][RPL * lane];
-      float d = 0.f;
+    for (int c0 = 0; c0 < NC; c0 += 4) {
+      if (c0 >= nc) break;
 #pragma unroll
-      for (int q = 0; q < RPL; ++q) d = fmaf(src[q], w1[q], d);
-      acc[c] += d;
+      for (int u = 0; u < 4; ++u) {
+        float d = 0.f;
+#pragma unroll
+        for (int q = 0; q < RPL; ++q) d = fmaf(v[c0 + u][q], w1[q], d);
+        acc[c0 + u] += d;
+      }
     }
-    __syncthreads();  // Vs and red are rewritten by the next sub-tile
   }
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
@@ -526,41 +511,55 @@ __device__ __forceinline__ void apply_project_tile(int64_t n, const float* __res
   }
 }
 
-template <int SR, int JW>
-__global__ __launch_bounds__(256) void lz_apply_project_lds(int64_t n, float* __restrict__ V, int64_t ldv,
+template <int RPL, int NC, int WPE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void lz_apply_project_one(int64_t n, float* __restrict__ V, int64_t ldv,
                                                             int64_t ldb, int wcol, int j0, int j1,
                                                             const float* __restrict__ h, int M2,
                                                             float* __restrict__ hpart, int P,
                                                             const int* __restrict__ done) {
   if (done && *done) return;
-  __shared__ float hs[1056];
-  __shared__ __align__(16) float Vs[16 * JW][SR];
-  __shared__ __align__(16) float red[4][SR];
+  __shared__ __align__(16) float hs[4 * NC];  // by wave, zero past its columns
+  __shared__ __align__(16) float red[2][4][64 * RPL];
   const int b = blockIdx.y, blk = blockIdx.x;
-  for (int j = threadIdx.x; j < M2 && j < 1056; j += 256) hs[j] = h[b * M2 + j];
+  if (threadIdx.x < 4 * NC) {
+    const int j = j0 + (threadIdx.x / NC) + 4 * (threadIdx.x % NC);
+    hs[threadIdx.x] = j <= j1 ? h[b * M2 + j] : 0.f;
+  }
   __syncthreads();
   float* Vb = V + b * ldb;
   float* w = Vb + (int64_t)wcol * ldv;
   const int64_t i0 = (int64_t)blk * kTile;
   float* hp = hpart + (int64_t)b * M2 * P;
-  if (i0 + kTile <= n)
-    apply_project_tile<SR, JW, true>(n, Vb, ldv, w, i0, j0, j1, hs, Vs, red, hp, P, blk);
+  const int64_t left = n - i0;
+  if (left >= kTile)
+    apply_project_tile<RPL, NC, false>(kTile, Vb, ldv, w, i0, j0, j1, hs, red, hp, P, blk);
   else
-    apply_project_tile<SR, JW, false>(n, Vb, ldv, w, i0, j0, j1, hs, Vs, red, hp, P, blk);
+    apply_project_tile<RPL, NC, true>((int)left, Vb, ldv, w, i0, j0, j1, hs, red, hp, P, blk);
 }
 
 // w -= V[:, j0..j1] h, then the partials of V[:, j0..j1]^T w (the two CGS2 passes between
-// the reductions): one read of the basis for up to 32 columns, else lz_apply_project.
+// the reductions).  Up to 128 columns the basis is read once: a wave's share of the columns fits
+// its registers, as many rows per lane as leave two waves per SIMD or more.  HBM bound, and as fast as
+// one plain sweep: 630900 x 48 columns 22.4 us (5.4 TB/s), x 80 36.5 us, x 98 49 us, where two sweeps
+// take 36 us at 50 columns and 47 at 66; 16 x 262144 x 15.5 columns 52.7 us against 59 with the columns
+// staged in LDS.
 inline void launch_apply_project(dim3 grid, hipStream_t s, int64_t n, float* V, int64_t ldv, int64_t ldb, int wcol,
                                  int j0, int j1, const float* h, int M2, float* hpart, int P, const int* done) {
-  // measured on a 1024^2 Laplacian basis: the staged kernel wins up to 32 columns (SLQ's 32-probe
-  // bases of 30 steps: 14% per step); with more columns its smaller sub-tiles and lower occupancy
-  // lose to the two-sweep kernel, whose second sweep partly hits the caches
-  if (j1 - j0 + 1 <= 32)
-    hipLaunchKernelGGL((lz_apply_project_lds<256, 2>), grid, dim3(256), 0, s, n, V, ldv, ldb, wcol, j0, j1, h, M2,
-                       hpart, P, done);
+  const int cols = j1 - j0 + 1;
+#define CK_ONE(RPL_, NC_, W_)                                                                                             \
+  hipLaunchKernelGGL((lz_apply_project_one<RPL_, NC_, W_>), grid, dim3(256), 0, s, n, V, ldv, ldb, wcol, j0, j1, h, M2, \
+                     hpart, P, done)
+  if (cols <= 32)
+    CK_ONE(4, 8, 5);
+  else if (cols <= 64)
+    CK_ONE(4, 16, 3);
+  else if (cols <= 96)
+    CK_ONE(4, 24, 2);
+  else if (cols <= 128)
+    CK_ONE(2, 32, 2);
   else
     hipLaunchKernelGGL(lz_apply_project, grid, dim3(256), 0, s, n, V, ldv, ldb, wcol, j0, j1, h, M2, hpart, P, done);
+#undef CK_ONE
 }
 
 // beta_i = ||w||, errors and the loop condition (lanczos.py:251-268)
