@@ -4,7 +4,8 @@
 // normalisation, threshold tol*||r0|| + tol, safe division at 1e-40, frozen columns), the
 // loop of cola/utils/torch_tqdm.py:86-90 runs inside the kernel.  Scope: small dense
 // operators (y = scale*A x + shift*x) whose solves are launch- and latency-bound, with no
-// preconditioner or a diagonal one.
+// preconditioner or a diagonal one.  Orders whose matrix fits the registers of one workgroup
+// are solved by one (second half of this file); the rest as follows.
 //
 // Each workgroup owns a contiguous block of R <= 64 rows.  Its rows of A are staged in LDS
 // once (when they fit), and every workgroup keeps the FULL r and p vectors in LDS.  A step:
@@ -470,6 +471,301 @@ __global__ __launch_bounds__(kNT) void fused_cg_kernel(FusedArgs a) {
   }
 }
 
+// ------------------------------------------------------------------ one workgroup
+// Up to 320 unknowns (256 for two to four columns) the whole matrix fits the registers of one
+// workgroup, and the solve needs no exchange between workgroups, which is what a step costs
+// above: stores that land, polls that see them, about 4 of 6 us on eight XCDs.
+//
+// 512 threads hold A as 8 waves x 4Q rows: lane (b, i) = (lane / 4, lane % 4) of a wave keeps
+// row 4q + i at columns 64c + 4b .. + 3 for q < Q, c < KC (Q = 2 KC; 200 registers at 320),
+// loaded once with 16-byte loads.  A step reads p from LDS, 16 bytes per lane and chunk of 64
+// columns, and needs no other operand: one column on the VALU (4 Q KC FMAs per lane, 1600
+// cycles at 320), two to four columns on v_mfma_f32_4x4x1_16b, whose sixteen blocks take the
+// sixteen b's as sixteen different k and whose A operand is the same register.  The sums over
+// b are two rounds of half swaps, which halve the registers as they go, and two rotations
+// within a row of sixteen.  Entry j of x, r, p is thread j's; the scalars of column c are
+// computed by the lanes = c mod NB of every wave alike, so a step has four barriers.
+// Bound by that serial chain: orders 64 / 150 / 300 and 256 x 4 columns take 1.4 / 1.6 / 1.9 and
+// 4.3 us a step, over n / 8 workgroups 5.0 / 5.4 / 6.0 and 10.9.  At 300 x 2 to 4 columns the
+// matrix, 40 accumulators and the columns' vectors no longer fit 256 registers.
+constexpr int kOneThreads = 512;
+constexpr int kOneChunks = 5, kOneChunksMulti = 4;  // chunks of 64 unknowns: one column; two to four
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// a + its half swap with b: the sums over lane bit 5 (or 4) of a in the lanes where the bit is
+// clear and of b where it is set.
+__device__ inline float add_swap32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ inline float add_swap16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// v[m] summed over lane bits 2..5; f(m, sum) is called with the m that this lane's row of
+// sixteen holds.
+template <int M, typename F>
+__device__ inline void sum_over_blocks(float (&v)[M], int lane, F f) {
+  constexpr int M1 = (M + 1) / 2, M2 = (M1 + 1) / 2;
+  float u[M1];
+#pragma unroll
+  for (int i = 0; i < M1; ++i) u[i] = add_swap32(v[2 * i], 2 * i + 1 < M ? v[2 * i + 1 < M ? 2 * i + 1 : 0] : 0.f);
+#pragma unroll
+  for (int i = 0; i < M2; ++i) {
+    float w = add_swap16(u[2 * i], 2 * i + 1 < M1 ? u[2 * i + 1 < M1 ? 2 * i + 1 : 0] : 0.f);
+    w += dpp_f32<0x124>(w);  // row_ror:4
+    w += dpp_f32<0x128>(w);  // row_ror:8
+    const int m = 4 * i + 2 * ((lane >> 4) & 1) + (lane >> 5);
+    if (m < M) f(m, w);
+  }
+}
+
+template <int NB, int KC>
+__global__ __launch_bounds__(kOneThreads) void fused_one_kernel(FusedArgs a) {
+  constexpr int Q = 2 * KC, NP = 64 * KC, LD = NP + 16, NW = kOneThreads / 64;
+  __shared__ float pv[NB * LD];  // columns 16 banks apart: the four columns of a 16-byte read don't collide
+  __shared__ float yv[NB * NP];
+  __shared__ double red1[NW * NB], red2[2 * NW * NB];
+  const int n = a.n, B = a.nrhs, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int col = min(lane & (NB - 1), B - 1);  // the column whose scalars this lane computes
+  const bool own = tid < n, pre = a.d != nullptr;
+  CgView v = cg_view(a.state, B);
+
+  float av[KC][Q][4];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int row = 4 * (wave * Q + q) + (lane & 3);
+    const float* rp = a.A + (int64_t)min(row, n - 1) * a.lda;
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const int k = 64 * c + 4 * (lane >> 2);
+      f32x4 t = {0.f, 0.f, 0.f, 0.f};
+      if (c < KC - 1 || k + 3 < n) {  // KC = ceil(n / 64): only the last chunk can be short
+        t = *reinterpret_cast<const f32x4u*>(rp + k);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          if (k + e < n) t[e] = rp[k + e];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) av[c][q][e] = row < n ? t[e] : 0.f;
+    }
+  }
+  // yv = A p for p in pv, all columns
+  auto product = [&]() {
+    if constexpr (NB == 1) {
+      float acc[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) acc[q] = 0.f;
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        const f32x4 p4 = *reinterpret_cast<const f32x4*>(pv + 64 * c + 4 * (lane >> 2));
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int q = 0; q < Q; ++q) acc[q] = fmaf(av[c][q][e], p4[e], acc[q]);
+      }
+      sum_over_blocks<Q>(acc, lane, [&](int q, float s) {
+        if ((lane & 12) == 0) yv[4 * (wave * Q + q) + (lane & 3)] = s;
+      });
+    } else {
+      f32x4 acc[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        const f32x4 p4 = *reinterpret_cast<const f32x4*>(pv + col * LD + 64 * c + 4 * (lane >> 2));
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int q = 0; q < Q; ++q) acc[q] = __builtin_amdgcn_mfma_f32_4x4x1f32(av[c][q][e], p4[e], acc[q], 0, 0, 0);
+      }
+      float flat[4 * Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) flat[4 * q + i] = acc[q][i];
+      sum_over_blocks<4 * Q>(flat, lane, [&](int m, float s) {
+        if ((lane & 12) == 0) yv[(lane & 3) * NP + 4 * wave * Q + m] = s;
+      });
+    }
+  };
+  // sums over the block of w[c]; the result is this lane's column's, after a barrier
+  auto put_sum = [&](double* red, int c, double w) {
+    w = wave_sum(w);
+    if (lane == 0) red[wave * NB + c] = w;
+  };
+  auto total = [&](const double* red) {
+    double t[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) t[i] = red[i * NB + col];
+    return ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+  };
+
+  // cg.py:96-97: column norms of b and r = b / ||b||
+  float x[NB], r[NB], p[NB], z[NB];
+#pragma unroll
+  for (int c = 0; c < NB; ++c) {
+    x[c] = p[c] = z[c] = 0.f;
+    r[c] = own && c < B ? a.b[(int64_t)tid * a.b_rs + (int64_t)c * a.b_cs] : 0.f;
+    if (c < B) put_sum(red1, c, (double)r[c] * (double)r[c]);
+  }
+  const float dj = pre && own ? a.d[tid] : 0.f;
+  for (int i = tid; i < NB * LD; i += kOneThreads) pv[i] = 0.f;
+  __syncthreads();
+  const float mult = (float)sqrt(total(red1));
+#pragma unroll
+  for (int c = 0; c < NB; ++c) {
+    float m = readlane_f32(mult, c);
+    if (fabsf(m) < 1e-40f) m = 1e-40f;
+    r[c] /= m;
+  }
+  if (a.x0) {
+    // cg.py:123: r0 = b_norm - A x0 (x0 as given)
+#pragma unroll
+    for (int c = 0; c < NB; ++c)
+      if (own && c < B) pv[c * LD + tid] = x[c] = a.x0[(int64_t)tid * a.x0_rs + (int64_t)c * a.x0_cs];
+    __syncthreads();
+    product();
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < NB; ++c)
+      if (own && c < B) {
+        float y = a.scale * yv[c * NP + tid];
+        if (a.shift != 0.f) y = fmaf(a.shift, x[c], y);
+        r[c] -= y;
+      }
+  }
+  // cg.py:98-101,122-130: z = P r, p = z, gamma = r.z, threshold tol*||r0|| + tol
+#pragma unroll
+  for (int c = 0; c < NB; ++c)
+    if (c < B) {
+      z[c] = pre ? fmaf(a.dscale * dj, r[c], a.dshift * r[c]) : r[c];
+      p[c] = z[c];
+      if (own) pv[c * LD + tid] = p[c];
+      put_sum(red2, c, own ? (double)r[c] * (double)r[c] : 0.0);
+      put_sum(red2 + NW * NB, c, own ? (double)r[c] * (double)z[c] : 0.0);
+    }
+  __syncthreads();
+  float rnorm = (float)sqrt(total(red2)), gamma = (float)total(red2 + NW * NB), alpha = 0.f, beta = 0.f;
+  const float tol = a.tol * rnorm + a.tol;
+  int k = 0, status = CK_OK;
+  bool any, finite;
+  // errors[k] and the loop condition (cg.py:133-138)
+  auto check = [&]() {
+    float mean = 0.f;
+    any = false;
+    finite = true;
+#pragma unroll
+    for (int c = 0; c < NB; ++c)
+      if (c < B) {
+        const float rn = readlane_f32(rnorm, c);
+        mean += rn;
+        any = any || rn > readlane_f32(tol, c);
+        finite = finite && isfinite(rn);
+      }
+    if (tid == 0) v.errors[k] = mean / (float)B;
+    return !(any && k < a.max_iters);
+  };
+  bool done = check();
+  if (!finite) status = CK_ERR_NAN;
+  while (!done) {
+    product();
+    __syncthreads();
+    // p.Ap -> alpha (cg.py:143-147)
+    float ap[NB];
+#pragma unroll
+    for (int c = 0; c < NB; ++c)
+      if (c < B) {
+        ap[c] = own ? a.scale * yv[c * NP + tid] : 0.f;
+        if (a.shift != 0.f) ap[c] = fmaf(a.shift, p[c], ap[c]);
+        put_sum(red1, c, own ? (double)p[c] * (double)ap[c] : 0.0);
+      }
+    __syncthreads();
+    const double pap = total(red1);
+    const bool frozen = (double)rnorm < kSmall;
+    alpha = frozen ? 0.f : (float)safe_div((double)gamma, pap);
+    if (status == CK_OK && __ballot(!frozen && !(pap > 0.0)) != 0) status = CK_ERR_BREAKDOWN;
+    // x += alpha p, r -= alpha Ap, gamma' = r.z, ||r||^2
+#pragma unroll
+    for (int c = 0; c < NB; ++c)
+      if (c < B) {
+        const float al = readlane_f32(alpha, c);
+        x[c] = fmaf(al, p[c], x[c]);
+        r[c] = fmaf(-al, ap[c], r[c]);
+        z[c] = pre ? fmaf(a.dscale * dj, r[c], a.dshift * r[c]) : r[c];
+        put_sum(red2, c, own ? (double)r[c] * (double)r[c] : 0.0);
+        put_sum(red2 + NW * NB, c, own ? (double)r[c] * (double)z[c] : 0.0);
+      }
+    __syncthreads();
+    // beta = gamma'/gamma (cg.py:150-154), frozen columns keep beta = 0
+    const double rr = total(red2), rz = total(red2 + NW * NB);
+    beta = frozen ? 0.f : (float)safe_div(rz, (double)gamma);
+    gamma = (float)rz;
+    rnorm = (float)sqrt(rr);
+#pragma unroll
+    for (int c = 0; c < NB; ++c)
+      if (c < B) {
+        p[c] = fmaf(readlane_f32(beta, c), p[c], z[c]);
+        if (own) pv[c * LD + tid] = p[c];
+      }
+    ++k;
+    done = check();
+    if (done) {
+      if (!finite)
+        status = CK_ERR_NAN;
+      else if (any && status == CK_OK)
+        status = CK_ERR_MAXITER;
+    }
+    __syncthreads();
+  }
+  // cg.py:119: x and r back to the scale of b
+#pragma unroll
+  for (int c = 0; c < NB; ++c)
+    if (own && c < B) {
+      const float m = readlane_f32(mult, c);
+      a.x[(int64_t)tid * a.x_rs + (int64_t)c * a.x_cs] = x[c] * m;
+      if (a.r) a.r[(int64_t)tid * a.r_rs + (int64_t)c * a.r_cs] = r[c] * m;
+    }
+  if (tid < B) {
+    v.mult[tid] = mult;
+    v.tol[tid] = tol;
+    v.gamma[tid] = gamma;
+    v.alpha[tid] = alpha;
+    v.beta[tid] = beta;
+    v.rnorm[tid] = rnorm;
+  }
+  if (tid == 0) {
+    v.ctrl->k = k;
+    v.ctrl->done = 1;
+    v.ctrl->max_iters = a.max_iters;
+    v.ctrl->nrhs = B;
+    v.ctrl->nparts = 1;
+    v.ctrl->status = status;
+  }
+}
+
+// One workgroup takes the solve when nobody asks for more and the matrix fits its registers
+// (a wait_offset concerns the waits of the exchange, which one workgroup does not have).
+bool one_workgroup(int n, int B, int nblocks, int wait_offset) {
+  return nblocks <= 1 && wait_offset == 0 && n <= 64 * (B == 1 ? kOneChunks : kOneChunksMulti);
+}
+
+template <int KC>
+void launch_one(const FusedArgs& a, hipStream_t s) {
+  if (a.n > 64 * (KC - 1)) {
+    if (a.nrhs == 1)
+      hipLaunchKernelGGL((fused_one_kernel<1, KC>), dim3(1), dim3(kOneThreads), 0, s, a);
+    else if constexpr (KC <= kOneChunksMulti)
+      hipLaunchKernelGGL((fused_one_kernel<4, KC>), dim3(1), dim3(kOneThreads), 0, s, a);
+  } else if constexpr (KC > 1) {
+    launch_one<KC - 1>(a, s);
+  }
+}
+
 // Clears the exchange tags and the status before a solve.
 __global__ void fused_reset_kernel(uint64_t* xbuf, int64_t words, void* state) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words; i += (int64_t)gridDim.x * blockDim.x)
@@ -595,7 +891,8 @@ int fused_launch(const ck_op* A, const ck_op* P, int32_t nrhs, const float* b, i
   if (!pl.ok) return CK_ERR_UNSUPPORTED;
   if (xbuf_bytes < work_bytes_of(pl.nn, nrhs)) return CK_ERR_WORKSPACE;
   const int nb = nb_of(nrhs);
-  if (pl.G > max_coresident(pl.tile, nb, pl.lds)) return CK_ERR_UNSUPPORTED;
+  const bool one = one_workgroup(n, nrhs, nblocks, wait_offset);
+  if (!one && pl.G > max_coresident(pl.tile, nb, pl.lds)) return CK_ERR_UNSUPPORTED;
   FusedArgs a{};
   a.n = n;
   a.nn = pl.nn;
@@ -630,6 +927,11 @@ int fused_launch(const ck_op* A, const ck_op* P, int32_t nrhs, const float* b, i
   a.spin_limit = spin_limit > 0 ? spin_limit : kDefaultSpin;
   a.wait_offset = (uint32_t)wait_offset;
   hipStream_t s = (hipStream_t)stream;
+  if (one) {
+    launch_one<kOneChunks>(a, s);
+    CK_CHECK_LAUNCH();
+    return CK_OK;
+  }
   const int64_t words = (int64_t)2 * nrhs * pl.nn;
   const unsigned rblocks = (unsigned)(cdiv(words, 1024) < 64 ? cdiv(words, 1024) : 64);
   hipLaunchKernelGGL(fused_reset_kernel, dim3(rblocks), dim3(256), 0, s, a.xbuf, words, state);

@@ -310,7 +310,9 @@ int ck_cg_finish(int64_t n, int32_t nrhs, float* x, float* r, int64_t ld, const 
  * element strides (row stride, column stride), i.e. the reference's layout directly.
  * state: ck_cg_state_bytes(nrhs, max_iters), laid out and filled as by the chained
  * entry points (k, done, status, errors[0..k], per-column scalars); work:
- * ck_cg_fused_workspace_bytes.  nblocks = 0 picks the workgroup count.  Every grid-wide
+ * ck_cg_fused_workspace_bytes.  nblocks = 0 picks the workgroup count: one, with A in its
+ * registers and no exchange, up to n = 320 (256 for 2 to 4 columns), else one per 8 rows (at
+ * most 256).  Every grid-wide
  * wait gives up after spin_limit polling rounds (<= 0: about a second), records
  * CK_ERR_TIMEOUT in ctrl.status and ends the kernel; wait_offset (0 in normal use) is
  * added to the tag each wait expects, so a host can make every wait time out and exercise

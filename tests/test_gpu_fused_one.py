@@ -1,0 +1,87 @@
+"""The persistent CG on one workgroup (up to 320 unknowns, 256 for two to four columns: the matrix in
+registers) at the edges of its chunks of 64, against the same solve over several workgroups and FP64."""
+import pytest
+import torch
+
+import cola_amd as ca
+from cola_amd.linalg.cg import fused_solve
+from oracle import cg as ocg
+
+pytestmark = pytest.mark.gpu
+
+EPS = 2.0**-24
+
+
+def rel(a, b):
+    return float((a.double().cpu() - b.double().cpu()).norm() / b.double().norm())
+
+
+@pytest.mark.parametrize("n,B", [(1, 1), (2, 3), (5, 4), (63, 1), (64, 2), (65, 1), (127, 4), (128, 1), (129, 3), (192, 1),
+                                 (193, 2), (255, 1), (256, 4), (257, 1), (257, 2), (319, 1), (320, 1), (321, 1)])
+@pytest.mark.parametrize("pre", [False, True])
+def test_one_workgroup(dev, n, B, pre):
+    """nblocks = 0 (one workgroup at these orders) against nblocks = 64 and FP64.  The matrix is a view
+    with an odd row stride and a dword offset, b and x0 have the columns apart, A is not symmetric to the
+    bit.  cond(A) <= 200: both stop at 1e-6 of the residual, and a step's 32-bit sums of n terms err by
+    at most n EPS ||A|| in norm, so the iterates differ by at most cond * (2e-6 + n EPS)."""
+    g = torch.Generator().manual_seed(n + B)
+    M = torch.randn(n, n, generator=g)
+    A = M @ M.T / n
+    A = A / torch.linalg.matrix_norm(A, 2) + 0.01 * torch.eye(n)
+    A = A + EPS * torch.randn(n, n, generator=g) * A.abs()
+    big = torch.zeros(n + 1, n + 2 + n % 2 + 1)
+    big[1:, 1:n + 1] = A
+    view = big.to(dev)[1:, 1:n + 1]
+    b = torch.randn(B, n, generator=g)
+    x0 = 0.1 * torch.randn(B, n, generator=g)
+    d = torch.rand(n, generator=g) + 0.5
+    op = ca.Dense(view) * 2.0 + 0.25 * ca.I_like(ca.Dense(view)) if pre else ca.Dense(view)
+    Ad = (2.0 * A.double() + 0.25 * torch.eye(n)) if pre else A.double()
+    P = ca.Diagonal(d.to(dev)) if pre else None
+    x0d = x0.to(dev).T if pre else None
+    args = (op, b.to(dev).T, x0d, 600, 1e-6, P)
+    x, r, k, info = fused_solve(*args)
+    xm, rm, km, im = fused_solve(*args, nblocks=64)
+    x64, r64, k64, _ = ocg.run_batched_cg(lambda V: Ad @ V, b.T.double(), x0.T.double() if pre else None, 600, 1e-6,
+                                          (lambda V: d.double()[:, None] * V) if pre else None)
+    bound = 200 * (2e-6 + n * EPS)
+    print(n, B, pre, k, km, k64, rel(x, xm), rel(x, x64), rel(xm, x64), flush=True)
+    assert info["status"] == im["status"] == "ok"
+    # 32-bit recurrences lose conjugacy from about n steps on: the counts agree to a few steps there
+    assert abs(k - km) <= 2 + km // 10 and abs(k - k64) <= 2 + max(k64, n // 8) // 10 * 3
+    assert rel(x, x64) < bound and rel(x, xm) < 2 * bound
+    assert len(info["errors"]) == k
+    m = min(3, k)
+    assert torch.allclose(torch.tensor(info["errors"][:m]), torch.tensor(im["errors"][:m]), rtol=1e-4, atol=1e-7)
+
+
+@pytest.mark.parametrize("n,B", [(100, 1), (100, 3), (300, 1)])
+def test_one_workgroup_capture(dev, n, B):
+    """The solve under graph capture (one node) replays on new values of its inputs."""
+    import cola_amd._native as N
+    from cola_amd.linalg._engine import lower
+    g = torch.Generator().manual_seed(n)
+    M = torch.randn(n, 2 * n, generator=g)
+    A = (M @ M.T / (2 * n) + 0.5 * torch.eye(n)).to(dev)
+    aop = lower(ca.Dense(A))
+    b, x = torch.zeros(n, B, device=dev), torch.empty(n, B, device=dev)
+    state = torch.zeros(N.q("ck_cg_state_bytes", B, 200), dtype=torch.uint8, device=dev)
+
+    def solve():
+        N.call("ck_cg_fused_noalloc", aop[0], None, B, N.ptr(b), B, 1, None, 0, 0, N.ptr(x), B, 1, None, 0, 0,
+               N.ptr(state), 1e-6, 200, 0, 0, 0, 0, N.stream_ptr(dev))
+
+    graph = torch.cuda.CUDAGraph()
+    solve()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        solve()
+    for rep in range(3):
+        b.copy_(torch.randn(n, B, generator=g))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = x.clone()
+        solve()
+        torch.cuda.synchronize()
+        assert torch.equal(got, x)
+        assert rel(x, torch.linalg.solve(A.double(), b.double())) < 2e-5  # cond <= 12: stopped at 1e-6
