@@ -8,6 +8,9 @@ to an engine kernel, otherwise step by step around ``A._matmat``) and reads
 the 8-byte control block once per chunk instead of syncing twice per step
 (cola/utils/torch_tqdm.py:42,88).
 """
+import collections
+import contextlib
+import threading
 import time
 from dataclasses import dataclass
 
@@ -116,6 +119,30 @@ def _fused_buffers(dev, n, B, max_iters):
     return bufs
 
 
+class _Workgroups:
+    """Bound on the workgroups of persistent solves in flight on one device.  Solves over several
+    workgroups wait for one another's words inside the kernel, so those of concurrent threads have to
+    fit the device together: one workgroup per CU, 256."""
+
+    def __init__(self, total=256):
+        self.total, self.used, self.changed = total, 0, threading.Condition()
+
+    @contextlib.contextmanager
+    def hold(self, count):
+        with self.changed:
+            self.changed.wait_for(lambda: self.used + count <= self.total)
+            self.used += count
+        try:
+            yield
+        finally:
+            with self.changed:
+                self.used -= count
+                self.changed.notify_all()
+
+
+_WORKGROUPS = collections.defaultdict(_Workgroups)
+
+
 def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin_limit=0, wait_offset=0,
                 cooperative=False):
     """cg.py:94-119 as one persistent launch (ck_cg_fused) when A lowers to a dense fp32
@@ -138,13 +165,15 @@ def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin
         x0f = x0.reshape(n, B)
         x0f = x0f if x0f.dtype == torch.float32 else x0f.float()
     t0 = time.time()
-    N.call("ck_cg_fused", aop[0], pop[0] if pop else None, B, N.ptr(bf), bf.stride(0), bf.stride(1), N.ptr(x0f),
-           x0f.stride(0) if x0f is not None else 0, x0f.stride(1) if x0f is not None else 0, N.ptr(x), x.stride(0),
-           x.stride(1), N.ptr(r), r.stride(0), r.stride(1), N.ptr(state), float(tol), int(max_iters), N.ptr(work),
-           work.numel() * 8, int(nblocks), int(spin_limit), int(wait_offset), int(bool(cooperative)),
-           N.stream_ptr(dev))
-    host.copy_(state, non_blocking=True)
-    torch.cuda.current_stream(dev).synchronize()
+    # 16 rows a workgroup or more, unless more workgroups are asked for
+    with _WORKGROUPS[dev.index].hold(min(256, max(-(-n // 16), nblocks))):
+        N.call("ck_cg_fused", aop[0], pop[0] if pop else None, B, N.ptr(bf), bf.stride(0), bf.stride(1), N.ptr(x0f),
+               x0f.stride(0) if x0f is not None else 0, x0f.stride(1) if x0f is not None else 0, N.ptr(x), x.stride(0),
+               x.stride(1), N.ptr(r), r.stride(0), r.stride(1), N.ptr(state), float(tol), int(max_iters), N.ptr(work),
+               work.numel() * 8, int(nblocks), int(spin_limit), int(wait_offset), int(bool(cooperative)),
+               N.stream_ptr(dev))
+        host.copy_(state, non_blocking=True)
+        torch.cuda.current_stream(dev).synchronize()
     ctrl = host[:N.CTRL_BYTES].view(torch.int32)
     k, status = int(ctrl[0]), int(ctrl[5])
     if status == N.CK_ERR_TIMEOUT:
@@ -186,7 +215,12 @@ def run_batched_cg(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, chunk=16, re
     if B > 1024:
         raise ValueError("at most 1024 right-hand sides per solve")
     if fused and not return_state:
-        out = fused_solve(A, b, x0, max_iters, tol, P)
+        try:
+            out = fused_solve(A, b, x0, max_iters, tol, P)
+        except N.KrylovError as e:  # other processes' kernels kept some workgroups off the device
+            if e.status != N.CK_ERR_TIMEOUT:
+                raise
+            out = None
         if out is not None:
             return out
     st = CGState(n, B, max_iters, b.device, P is not None)

@@ -301,18 +301,19 @@ int ck_cg_finish(int64_t n, int32_t nrhs, float* x, float* r, int64_t ld, const 
  * The whole batched CG solve of cola/linalg/inverse/cg.py:94-178 -- normalisation,
  * start, every step and the loop of cola/utils/torch_tqdm.py:86-90, un-normalisation --
  * in ONE cooperative launch (plus a one-block reset), for a dense fp32 operator
- * A = CK_OP_DENSE_F32 (y = scale*A x + shift*x) and P = NULL or CK_OP_DIAG_F32, 1 <= nrhs
- * <= 4, n*nrhs <= 7168 (and n <= 2560 for 3 or 4 columns): two n x nrhs fp32 vectors in LDS
- * and each thread's share of A p in registers.  Each workgroup keeps its rows of A in LDS
- * when they fit and the full r and p vectors; a step costs one grid-wide exchange: each
- * workgroup publishes its rows of A p as words tagged with the step, and every workgroup
+ * A = CK_OP_DENSE_F32 (y = scale*A x + shift*x) and P = NULL or CK_OP_DIAG_F32: n <= 3584
+ * for 1 to 4 columns (7168 for one), n <= 2048 for 5 to 8.  Each workgroup keeps its rows of A
+ * in registers (read again in every step above 3584) and the full r and p vectors in LDS; a
+ * step costs one grid-wide exchange: each workgroup publishes its rows of A p as words tagged
+ * with the step, and every workgroup
  * reads all of A p back.  b, x0 (optional) and x, r (r optional) are (n x nrhs) arrays with
  * element strides (row stride, column stride), i.e. the reference's layout directly.
  * state: ck_cg_state_bytes(nrhs, max_iters), laid out and filled as by the chained
  * entry points (k, done, status, errors[0..k], per-column scalars); work:
  * ck_cg_fused_workspace_bytes.  nblocks = 0 picks the workgroup count: one, with A in its
- * registers and no exchange, up to n = 320 (256 for 2 to 4 columns), else one per 8 rows (at
- * most 256).  Every grid-wide
+ * registers and no exchange, up to n = 320 (256 for 2 to 4 columns), else one per 16 rows (20
+ * above 3072, 28 above 3584).  Solves that overlap on one GPU have to fit it together, one
+ * workgroup per CU, or their waits may time out.  Every grid-wide
  * wait gives up after spin_limit polling rounds (<= 0: about a second), records
  * CK_ERR_TIMEOUT in ctrl.status and ends the kernel; wait_offset (0 in normal use) is
  * added to the tag each wait expects, so a host can make every wait time out and exercise
