@@ -60,7 +60,7 @@ class CkOp(ctypes.Structure):
 class CkBcgPlan(ctypes.Structure):
     """Mirror of ck_bcg_plan in include/cola_krylov.h (batched uneven systems)."""
     _fields_ = [("nsys", ctypes.c_int32), ("rows_per_tile", ctypes.c_int32), ("ntiles_mv", ctypes.c_int32),
-                ("ntiles_vec", ctypes.c_int32), ("max_iters", ctypes.c_int32), ("pad0", ctypes.c_int32)] + \
+                ("ntiles_vec", ctypes.c_int32), ("max_iters", ctypes.c_int32), ("max_vtiles", ctypes.c_int32)] + \
                [(name, ctypes.c_void_p) for name in
                 ("tile_sys", "tile_row0", "vtile_sys", "vtile_i0", "n", "lda", "voff", "moff", "mt_begin", "mt_end",
                  "vt_begin", "vt_end", "shift", "prec", "A32", "A16", "x", "r", "p", "Ap", "part_mv", "part_vec",

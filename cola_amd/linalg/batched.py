@@ -136,6 +136,7 @@ class BatchedCG:
         pl = N.CkBcgPlan()
         pl.nsys, pl.rows_per_tile, pl.ntiles_mv, pl.ntiles_vec = S, rows_per_tile, len(tsys), len(vsys)
         pl.max_iters = self.max_iters
+        pl.max_vtiles = int(np.max(np.asarray(vte) - np.asarray(vtb)))
         for name, tns in self.t.items():
             setattr(pl, name, tns.data_ptr())
         pl.shift, pl.prec = sy.shift.data_ptr(), self.prec.data_ptr()

@@ -631,7 +631,7 @@ typedef struct ck_bcg_plan {
   int32_t ntiles_mv;
   int32_t ntiles_vec;
   int32_t max_iters;
-  int32_t pad0;
+  int32_t max_vtiles; /* most vector tiles of one system (0: not given) */
   const int32_t* tile_sys;
   const int32_t* tile_row0;
   const int32_t* vtile_sys;
@@ -680,7 +680,8 @@ int32_t ck_bcg_vec_tile(void);
 /* x = 0, r = p = b for systems with done[s] == 0 on entry (others are left alone);
  * thresh = tol_rel * ||b_s|| + tol_abs; systems already below it are marked done. */
 int ck_bcg_start(const ck_bcg_plan* plan, const float* b, float tol_rel, float tol_abs, void* stream);
-/* `iters` CG iterations for every system not done (five launches each, no host sync).
+/* `iters` CG iterations for every system not done (two launches each where max_vtiles is 1 to 4 and
+ * rank is 0, else five; no host sync).
  * A system stops when ||r|| <= thresh or after max_iters iterations. */
 int ck_bcg_iterate(const ck_bcg_plan* plan, int32_t iters, void* stream);
 /* Ap = (K + shift I) p alone (tile-shape timing for the autotuner). */
