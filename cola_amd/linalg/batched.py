@@ -46,6 +46,9 @@ class BatchedSystems:
         self.voff = np.concatenate([[0], np.cumsum(vsz)[:-1]]).astype(np.int64)
         self.total_v = int(vsz.sum())
         self.total_m = int(msz.sum())
+        # where each entry of the concatenated systems sits in the padded layout
+        at = np.arange(int(self.sizes.sum())) + np.repeat(self.voff - (np.cumsum(self.sizes) - self.sizes), self.sizes)
+        self.entries = torch.tensor(at, device=self.device)
         self.A32 = torch.zeros(self.total_m, dtype=torch.float32, device=self.device)
         self.A16 = torch.zeros(self.total_m, dtype=torch.bfloat16, device=self.device) if bf16 else None
         self.shift = torch.tensor(np.asarray(shifts, dtype=np.float32).reshape(-1).repeat(
@@ -157,7 +160,8 @@ class BatchedCG:
         self.plan = pl
         self.stream = torch.cuda.Stream(device=dev)  # default priority; graphs need a non-legacy stream
         self.graphs = {}
-        self._pinned = torch.empty(S, dtype=torch.int32, pin_memory=True)
+        self._pinned = torch.empty((2, S), dtype=torch.int32, pin_memory=True)
+        self._events = [torch.cuda.Event(), torch.cuda.Event()]
 
     def set_precision(self, bf16_mask):
         """Per-system matvec storage: True reads the bf16 copy (needs systems built with bf16)."""
@@ -197,17 +201,28 @@ class BatchedCG:
             else:
                 self.done.copy_(torch.from_numpy((~np.asarray(active, dtype=bool)).astype(np.int32)))
             N.call("ck_bcg_start", ctypes.byref(self.plan), N.ptr(b), float(tol_rel), float(tol_abs), st)
-            steps = 0
-            while steps < self.max_iters:
-                n_it = min(int(chunk), self.max_iters - steps)
-                if use_graph:
-                    N.call("ck_graph_launch", self._graph(n_it), st)
-                else:
-                    N.call("ck_bcg_iterate", ctypes.byref(self.plan), n_it, st)
-                steps += n_it
-                self._pinned.copy_(self.done, non_blocking=True)
-                self.stream.synchronize()
-                if bool(self._pinned.all()):
+            steps, sent = 0, 0
+            waiting = []  # flags of chunks enqueued and not read: one chunk runs while the last one's are read
+            while True:
+                if steps < self.max_iters:
+                    n_it = min(int(chunk), self.max_iters - steps)
+                    if use_graph:
+                        N.call("ck_graph_launch", self._graph(n_it), st)
+                    else:
+                        N.call("ck_bcg_iterate", ctypes.byref(self.plan), n_it, st)
+                    steps += n_it
+                    flags, event = self._pinned[sent % 2], self._events[sent % 2]
+                    flags.copy_(self.done, non_blocking=True)
+                    event.record(self.stream)
+                    waiting.append((flags, event))
+                    sent += 1
+                    if len(waiting) < 2 and steps < self.max_iters:
+                        continue
+                if not waiting:
+                    break
+                flags, event = waiting.pop(0)
+                event.synchronize()
+                if bool(flags.all()):
                     break
             ks = self.k.cpu().numpy().copy()
         torch.cuda.current_stream(self.systems.device).wait_stream(self.stream)
@@ -474,13 +489,11 @@ class BatchedInverse(LinearOperator):
         sy = self.systems
         cols = []
         iters = []
-        sizes = sy.sizes.tolist()
-        bounds = np.concatenate([[0], np.cumsum(sizes)])
         for j in range(X.shape[1]):
-            col = X[:, j].to(torch.float32)
-            b = sy.concat([col[bounds[s]:bounds[s + 1]] for s in range(sy.nsys)])
+            b = torch.zeros(sy.total_v, dtype=torch.float32, device=sy.device)
+            b[sy.entries] = X[:, j].to(device=sy.device, dtype=torch.float32)
             x, ks = self.cg.solve(b, tol_rel=self.alg.tol, chunk=self.alg.chunk, use_graph=self.alg.use_graph)
-            cols.append(torch.cat(sy.split(x)).clone())
+            cols.append(x[sy.entries])
             iters.append(ks)
         self.info = {"iterations": np.stack(iters), "rows_per_tile": self.cg.rows, "autotune": self.tune}
         return torch.stack(cols, dim=1).to(X.dtype)
