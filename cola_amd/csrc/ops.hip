@@ -309,69 +309,79 @@ __global__ __launch_bounds__(256) void dense_bf16_kernel(int n, const uint16_t* 
   }
 }
 
-// Multi-rhs product of a bf16 matrix, the vector chunk staged in LDS as in dense_f32_lds_kernel.
-// Requires n % 8 == 0 and 16-byte aligned rows; lanes take 8 consecutive columns.
+// Multi-rhs product of a bf16 matrix, the vector chunk staged in LDS as in dense_f32_lds_kernel and
+// each piece of a row loaded again as soon as it is used.  Requires n % 8 == 0 and 16-byte aligned
+// rows; lanes take 8 consecutive columns, whose two halves of X lie 64 apart in LDS, so that 16
+// lanes read 256 contiguous bytes (side by side they met in the same banks two by two).  Bound by
+// HBM up to 4 rhs, by the VALU (9 instructions an entry) and the LDS reads at 8: 24576 x 4 / 8 / 16
+// 187 / 240 / 400 us, without the rolling loads and at 4 rows a wave (2 at 16) 225 / 265 / 450;
+// 5000 x 4 / 8 13.6 / 20 against 20 / 26; 16384 x 4 / 16 93 / 215 against 91 / 203.
+// v_mfma_f32_16x16x32_bf16 with x in three bf16 terms reads 4.2 TB/s where this does 5 to 6.5, takes
+// values below 1e-31 for zero and rounds its sums worse (4.9e-7 against 3.6e-7 at 24576).
 typedef float f32x2_nt __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4_nt __attribute__((ext_vector_type(4)));
 
 template <int NB, int ROWS>
-__global__ __launch_bounds__(64 * kDenseWaves) void dense_bf16_lds_kernel(int n, const uint16_t* __restrict__ A,
-                                                                          int64_t lda, const float* __restrict__ X,
-                                                                          int64_t ldx, float* __restrict__ Y,
-                                                                          int64_t ldy, int nbr, float scale,
-                                                                          float shift,
-                                                                          const int* __restrict__ done) {
+__global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_eu(4))) void dense_bf16_lds_kernel(
+    int n, const uint16_t* __restrict__ A, int64_t lda, const float* __restrict__ X, int64_t ldx,
+    float* __restrict__ Y, int64_t ldy, int nbr, float scale, float shift, const int* __restrict__ done) {
   if (done && *done) return;
-  __shared__ float4 xs[NB][kDenseChunk / 4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int Q = kDenseChunk / 512;                               // pieces of a row per lane and chunk
+  constexpr int XN = NB * (kDenseChunk / 4);                         // float4 of X per chunk
+  __shared__ float4 xs[NB][Q][2][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // rows and their pointers stay scalar
   const int row0 = blockIdx.x * (kDenseWaves * ROWS) + wave * ROWS;
+  const uint16_t* arow[ROWS];  // rows past the last: its copy, never stored
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) arow[r] = A + (int64_t)(row0 + r < n ? row0 + r : n - 1) * lda;
   float acc[ROWS][NB];
 #pragma unroll
   for (int r = 0; r < ROWS; ++r)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[r][b] = 0.f;
+  u32x4_nt a[Q][ROWS];
+  auto fetch_a = [&](int c0, int q) {
+    const int j = c0 + q * 512 + lane * 8, c = j < n ? j : n - 8;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) a[q][r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_nt*>(arow[r] + c));
+  };
+#pragma unroll
+  for (int q = 0; q < Q; ++q) fetch_a(0, q);
   for (int c0 = 0; c0 < n; c0 += kDenseChunk) {
-    const int cn = n - c0 < kDenseChunk ? n - c0 : kDenseChunk;  // multiple of 8
     __syncthreads();
-    for (int e = threadIdx.x; e < NB * (kDenseChunk / 4); e += 64 * kDenseWaves) {
-      const int b = e / (kDenseChunk / 4), j4 = e % (kDenseChunk / 4);
-      xs[b][j4] = (b < nbr && 4 * j4 < cn) ? *reinterpret_cast<const float4*>(X + (int64_t)b * ldx + c0 + 4 * j4)
-                                            : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int e0 = 0; e0 < XN; e0 += 64 * kDenseWaves) {
+      const int e = e0 + threadIdx.x, b = e / (kDenseChunk / 4), j4 = e % (kDenseChunk / 4);
+      if (XN % (64 * kDenseWaves) == 0 || e < XN)
+        xs[b][j4 / 128][j4 % 2][j4 / 2 % 64] = (b < nbr && c0 + 4 * j4 < n)
+                                                   ? *reinterpret_cast<const float4*>(X + (int64_t)b * ldx + c0 + 4 * j4)
+                                                   : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     __syncthreads();
+    const bool more = c0 + kDenseChunk < n;
 #pragma unroll
-    for (int q = 0; q < kDenseChunk / 512; ++q) {
-      const int j = q * 512 + lane * 8;
-      if (j < cn) {
-        uint4 w[ROWS];
-#pragma unroll
-        for (int r = 0; r < ROWS; ++r) {
-          if (row0 + r < n) {
-            const u32x4_nt v = __builtin_nontemporal_load(
-                reinterpret_cast<const u32x4_nt*>(A + (int64_t)(row0 + r) * lda + c0 + j));
-            w[r] = make_uint4(v.x, v.y, v.z, v.w);
-          } else {
-            w[r] = make_uint4(0u, 0u, 0u, 0u);
-          }
-        }
+    for (int q = 0; q < Q; ++q) {
+      if (c0 + q * 512 + lane * 8 < n) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-          const float4 x0 = xs[b][j / 4], x1 = xs[b][j / 4 + 1];
+          const float4 x0 = xs[b][q][0][lane], x1 = xs[b][q][1][lane];
 #pragma unroll
           for (int r = 0; r < ROWS; ++r) {
             float t = acc[r][b];
-            t = fmaf(__uint_as_float(w[r].x << 16), x0.x, t);
-            t = fmaf(__uint_as_float(w[r].x & 0xFFFF0000u), x0.y, t);
-            t = fmaf(__uint_as_float(w[r].y << 16), x0.z, t);
-            t = fmaf(__uint_as_float(w[r].y & 0xFFFF0000u), x0.w, t);
-            t = fmaf(__uint_as_float(w[r].z << 16), x1.x, t);
-            t = fmaf(__uint_as_float(w[r].z & 0xFFFF0000u), x1.y, t);
-            t = fmaf(__uint_as_float(w[r].w << 16), x1.z, t);
-            t = fmaf(__uint_as_float(w[r].w & 0xFFFF0000u), x1.w, t);
+            t = fmaf(bf16_lo(a[q][r][0]), x0.x, t);
+            t = fmaf(bf16_hi(a[q][r][0]), x0.y, t);
+            t = fmaf(bf16_lo(a[q][r][1]), x0.z, t);
+            t = fmaf(bf16_hi(a[q][r][1]), x0.w, t);
+            t = fmaf(bf16_lo(a[q][r][2]), x1.x, t);
+            t = fmaf(bf16_hi(a[q][r][2]), x1.y, t);
+            t = fmaf(bf16_lo(a[q][r][3]), x1.z, t);
+            t = fmaf(bf16_hi(a[q][r][3]), x1.w, t);
             acc[r][b] = t;
           }
         }
       }
+      if (more) fetch_a(c0 + kDenseChunk, q);
     }
   }
 #pragma unroll
@@ -751,16 +761,40 @@ int dense_dispatch(const ck_op* op, int nrhs, const float* X, int64_t ldx, float
 #define CK_DENSE_LAUNCH(NB_, ROWS_)                                                                              \
   hipLaunchKernelGGL((dense_bf16_kernel<NB_, ROWS_>), dim3((unsigned)cdiv(n, 4 * (ROWS_))), dim3(256), 0, s, n, A, \
                      op->lda, Xb, ldx, Yb, ldy, nb, op->scale, op->shift, done)
-    if (nb == 1)
+    // Rows per wave.  A round of resident blocks takes 16384 rows at 4 rows a wave (2 blocks a CU) and
+    // 12288 at 2 (3 blocks); the fewer rows' worth of rounds wins: 14336 x 8 84 us at 4 rows, 118 at 2;
+    // 18432 x 8 185 and 165.  One row where that fills the chip better: 8192 x 4 24 us, 31 at two rows.
+    auto rounds = [&](int64_t cap) { return cdiv(n, cap) * cap; };
+    const int rows = n <= (nb <= 4 ? 8192 : 2048) ? 1 : nb <= 8 && rounds(16384) < rounds(12288) ? 4 : 2;
+#define CK_DENSE_ROWS(NB_)  \
+  do {                      \
+    if (rows == 1)          \
+      CK_DENSE_LDS(NB_, 1); \
+    else if (rows == 2)     \
+      CK_DENSE_LDS(NB_, 2); \
+    else                    \
+      CK_DENSE_LDS(NB_, 4); \
+  } while (0)
+    // One and two rhs: straight from cache while the 256 MB last level holds the matrix (10000: 31 us, 33
+    // staged), staged above it (24576: 246 us, 187 staged).
+    const bool cached = 2 * (int64_t)n * op->lda <= (int64_t)256 << 20;
+    if (nb == 1 && cached)
       CK_DENSE_LAUNCH(1, 1);
-    else if (nb == 2)
+    else if (nb == 2 && cached)
       CK_DENSE_LAUNCH(2, 2);
+    else if (nb == 1)
+      CK_DENSE_LDS(1, 2);
+    else if (nb == 2)
+      CK_DENSE_LDS(2, 2);
     else if (nb <= 4)
-      CK_DENSE_LDS(4, 4);
+      CK_DENSE_ROWS(4);
     else if (nb <= 8)
-      CK_DENSE_LDS(8, 4);
+      CK_DENSE_ROWS(8);
+    else if (rows == 1)
+      CK_DENSE_LDS(16, 1);
     else
       CK_DENSE_LDS(16, 2);
+#undef CK_DENSE_ROWS
 #undef CK_DENSE_LDS
 #undef CK_DENSE_LAUNCH
   }
