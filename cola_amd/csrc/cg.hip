@@ -749,45 +749,57 @@ __global__ __launch_bounds__(256) void wbf_xr_kernel(int64_t n, int nrhs, const 
     const int b = o / 64, c = o % 64;
     if (c >= k) continue;
     const double t = (red[0][c][b] + red[1][c][b]) + (red[2][c][b] + red[3][c][b]);
-    ftr[((int64_t)b * k + c) * T + tile] = t;
+    ftr[((int64_t)b * T + tile) * k + c] = t;
   }
 }
 
-// u_b = C^-1 sum_tiles F^T r (tiles in index order within four fixed slices), one block per rhs
-__global__ __launch_bounds__(256) void wbf_core_kernel(int k, int nrhs, const double* __restrict__ ftr, int T,
-                                                       const double* __restrict__ Cinv, double* __restrict__ u,
-                                                       void* state) {
+// u_b = C^-1 sum_tiles F^T r, one block per rhs: wave w sums the tiles = w mod 16 (column = lane, so a
+// tile is one coalesced read and the wave's loads are in flight together), the waves' sums in order;
+// then lane (c, q) of a 64 x 16 grid takes four columns of row c of C^-1, loaded at the start.
+// Latency-bound: 128 tiles, rank 64, 8 rhs 4.6 us; with a lane per column walking its tiles and then a
+// row of C^-1 6.0.
+__global__ __launch_bounds__(1024) void wbf_core_kernel(int k, int nrhs, const double* __restrict__ ftr, int T,
+                                                        const double* __restrict__ Cinv, double* __restrict__ u,
+                                                        void* state) {
+  __shared__ double red[16][64];
+  __shared__ double ts[64];
+  const int b = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int cc = threadIdx.x >> 4, q = threadIdx.x & 15, c = lane < k ? lane : k - 1;
+  double ci[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {  // clamped addresses, masked where they are used
+    const int row = cc < k ? cc : k - 1, col = 4 * q + j < k ? 4 * q + j : k - 1;
+    ci[j] = Cinv[row * k + col];
+  }
+  const double* pc = ftr + (int64_t)b * T * k + c;
+  double acc = 0.0;
+  for (int t0 = wave; t0 < T; t0 += 16 * 8) {
+    double a[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) a[j] = pc[(int64_t)(t0 + 16 * j < T ? t0 + 16 * j : T - 1) * k];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc += t0 + 16 * j < T ? a[j] : 0.0;
+  }
+  // read after the loads are issued (they read valid memory either way)
   CgView v = view(state, nrhs);
   if (v.ctrl->done) return;
-  __shared__ double red[4][64];
-  __shared__ double ts[64];
-  const int b = blockIdx.x, c = threadIdx.x & 63, sl = threadIdx.x >> 6;
-  if (c < k) {
-    const int per = (T + 3) / 4;
-    const int t0 = sl * per, t1 = t0 + per < T ? t0 + per : T;
-    const double* pc = ftr + ((int64_t)b * k + c) * T;
-    double acc = 0.0;
-    int t = t0;
-    for (; t + 4 <= t1; t += 4) {
-      const double a0 = pc[t], a1 = pc[t + 1], a2 = pc[t + 2], a3 = pc[t + 3];
-      acc += a0;
-      acc += a1;
-      acc += a2;
-      acc += a3;
-    }
-    for (; t < t1; ++t) acc += pc[t];
-    red[sl][c] = acc;
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (wave == 0) {
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) t += red[w][lane];
+    ts[lane] = lane < k ? t : 0.0;
   }
   __syncthreads();
-  if (threadIdx.x < k)
-    ts[threadIdx.x] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
-  __syncthreads();
-  if (threadIdx.x < k) {
-    const int cc = threadIdx.x;
-    double acc = 0.0;
-    for (int j = 0; j < k; ++j) acc = fma(Cinv[cc * k + j], ts[j], acc);
-    u[(int64_t)b * k + cc] = acc;
-  }
+  double s = 0.0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) s = fma(4 * q + j < k ? ci[j] : 0.0, ts[4 * q + j], s);
+  s += dpp_f64<0xB1>(s);
+  s += dpp_f64<0x4E>(s);
+  s += dpp_f64<0x124>(s);
+  s += dpp_f64<0x128>(s);
+  if (q == 0 && cc < k) u[(int64_t)b * k + cc] = s;
 }
 
 // z = scale (r - F u) + shift r over the tile (F tile staged in LDS), r.z partials; the F
@@ -931,7 +943,7 @@ int cg_iterate(const ck_op* A, const ck_op* P, int32_t nrhs, float* x, float* r,
                          r, ld, (const float*)W.pap, W.npap, W.rr, F, P->lda, k, W.ftr, W.T, state);
       CK_CHECK_LAUNCH();
       if (last) break;
-      hipLaunchKernelGGL(wbf_core_kernel, dim3(nrhs), dim3(256), 0, s, k, (int)nrhs, (const double*)W.ftr, W.T,
+      hipLaunchKernelGGL(wbf_core_kernel, dim3(nrhs), dim3(1024), 0, s, k, (int)nrhs, (const double*)W.ftr, W.T,
                          reinterpret_cast<const double*>(P->aux), W.u, state);
       hipLaunchKernelGGL(wbf_z_kernel, dim3(W.T), dim3(256), 0, s, n, (int)nrhs, (const float*)r, z, ld, F, P->lda, k,
                          (const double*)W.u, (double)P->scale, (double)P->shift, W.rz, W.T, state);
