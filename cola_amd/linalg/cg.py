@@ -8,7 +8,6 @@ to an engine kernel, otherwise step by step around ``A._matmat``) and reads
 the 8-byte control block once per chunk instead of syncing twice per step
 (cola/utils/torch_tqdm.py:42,88).
 """
-import collections
 import contextlib
 import threading
 import time
@@ -140,7 +139,7 @@ class _Workgroups:
                 self.changed.notify_all()
 
 
-_WORKGROUPS = collections.defaultdict(_Workgroups)
+_WORKGROUPS = {}
 
 
 def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin_limit=0, wait_offset=0,
@@ -165,8 +164,10 @@ def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin
         x0f = x0.reshape(n, B)
         x0f = x0f if x0f.dtype == torch.float32 else x0f.float()
     t0 = time.time()
-    # 16 rows a workgroup or more, unless more workgroups are asked for
-    with _WORKGROUPS[dev.index].hold(min(256, max(-(-n // 16), nblocks))):
+    # 16 rows a workgroup or more, unless more workgroups are asked for; one needs no company
+    gate = _WORKGROUPS.get(dev.index) or _WORKGROUPS.setdefault(dev.index, _Workgroups())
+    alone = n <= 256 and B <= 4 and nblocks <= 1
+    with gate.hold(0 if alone else min(256, max(-(-n // 16), nblocks))):
         N.call("ck_cg_fused", aop[0], pop[0] if pop else None, B, N.ptr(bf), bf.stride(0), bf.stride(1), N.ptr(x0f),
                x0f.stride(0) if x0f is not None else 0, x0f.stride(1) if x0f is not None else 0, N.ptr(x), x.stride(0),
                x.stride(1), N.ptr(r), r.stride(0), r.stride(1), N.ptr(state), float(tol), int(max_iters), N.ptr(work),
