@@ -435,7 +435,7 @@ def bench_dense_cg(args, dev):
                        "cg_steps": int(k), "oracle_steps": int(io["iterations"] - 1), "fp64_rel_residual": res,
                        "chained_launch_solves_per_s": 1 / dtc, "chained_cg_steps": int(kc),
                        "solve_gpu_us": t_kernel * 1e6, "us_per_cg_step_gpu": t_kernel * 1e6 / max(int(k), 1)},
-            "roofline": {"bound": "hbm", "kernel": "fused_cg_kernel<true, 1> (whole solve, A rows held in LDS)",
+            "roofline": {"bound": "hbm", "kernel": "fused_cg_kernel<1, 4, 2, true> (whole solve, A rows held in registers)",
                          "achieved": ach, "peak": HBM_PEAK, "unit": "GB/s", "frac": ach / HBM_PEAK, "traffic": None,
                          "algorithmic_bytes_per_step": step_bytes,
                          "note": "latency-bound: one grid-wide exchange per step; A is read from LDS, not HBM"},
