@@ -41,6 +41,47 @@ def test_mlp_edges(dev, n, din, dout):
     assert rel(grad, ref) < 3e-6
 
 
+def _chain(acc, x, w):
+    """acc[i, j] + sum_k x[i, k] w[k, j] in fp32, k ascending, one fma a term (a product of two fp32 numbers
+    is exact in 64 bits)."""
+    acc = np.broadcast_to(acc, (x.shape[0], w.shape[1])).astype(np.float32)
+    for k in range(x.shape[1]):
+        acc = (acc.astype(np.float64) + x[:, k:k + 1].astype(np.float64) * w[k:k + 1].astype(np.float64)).astype(
+            np.float32)
+    return acc
+
+
+@pytest.mark.parametrize("n,din,dout", [(150, 5, 37), (64, 8, 64), (17, 1, 128)])
+def test_mlp_sums_in_index_order(dev, n, din, dout):
+    """Every sum starts from its bias and adds its terms in index order.  At arguments of 20 and more GELU is
+    the identity and its derivative one to the bit, so the whole pass can be restated exactly."""
+    rs = np.random.RandomState(n)
+    f = lambda *s: rs.randn(*s).astype(np.float32)  # noqa: E731
+    W1, W2, W3, b3 = 0.3 * f(din, 128), 0.05 * f(128, 128), f(128, dout), f(dout)
+    b1, b2 = 30 + f(128), 300 + f(128)
+    X, dG = rs.rand(n, din).astype(np.float32), f(n, dout)
+    net = PointMLP(din, dout, device=dev, params=np.concatenate([a.reshape(-1) for a in (W1, b1, W2, b2, W3, b3)]))
+    Xd = torch.from_numpy(X).to(dev)
+    G, Z1, Z2 = net.forward(Xd, save=True)
+    z1 = _chain(b1, X, W1)
+    z2 = _chain(b2, z1, W2)
+    assert z1.min() > 20 and z2.min() > 20
+    for got, want in ((Z1, z1), (Z2, z2), (G, _chain(b3, z2, W3))):
+        assert np.array_equal(got[:, :n].cpu().numpy().T, want)
+    d = torch.zeros(dout, G.shape[1])
+    d[:, :n] = torch.from_numpy(dG.T.copy())
+    grad = net.backward(Xd, Z1, Z2, d.to(dev), scale=1.0)
+    dz2 = _chain(np.float32(0), dG, W3.T)
+    dz1 = _chain(np.float32(0), dz2, W2.T)
+    total, zero, one = 0.0, np.float32(0), np.ones((1, n), np.float32)
+    for p in range(0, n, 64):  # a chunk's sums in fp32, the chunks' in fp64
+        c = slice(p, p + 64)
+        parts = [(X.T[:, c], dz1[c]), (one[:, c], dz1[c]), (z1.T[:, c], dz2[c]), (one[:, c], dz2[c]),
+                 (z2.T[:, c], dG[c]), (one[:, c], dG[c])]
+        total = total + np.concatenate([_chain(zero, a, b).astype(np.float64).reshape(-1) for a, b in parts])
+    assert np.array_equal(grad.cpu().numpy(), total.astype(np.float32))
+
+
 def test_mlp_row_major_output(dev):
     """Outputs and their gradient by rows, no saved pre-activations: the same numbers."""
     n, din, dout = 100, 4, 40
