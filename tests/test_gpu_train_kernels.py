@@ -129,6 +129,22 @@ def test_spd_inverse_orders(dev, k):
         assert torch.equal(inv32[b], inv[b].float()) and torch.equal(lT[b], linv[b].T.float())
 
 
+@pytest.mark.parametrize("scale,e", [(1.0, 100), (1e-291, 100), (1e291, 511)])
+def test_spd_inverse_divides(dev, scale, e):
+    """[[p, a], [a, 4^e]] with a^2 / p below half a unit of 4^e: the inverse factor's (1, 0) entry is -a / p
+    scaled by 2^-e, rounded once."""
+    rs, n = np.random.RandomState(5), 4096
+    p, a = scale * (1 + rs.rand(n)), scale * rs.rand(n)
+    A = np.zeros((n, 2, 2))
+    A[:, 0, 0], A[:, 1, 0], A[:, 1, 1] = p, a, 4.0**e
+    f64 = lambda: torch.empty(n, 2, 2, dtype=torch.float64, device=dev)  # noqa: E731
+    Ad, linv, st = torch.from_numpy(A).to(dev), f64(), torch.empty(n, dtype=torch.int32, device=dev)
+    N.call("ck_spd_inverse_f64", n, 2, N.ptr(Ad), 2, 4, 0.0, 0.0, N.ptr(linv), None, None, None, N.ptr(st),
+           N.stream_ptr(dev))
+    assert not st.any()
+    assert np.array_equal(linv[:, 1, 0].cpu().numpy(), -(a / p) * 2.0**-e)
+
+
 @pytest.mark.parametrize("k,bad", [(7, 0), (7, 3), (8, 7), (33, 32), (64, 41)])
 def test_spd_inverse_reports_the_failing_pivot(dev, k, bad):
     A = np.eye(k)
