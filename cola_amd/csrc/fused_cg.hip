@@ -19,8 +19,8 @@
 //
 // One workgroup, up to 320 unknowns (256 for two to four columns): wave w holds rows 4Qw on,
 // all columns (Q = 2 KC), entry j of x, r, p is thread j's, and a step has four barriers.
-// Bound by that serial chain: orders 64 / 150 / 300 and 256 x 4 columns take 1.3 / 1.5 / 1.9
-// and 3.2 us a step, over several workgroups 2.4 / 2.4 / 2.5 and 3.9.  At 300 x 2 to 4 columns
+// Bound by that serial chain: orders 64 / 150 / 300 and 256 x 4 columns take 1.3 / 1.6 / 1.9
+// and 3.8 us a step, over several workgroups 2.4 / 2.4 / 2.5 and 3.9.  At 300 x 2 to 4 columns
 // the matrix, 40 accumulators and the columns' vectors no longer fit 256 registers.
 //
 // Several workgroups, up to 3584 unknowns: a workgroup holds R <= 4Q rows, wave w the chunks
@@ -228,11 +228,7 @@ __device__ inline void load_rows(const FusedArgs& a, int row0, int row1, int wc,
 // acc += the wave's 4Q rows at four columns per b times p there; after all chunks `finish` hands the
 // sums over b to f(row, column, sum).  pk: the lane's column of p (lane & 3 of the first four) at its
 // four k; the next four columns LD * 4 further.
-// PIECES (one column): the four products of a chunk are added on their own first, so that a lane's sum
-// of 20 at 320 unknowns is one of five fours: with one chain the solutions at 300 unknowns erred by
-// 9.9e-7 in the mean of 20 systems, with pieces by 8.4e-7 (64 lanes a row: 7.9e-7), at 1.9 us a step
-// either way.
-template <int NB, int Q, int LD, bool PIECES = false>
+template <int NB, int Q, int LD>
 struct Acc {
   static constexpr int NG = NB == 1 ? 1 : NB / 4;
   float s[NB == 1 ? Q : 1];
@@ -244,15 +240,6 @@ struct Acc {
     for (f32x4& v : m) v = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   __device__ inline void add(const float (&av)[Q][4], const float* pk) {
-    if constexpr (PIECES) {
-      const f32x4 p4 = *reinterpret_cast<const f32x4*>(pk);
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        const float t = fmaf(av[q][1], p4[1], av[q][0] * p4[0]);
-        s[q] += fmaf(av[q][3], p4[3], fmaf(av[q][2], p4[2], t));
-      }
-      return;
-    }
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
       const f32x4 p4 = *reinterpret_cast<const f32x4*>(pk + 4 * g * LD);
@@ -432,9 +419,44 @@ __global__ __launch_bounds__(kNT) void fused_one_kernel(FusedArgs a) {
   float av[KC][Q][4];
   load_rows<Q, KC, 1>(a, 4 * Q * wave, n, 0, lane, av);
   auto product = [&]() {  // yv = A p for p in pv, all columns
-    Acc<NB, Q, LD, NB == 1 && (KC > 2)> acc;
+    Acc<NB, Q, LD> acc;
+    auto at = [&](int c) {
+      return *reinterpret_cast<const f32x4*>(pv + (NB > 1 ? lane & 3 : 0) * LD + 64 * c + 4 * (lane >> 2));
+    };
+    // A lane's sum (20 products at 320 unknowns) as a tree of chunks, those of one column in pairs, as if more
+    // lanes had shared the row.  The solutions' errors (means of 60 systems), as multiples of what 64 lanes a
+    // row give: 300 x 1 1.25 with one chain and 1.01 as a tree, 256 x 2 1.14 and 0.99, 256 x 4 1.20 and 1.02.
+    // A tree costs 0.05 to 0.1 us a step for one column, 0.7 at 256 x 4.
+    constexpr int K4 = KC < 4 ? KC : 4;
+    auto piece = [&](int c, int q, const f32x4& p) {
+      if constexpr (NB == 1) {
+        return fmaf(av[c][q][1], p[1], av[c][q][0] * p[0]) + fmaf(av[c][q][3], p[3], av[c][q][2] * p[2]);
+      } else {
+        f32x4 t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int c = 0; c < KC; ++c) acc.add(av[c], pv + (NB > 1 ? lane & 3 : 0) * LD + 64 * c + 4 * (lane >> 2));
+        for (int e = 0; e < 4; ++e) t = __builtin_amdgcn_mfma_f32_4x4x1f32(av[c][q][e], p[e], t, 0, 0, 0);
+        return t;
+      }
+    };
+    f32x4 p4[K4];
+#pragma unroll
+    for (int c = 0; c < K4; ++c) p4[c] = at(c);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      auto t = piece(0, q, p4[0]);
+      if constexpr (K4 > 1) t += piece(1, q, p4[1]);
+      if constexpr (K4 == 3) t += piece(2, q, p4[2]);
+      if constexpr (K4 == 4) t += piece(2, q, p4[2]) + piece(3, q, p4[3]);
+      if constexpr (NB == 1)
+        acc.s[q] = t;
+      else
+        acc.m[q] = t;
+    }
+    if constexpr (KC == 5) {  // one column only
+      const f32x4 p = at(4);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) acc.s[q] += piece(4, q, p);
+    }
     acc.finish(lane, [&](int row, int c, float s) { yv[c * NP + 4 * Q * wave + row] = s; });
   };
   float x[NB], r[NB], p[NB], z[NB];  // of column c < nrhs at entry tid < n, else zero
