@@ -102,7 +102,9 @@ _FUSED_BUFFERS = {}
 
 def _fused_buffers(dev, n, B, max_iters):
     """State, workspace and pinned host copy of the state for ck_cg_fused, kept per (device,
-    stream, shape): solves enqueued on one stream run in order, so they can share them."""
+    stream, shape), and their lock: solves enqueued on one stream run in order, so they can share
+    them, but threads may share a stream.  Whoever holds the lock owns all of them until the host
+    copy is read."""
     stream = torch.cuda.current_stream(dev).cuda_stream
     key = (dev.index, stream, n, B, int(max_iters))
     bufs = _FUSED_BUFFERS.get(key)
@@ -113,8 +115,8 @@ def _fused_buffers(dev, n, B, max_iters):
         wb = N.q("ck_cg_fused_workspace_bytes", n, B)
         bufs = (torch.empty(nbytes, dtype=torch.uint8, device=dev),
                 torch.empty((wb + 7) // 8, dtype=torch.float64, device=dev),
-                torch.empty(nbytes, dtype=torch.uint8, pin_memory=True), N.q("ck_cg_stride", B))
-        _FUSED_BUFFERS[key] = bufs
+                torch.empty(nbytes, dtype=torch.uint8, pin_memory=True), N.q("ck_cg_stride", B), threading.Lock())
+        bufs = _FUSED_BUFFERS.setdefault(key, bufs)
     return bufs
 
 
@@ -158,7 +160,7 @@ def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin
     bf = b if b.dtype == torch.float32 else b.float()
     xr = torch.empty((2, n, B), dtype=torch.float32, device=dev)
     x, r = xr[0], xr[1]
-    state, work, host, stride = _fused_buffers(dev, n, B, max_iters)
+    state, work, host, stride, lock = _fused_buffers(dev, n, B, max_iters)
     x0f = None
     if x0 is not None:
         x0f = x0.reshape(n, B)
@@ -167,7 +169,7 @@ def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin
     # 16 rows a workgroup or more, unless more workgroups are asked for; one needs no company
     gate = _WORKGROUPS.get(dev.index) or _WORKGROUPS.setdefault(dev.index, _Workgroups())
     alone = n <= 256 and B <= 4 and nblocks <= 1
-    with gate.hold(0 if alone else min(256, max(-(-n // 16), nblocks))):
+    with lock, gate.hold(0 if alone else min(256, max(-(-n // 16), nblocks))):
         N.call("ck_cg_fused", aop[0], pop[0] if pop else None, B, N.ptr(bf), bf.stride(0), bf.stride(1), N.ptr(x0f),
                x0f.stride(0) if x0f is not None else 0, x0f.stride(1) if x0f is not None else 0, N.ptr(x), x.stride(0),
                x.stride(1), N.ptr(r), r.stride(0), r.stride(1), N.ptr(state), float(tol), int(max_iters), N.ptr(work),
@@ -175,17 +177,17 @@ def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin
                N.stream_ptr(dev))
         host.copy_(state, non_blocking=True)
         torch.cuda.current_stream(dev).synchronize()
-    ctrl = host[:N.CTRL_BYTES].view(torch.int32)
-    k, status = int(ctrl[0]), int(ctrl[5])
-    if status == N.CK_ERR_TIMEOUT:
-        raise N.KrylovError("ck_cg_fused", status, "a grid-wide wait of the persistent CG timed out")
-    f = host[N.CTRL_BYTES:].view(torch.float32).numpy()
-    errs = f[N.CK_CG_ERRORS * stride:N.CK_CG_ERRORS * stride + k + 1].astype(np.float64)
-    rn = f[N.CK_CG_RNORM * stride:N.CK_CG_RNORM * stride + B]
-    tl = f[N.CK_CG_TOL * stride:N.CK_CG_TOL * stride + B]
+        ctrl = host[:N.CTRL_BYTES].view(torch.int32)
+        k, status = int(ctrl[0]), int(ctrl[5])
+        if status == N.CK_ERR_TIMEOUT:
+            raise N.KrylovError("ck_cg_fused", status, "a grid-wide wait of the persistent CG timed out")
+        f = host[N.CTRL_BYTES:].view(torch.float32).numpy()
+        errs = f[N.CK_CG_ERRORS * stride:N.CK_CG_ERRORS * stride + k + 1].astype(np.float64)
+        rn = f[N.CK_CG_RNORM * stride:N.CK_CG_RNORM * stride + B]
+        converged = bool((rn <= f[N.CK_CG_TOL * stride:N.CK_CG_TOL * stride + B]).all())
     elapsed = time.time() - t0
     info = {"iterations": k + 1, "errors": np.concatenate([errs, errs[-1:]])[2:], "iteration_time": elapsed / (k + 1),
-            "converged": bool((rn <= tl).all()), "status": _status_name(status), "fused": True}
+            "converged": converged, "status": _status_name(status), "fused": True}
     return x, r, k, info
 
 

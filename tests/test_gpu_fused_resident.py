@@ -84,3 +84,27 @@ def test_threads(dev):
         x, _, _, info = out[i]
         assert info["fused"] and info["status"] == "ok"
         assert rel(x, sol[:, 2 * i:2 * i + 2]) < 32 * (2e-6 + n * EPS)
+
+
+@pytest.mark.parametrize("n", [64, 600])
+def test_threads_on_the_default_stream(dev, n):
+    """Six threads on one stream, equal shapes, right-hand sides of 1 to 6 eigenvectors: each solve reports
+    its own steps (exactly as many in a diagonal system with that many distinct eigenvalues)."""
+    A = torch.diag(torch.linspace(1, 2, n, device=dev))
+    bs = torch.zeros(6, n, 1, device=dev)
+    for i in range(6):
+        bs[i, torch.arange(i + 1) * (n // 7)] = 1.0
+    torch.cuda.synchronize()
+    want = [run_batched_cg(ca.Dense(A), b, None, 100, 1e-5, None)[2] for b in bs]
+    assert want == sorted(set(want)) and want[0] == 1
+    got = {}
+
+    def work(i):
+        for _ in range(20):
+            x, _, k, info = run_batched_cg(ca.Dense(A), bs[i], None, 100, 1e-5, None)
+            got.setdefault(i, []).append((k, info["status"], rel(x, bs[i] / A.diagonal()[:, None]) < 1e-4))
+
+    ts = [threading.Thread(target=work, args=(i, )) for i in range(6)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert got == {i: [(want[i], "ok", True)] * 20 for i in range(6)}
