@@ -966,6 +966,12 @@ int ck_cg_fused_supported(const ck_op* A, const ck_op* P, int32_t nrhs) {
   return p.ok ? CK_OK : CK_ERR_UNSUPPORTED;
 }
 
+int32_t ck_cg_fused_workgroups(const ck_op* A, const ck_op* P, int32_t nrhs, int32_t nblocks, int32_t wait_offset) {
+  if (!fused_eligible(A, P, nrhs)) return 0;
+  const Plan p = make_plan(A->n, nrhs, nblocks);
+  return !p.ok ? 0 : one_workgroup(A->n, nrhs, nblocks, wait_offset) ? 1 : p.G;
+}
+
 int ck_cg_fused(const ck_op* A, const ck_op* P, int32_t nrhs, const float* b, int64_t b_rs, int64_t b_cs,
                 const float* x0, int64_t x0_rs, int64_t x0_cs, float* x, int64_t x_rs, int64_t x_cs, float* r,
                 int64_t r_rs, int64_t r_cs, void* state, float tol, int32_t max_iters, void* work,

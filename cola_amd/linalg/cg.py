@@ -121,11 +121,11 @@ def _fused_buffers(dev, n, B, max_iters):
 
 
 class _Workgroups:
-    """Bound on the workgroups of persistent solves in flight on one device.  Solves over several
-    workgroups wait for one another's words inside the kernel, so those of concurrent threads have to
-    fit the device together: one workgroup per CU, 256."""
+    """Bound on the workgroups of persistent solves in flight on one device.  The workgroups of a solve
+    wait for one another's words inside the kernel, so those of concurrent threads have to fit the
+    device together, one per CU."""
 
-    def __init__(self, total=256):
+    def __init__(self, total):
         self.total, self.used, self.changed = total, 0, threading.Condition()
 
     @contextlib.contextmanager
@@ -144,6 +144,14 @@ class _Workgroups:
 _WORKGROUPS = {}
 
 
+def _workgroups(dev):
+    gate = _WORKGROUPS.get(dev.index)
+    if gate is None:
+        cus = torch.cuda.get_device_properties(dev).multi_processor_count
+        gate = _WORKGROUPS.setdefault(dev.index, _Workgroups(cus))
+    return gate
+
+
 def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin_limit=0, wait_offset=0,
                 cooperative=False):
     """cg.py:94-119 as one persistent launch (ck_cg_fused) when A lowers to a dense fp32
@@ -154,9 +162,11 @@ def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin
     if aop is None or (P is not None and pop is None):
         return None
     n, B = b.shape
-    if N.q("ck_cg_fused_supported", aop[0], pop[0] if pop else None, B) != N.CK_OK:
-        return None
     dev = b.device
+    count = N.q("ck_cg_fused_workgroups", aop[0], pop[0] if pop else None, B, int(nblocks), int(wait_offset))
+    gate = _workgroups(dev)
+    if count == 0 or count > gate.total:
+        return None
     bf = b if b.dtype == torch.float32 else b.float()
     xr = torch.empty((2, n, B), dtype=torch.float32, device=dev)
     x, r = xr[0], xr[1]
@@ -166,10 +176,7 @@ def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin
         x0f = x0.reshape(n, B)
         x0f = x0f if x0f.dtype == torch.float32 else x0f.float()
     t0 = time.time()
-    # 16 rows a workgroup or more, unless more workgroups are asked for; one needs no company
-    gate = _WORKGROUPS.get(dev.index) or _WORKGROUPS.setdefault(dev.index, _Workgroups())
-    alone = n <= 256 and B <= 4 and nblocks <= 1
-    with lock, gate.hold(0 if alone else min(256, max(-(-n // 16), nblocks))):
+    with lock, gate.hold(count if count > 1 else 0):  # one workgroup needs no company
         N.call("ck_cg_fused", aop[0], pop[0] if pop else None, B, N.ptr(bf), bf.stride(0), bf.stride(1), N.ptr(x0f),
                x0f.stride(0) if x0f is not None else 0, x0f.stride(1) if x0f is not None else 0, N.ptr(x), x.stride(0),
                x.stride(1), N.ptr(r), r.stride(0), r.stride(1), N.ptr(state), float(tol), int(max_iters), N.ptr(work),
