@@ -176,14 +176,17 @@ def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin
         x0f = x0.reshape(n, B)
         x0f = x0f if x0f.dtype == torch.float32 else x0f.float()
     t0 = time.time()
-    with lock, gate.hold(count if count > 1 else 0):  # one workgroup needs no company
+    stream = torch.cuda.current_stream(dev)
+    if count > 1:  # one workgroup needs no company
+        stream.synchronize()  # what the stream still has to do is not done with workgroups held
+    with lock, gate.hold(count if count > 1 else 0):
         N.call("ck_cg_fused", aop[0], pop[0] if pop else None, B, N.ptr(bf), bf.stride(0), bf.stride(1), N.ptr(x0f),
                x0f.stride(0) if x0f is not None else 0, x0f.stride(1) if x0f is not None else 0, N.ptr(x), x.stride(0),
                x.stride(1), N.ptr(r), r.stride(0), r.stride(1), N.ptr(state), float(tol), int(max_iters), N.ptr(work),
                work.numel() * 8, int(nblocks), int(spin_limit), int(wait_offset), int(bool(cooperative)),
                N.stream_ptr(dev))
         host.copy_(state, non_blocking=True)
-        torch.cuda.current_stream(dev).synchronize()
+        stream.synchronize()
         ctrl = host[:N.CTRL_BYTES].view(torch.int32)
         k, status = int(ctrl[0]), int(ctrl[5])
         if status == N.CK_ERR_TIMEOUT:

@@ -15,6 +15,7 @@ cgmod = importlib.import_module("cola_amd.linalg.cg")  # the package exports a f
 
 ENGINE = {}  # the stub: workgroups of a solve, of all solves in flight, the most there were
 LOCK = threading.Lock()
+BACKLOG, SOLVING = {}, set()  # by thread: seconds of earlier work on its stream; those with a solve in flight
 
 
 def running(change):
@@ -30,8 +31,12 @@ class Stream:
         self.cuda_stream = threading.get_ident()
 
     def synchronize(self):
-        time.sleep(0.03)
-        running(-ENGINE["workgroups"])
+        me = threading.get_ident()
+        time.sleep(BACKLOG.pop(me, 0.0))
+        if me in SOLVING:
+            SOLVING.remove(me)
+            time.sleep(0.03)
+            running(-ENGINE["workgroups"])
 
 
 @pytest.fixture
@@ -44,6 +49,7 @@ def engine(monkeypatch):
         b = (ctypes.c_float * 2).from_address(a[3].value)
         ints = (ctypes.c_int32 * 16).from_address(a[15].value)
         ints[0], ints[5] = int(b[0]), int(b[1])
+        SOLVING.add(threading.get_ident())
         running(ENGINE["workgroups"])
 
     monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **k: empty(*a, **k).zero_())
@@ -94,6 +100,23 @@ def test_solves_in_flight_fit_the_device(engine, workgroups, cus, most):
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert ENGINE["most"] == most and cgmod._WORKGROUPS[None].used == 0
+
+
+def test_earlier_work_of_a_stream_holds_up_nobody(engine):
+    """A thread whose stream is busy for a second does not keep another's solve off the device meanwhile."""
+    ENGINE["workgroups"], b, done = 256, torch.ones(64, 1), {}
+
+    def work(name, backlog):
+        BACKLOG[threading.get_ident()] = backlog
+        cgmod.fused_solve(None, b, None, 100, 1e-6)
+        done[name] = time.monotonic()
+
+    t0, ts = time.monotonic(), [threading.Thread(target=work, args=a) for a in (("busy", 1.0), ("idle", 0.0))]
+    ts[0].start()
+    time.sleep(0.1)
+    ts[1].start()
+    [t.join() for t in ts]
+    assert done["idle"] - t0 < 0.7 and done["busy"] - t0 >= 1.0
 
 
 def test_more_workgroups_than_the_device_has(engine):
