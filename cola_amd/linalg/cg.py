@@ -220,20 +220,22 @@ class CGState:
 
 
 def run_batched_cg(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, chunk=16, return_state=False, fused=True):
-    """cg.py:94-119. b is (n, B) on the HIP device. Returns (x, r, k, info)."""
+    """cg.py:94-119. b is (n, B) on the HIP device. Returns (x, r, k, info); info["fused_timeout"] says that
+    a persistent launch gave up waiting first and chained launches took over."""
     N.require_device(b, "right-hand side")
     if b.dim() == 1:
         b = b[:, None]
     n, B = b.shape
     if B > 1024:
         raise ValueError("at most 1024 right-hand sides per solve")
+    timed_out = False
     if fused and not return_state:
         try:
             out = fused_solve(A, b, x0, max_iters, tol, P)
         except N.KrylovError as e:  # other processes' kernels kept some workgroups off the device
             if e.status != N.CK_ERR_TIMEOUT:
                 raise
-            out = None
+            out, timed_out = None, True
         if out is not None:
             return out
     st = CGState(n, B, max_iters, b.device, P is not None)
@@ -242,6 +244,8 @@ def run_batched_cg(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, chunk=16, re
     k, done, info = cg_blocks(A, Bb, st, x0b, max_iters, tol, P, chunk)
     x = from_blocks(st.x, n)
     r = from_blocks(st.r, n)
+    if timed_out:
+        info["fused_timeout"] = True
     if return_state:
         info["state"] = st
     return x, r, k, info

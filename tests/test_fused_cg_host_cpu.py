@@ -1,5 +1,5 @@
 """Host side of the persistent CG with the engine's launch replaced by a stub that writes the control block:
-buffers shared by threads, the bound on workgroups in flight."""
+buffers shared by threads, the bound on workgroups in flight, the way out of a time-out."""
 import ctypes
 import importlib
 import threading
@@ -123,6 +123,20 @@ def test_more_workgroups_than_the_device_has(engine):
     cgmod._WORKGROUPS[None] = cgmod._Workgroups(32)
     ENGINE["workgroups"] = 33
     assert cgmod.fused_solve(None, torch.ones(64, 1), None, 100, 1e-6) is None
+
+
+def test_timeout_falls_back_to_chained_launches(engine, monkeypatch):
+    b = torch.zeros(64, 1)
+    b[0], b[1] = 5, N.CK_ERR_TIMEOUT
+    monkeypatch.setattr(N, "require_device", lambda *a: None)
+    monkeypatch.setattr(cgmod, "to_blocks", lambda t, ld: t)
+    monkeypatch.setattr(cgmod, "from_blocks", lambda t, n: t)
+    monkeypatch.setattr(cgmod, "cg_blocks", lambda *a: (7, True, {"status": "ok", "fused": False}))
+    _, _, k, info = cgmod.run_batched_cg(None, b, None, 100, 1e-6)
+    assert k == 7 and info == {"status": "ok", "fused": False, "fused_timeout": True}
+    b[1] = N.CK_ERR_NAN  # any other status is the solve's own
+    _, _, k, info = cgmod.run_batched_cg(None, b, None, 100, 1e-6)
+    assert k == 5 and info["status"] == "nan" and "fused_timeout" not in info
 
 
 @pytest.mark.parametrize("n,B,nblocks,offset,count", [(256, 1, 0, 0, 1), (257, 1, 0, 0, 1), (320, 1, 0, 0, 1), (321, 1, 0, 0, 21),

@@ -3,6 +3,9 @@ oracle's restatement of cola's run_batched_cg (cg.py:94-178), against the chaine
 engine path on the same inputs, and its status codes and bounded grid-wide waits.
 Tolerances as in test_gpu_cg: FP32 iterates agree with the FP32 oracle to rounding, step
 counts within +-2 (reduction order)."""
+import functools
+import importlib
+
 import numpy as np
 import pytest
 import torch
@@ -110,6 +113,17 @@ def test_fused_wait_times_out_and_recovers(dev):
     assert e.value.status == N.CK_ERR_TIMEOUT
     x, r, k, info = fused_solve(op, b.to(dev), None, 500, 1e-6, None)
     assert info["status"] == "ok"
+    assert rel(x, torch.linalg.solve(A.double(), b.double())) < 2e-5
+
+
+def test_solve_after_a_timeout(dev, monkeypatch):
+    """run_batched_cg takes the chained launches where the persistent one gave up, and says so."""
+    mod = importlib.import_module("cola_amd.linalg.cg")
+    A, b = system(512, 256, 0.1, 2, 6)
+    gives_up = functools.partial(fused_solve, spin_limit=1000, wait_offset=1 << 30)
+    monkeypatch.setattr(mod, "fused_solve", gives_up)
+    x, r, k, info = run_batched_cg(ca.Dense(A.to(dev)), b.to(dev), None, 500, 1e-6, None)
+    assert info["status"] == "ok" and not info["fused"] and info["fused_timeout"]
     assert rel(x, torch.linalg.solve(A.double(), b.double())) < 2e-5
 
 
