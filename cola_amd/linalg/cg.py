@@ -123,25 +123,30 @@ def _fused_buffers(dev, n, B, max_iters):
 class _Workgroups:
     """Bound on the workgroups of persistent solves in flight on one device.  The workgroups of a solve
     wait for one another's words inside the kernel, so those of concurrent threads have to fit the
-    device together, one per CU."""
+    device together, one per CU.  A solve that finds no room waits for others' solves (0.1 to some ms
+    each), but not for whatever else their streams were given first: after 20 ms it goes without."""
+    PATIENCE = 0.02
 
     def __init__(self, total):
         self.total, self.used, self.changed = total, 0, threading.Condition()
 
     @contextlib.contextmanager
     def hold(self, count):
+        """Whether there was room: yields True with `count` workgroups held, else False."""
         with self.changed:
-            self.changed.wait_for(lambda: self.used + count <= self.total)
-            self.used += count
+            held = self.changed.wait_for(lambda: self.used + count <= self.total, self.PATIENCE)
+            self.used += count if held else 0
         try:
-            yield
+            yield held
         finally:
-            with self.changed:
-                self.used -= count
-                self.changed.notify_all()
+            if held:
+                with self.changed:
+                    self.used -= count
+                    self.changed.notify_all()
 
 
 _WORKGROUPS = {}
+_ALONE = contextlib.nullcontext(True)  # one workgroup waits for nobody
 
 
 def _workgroups(dev):
@@ -155,7 +160,8 @@ def _workgroups(dev):
 def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin_limit=0, wait_offset=0,
                 cooperative=False):
     """cg.py:94-119 as one persistent launch (ck_cg_fused) when A lowers to a dense fp32
-    operator and P is None or diagonal; returns (x, r, k, info) or None when unsupported.
+    operator and P is None or diagonal; returns (x, r, k, info), or None when unsupported or
+    when other threads' solves leave no room on the device.
     b (n, B) is read in place (any strides), x and r are written in the same layout."""
     aop = lower(A)
     pop = lower(P) if P is not None else None
@@ -177,9 +183,9 @@ def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin
         x0f = x0f if x0f.dtype == torch.float32 else x0f.float()
     t0 = time.time()
     stream = torch.cuda.current_stream(dev)
-    if count > 1:  # one workgroup needs no company
-        stream.synchronize()  # what the stream still has to do is not done with workgroups held
-    with lock, gate.hold(count if count > 1 else 0):
+    with lock, (gate.hold(count) if count > 1 else _ALONE) as held:
+        if not held:
+            return None
         N.call("ck_cg_fused", aop[0], pop[0] if pop else None, B, N.ptr(bf), bf.stride(0), bf.stride(1), N.ptr(x0f),
                x0f.stride(0) if x0f is not None else 0, x0f.stride(1) if x0f is not None else 0, N.ptr(x), x.stride(0),
                x.stride(1), N.ptr(r), r.stride(0), r.stride(1), N.ptr(state), float(tol), int(max_iters), N.ptr(work),

@@ -89,12 +89,13 @@ def test_solves_in_flight_fit_the_device(engine, workgroups, cus, most):
     """Eight threads with a stream each: as many solves at once as the device has CUs for; one workgroup
     waits for nobody and does not count."""
     cgmod._WORKGROUPS[None] = cgmod._Workgroups(cus)
+    cgmod._WORKGROUPS[None].PATIENCE = 5.0
     ENGINE["workgroups"] = workgroups
     b, start = torch.ones(64, 1), threading.Barrier(8)
 
     def work():
         start.wait()
-        cgmod.fused_solve(None, b, None, 100, 1e-6)
+        assert cgmod.fused_solve(None, b, None, 100, 1e-6) is not None
 
     ts = [threading.Thread(target=work) for _ in range(8)]
     [t.start() for t in ts]
@@ -103,20 +104,22 @@ def test_solves_in_flight_fit_the_device(engine, workgroups, cus, most):
 
 
 def test_earlier_work_of_a_stream_holds_up_nobody(engine):
-    """A thread whose stream is busy for a second does not keep another's solve off the device meanwhile."""
+    """A thread whose stream is busy for a second keeps the device's workgroups meanwhile: another's solve
+    is told so after a moment and can take the chained launches."""
     ENGINE["workgroups"], b, done = 256, torch.ones(64, 1), {}
 
     def work(name, backlog):
         BACKLOG[threading.get_ident()] = backlog
-        cgmod.fused_solve(None, b, None, 100, 1e-6)
-        done[name] = time.monotonic()
+        out = cgmod.fused_solve(None, b, None, 100, 1e-6)
+        done[name] = time.monotonic(), out is not None
 
     t0, ts = time.monotonic(), [threading.Thread(target=work, args=a) for a in (("busy", 1.0), ("idle", 0.0))]
     ts[0].start()
     time.sleep(0.1)
     ts[1].start()
     [t.join() for t in ts]
-    assert done["idle"] - t0 < 0.7 and done["busy"] - t0 >= 1.0
+    assert done["idle"][0] - t0 < 0.7 and not done["idle"][1]
+    assert done["busy"][0] - t0 >= 1.0 and done["busy"][1] and cgmod._WORKGROUPS[None].used == 0
 
 
 def test_more_workgroups_than_the_device_has(engine):
