@@ -902,17 +902,22 @@ __global__ __launch_bounds__(XY ? 1024 : 256) void csr_lane_per_row(int n, const
 
 // Longer rows: a group of G lanes per row (4, or 8 at eight rhs so that each rhs has a lane to store
 // it; a whole wave for rows of more than 128 entries on average).  Lane l of the group takes the
-// row's entries l, l + G, ... in order, U of them per batch: the batch's column indices and values go
+// row's entries l, l + G, ..., U of them per batch: the batch's column indices and values go
 // out together, then its gathers of x, so a row costs two dependent memory waits per G * U entries.
-// The lanes' sums are added in a fixed tree, whether or not xy_part is asked for.
+// A row of more than kCsrLong batches (a hub among short rows) is taken by the whole wave after its
+// other rows: 100 rows of 100000 entries among 400000 of 35 took 2400 / 4740 us at 1 / 4 rhs by their
+// groups, 3 to 5 times as long as one wave per row and rhs (684 / 3000); by their waves 411 / 680.
+// The sums are added in a fixed order, whether or not xy_part is asked for.
 // Bound by the gathers, which land on a cache line of their own where the columns are scattered:
 // with several rhs they come from a copy of x with the rhs fastest (csr_interleave, 4-5 us at
 // 300000 x 4), one NB-wide load and one line per entry instead of NB.  Measured, 300000 rows of 14.9
 // entries, a quarter of them anywhere (36 MB): 1 rhs 69 -> 16 us, 4 rhs 246 -> 32 us (57 without
-// the copy), 8 rhs 511 -> 56 us, against one lane per row; 50000 rows of 69 entries, against one
-// wave per row and rhs: 1 rhs 13.6 -> 12.8, 4 rhs 34 -> 21, 8 rhs 62 -> 31 us.  Short regular rows
+// the copy), 8 rhs 511 -> 56 us, against one lane per row; 50000 rows of 69 entries anywhere, against one
+// wave per row and rhs: 1 rhs 19.2 -> 16.9, 4 rhs 60 -> 27, 8 rhs 117 -> 36 us.  Short regular rows
 // (5-point Laplacian, 631000 rows) stay with one lane per row: 7.6 us against 14.6, 4 rhs 12.7
 // against 19.4.
+constexpr int kCsrLong = 8;  // batches of a group beyond which its wave takes the row
+
 template <int G>
 __device__ __forceinline__ float group_sum(float v) {
   if (G == 64) return wave_sum(v);
@@ -958,7 +963,7 @@ __global__ __launch_bounds__(256) void csr_group_kernel(int n, const int32_t* __
   constexpr int R = 256 / G;  // rows per sweep of the block
   constexpr int V = NB < 4 ? NB : 4;
   typedef float vec __attribute__((ext_vector_type(V)));
-  const int l = threadIdx.x % G, g = threadIdx.x / G;
+  const int l = threadIdx.x % G, g = threadIdx.x / G, lane = threadIdx.x & 63;
   const int row0 = blockIdx.x * rows;
   const bool stores = l < nbr;
   const int lb = stores ? l : 0;  // the rhs this lane stores
@@ -969,36 +974,85 @@ __global__ __launch_bounds__(256) void csr_group_kernel(int n, const int32_t* __
     const int rc = in ? row : n - 1;
     const int k0 = rowptr[rc], k1 = in ? rowptr[rc + 1] : k0;
     const float xr = X[(int64_t)lb * ldx + rc];
-    float acc[NB];
+    float acc[NB], odd[NB];
 #pragma unroll
-    for (int j = 0; j < NB; ++j) acc[j] = 0.f;
-    for (int kb = k0; kb < k1; kb += G * U) {
-      int c[U];
-      float v[U], x[U][NB];
+    for (int j = 0; j < NB; ++j) acc[j] = odd[j] = 0.f;
+    // the entries [a, b) from lane `at` of `width`: a batch's products are added on their own, in pairs, and
+    // the batches in two chains, so that a lane's sum of 16 or 32 entries errs no more than those of 64 lanes
+    auto add = [&](int a, int b, int at, int width) {
+      for (int kb = a; kb < b; kb += width * U) {
+        int c[U];
+        float v[U], x[U][NB];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {  // past the row's end: its last entry again, dropped below
-        const int k = kb + u * G + l, kk = k < k1 ? k : k1 - 1;
-        c[u] = colind[kk];
-        v[u] = val[kk];
-      }
+        for (int u = 0; u < U; ++u) {  // past the row's end: its last entry again, dropped below
+          const int k = kb + u * width + at, kk = k < b ? k : b - 1;
+          c[u] = colind[kk];
+          v[u] = val[kk];
+        }
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (NB == 1) {
-          x[u][0] = X[c[u]];
-        } else {
+        for (int u = 0; u < U; ++u) {
+          if (NB == 1) {
+            x[u][0] = X[c[u]];
+          } else {
 #pragma unroll
-          for (int q = 0; q < NB; q += V) {
-            const vec t = *reinterpret_cast<const vec*>(Xt + (int64_t)c[u] * NB + q);
+            for (int q = 0; q < NB; q += V) {
+              const vec t = *reinterpret_cast<const vec*>(Xt + (int64_t)c[u] * NB + q);
 #pragma unroll
-            for (int j = 0; j < V; ++j) x[u][q + j] = t[j];
+              for (int j = 0; j < V; ++j) x[u][q + j] = t[j];
+            }
           }
+        }
+        // used once, behind a select: the compiler would move the first loads into a branch of their own,
+        // another memory wait per batch
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          asm("" : "+v"(v[u]));
+          if (NB == 1) asm("" : "+v"(x[u][0]));
+        }
+        float t[U / 2][NB];
+#pragma unroll
+        for (int u = 0; u < U; u += 2) {
+          const bool on0 = kb + u * width + at < b, on1 = kb + (u + 1) * width + at < b;
+#pragma unroll
+          for (int j = 0; j < NB; ++j) {
+            const float p = on0 ? v[u] * x[u][j] : 0.f;
+            t[u / 2][j] = on1 ? fmaf(v[u + 1], x[u + 1][j], p) : p;
+          }
+        }
+#pragma unroll
+        for (int w = U / 4; w >= 1; w /= 2)
+#pragma unroll
+          for (int u = 0; u < w; ++u)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) t[u][j] += t[u + w][j];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const float s = odd[j] + t[0][j];
+          odd[j] = acc[j];
+          acc[j] = s;
         }
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const bool on = kb + u * G + l < k1;
+      for (int j = 0; j < NB; ++j) acc[j] += odd[j];
+    };
+    const bool over = G < 64 && k1 - k0 > kCsrLong * G * U;
+    add(k0, over ? k0 : k1, l, G);
+    if (G < 64) {  // rows far longer than the others: one at a time by the whole wave
+      for (uint64_t left = __ballot(over); left != 0;) {
+        const int first = __builtin_ctzll(left);  // lane 0 of a group
+        float keep[NB];
 #pragma unroll
-        for (int j = 0; j < NB; ++j) acc[j] = on ? fmaf(v[u], x[u][j], acc[j]) : acc[j];
+        for (int j = 0; j < NB; ++j) {
+          keep[j] = acc[j];
+          acc[j] = odd[j] = 0.f;
+        }
+        add(__builtin_amdgcn_readlane(k0, first), __builtin_amdgcn_readlane(k1, first), lane, 64);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const float s = wave_sum(acc[j]);
+          acc[j] = lane == first ? s : keep[j];
+        }
+        left &= ~(((1ull << (G % 64)) - 1) << first);
       }
     }
     float mine = 0.f;
@@ -1056,8 +1110,12 @@ int csr_launch(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y,
     CK_CHECK_LAUNCH();
     return CK_OK;
   }
-  const int rows = csr_rows(op);
-  const dim3 grid((unsigned)csr_xy_nparts(op)), blk(256);
+  // One rhs and more than 64 entries a row: 16 lanes a row, one sweep a block (the partials' bound on blocks
+  // has no say without partials): 200000 rows of 69 61 us, 73 with 4 lanes, 68 with a wave a row;
+  // 150000 of 120 78, 89 and 80.
+  const bool wide = nrhs == 1 && !xy_part && !csr_long_rows(op) && (double)op->nnz > 64.0 * (double)n;
+  const int rows = wide ? 16 : csr_rows(op);
+  const dim3 grid(wide ? (unsigned)cdiv(n, rows) : (unsigned)csr_xy_nparts(op)), blk(256);
   // the interleaved x sits past the partials; without room for it the rhs go one at a time
   const size_t off = csr_xy_bytes(op, nrhs);
   const bool room = work && work_bytes >= off + csr_xt_bytes(n, nrhs);
@@ -1085,7 +1143,9 @@ int csr_launch(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y,
       else
         CK_CSR(64, 8, 2);
     } else {
-      if (step == 1)
+      if (wide)
+        CK_CSR(16, 1, 8);
+      else if (step == 1)
         CK_CSR(4, 1, 8);
       else if (step == 2)
         CK_CSR(4, 2, 4);

@@ -27,7 +27,7 @@ def matrix(n, avg, seed):
     return scipy.sparse.csr_matrix((vals, (rows, cols)), (n, n))
 
 
-@pytest.mark.parametrize("n,avg", [(65, 14), (700, 5), (700, 12), (700, 40), (301, 230), (5000, 11)])
+@pytest.mark.parametrize("n,avg", [(65, 14), (700, 5), (700, 12), (700, 40), (700, 90), (301, 230), (5000, 11)])
 @pytest.mark.parametrize("nrhs", [1, 2, 3, 5, 8, 11])
 @pytest.mark.parametrize("room", [True, False])
 def test_csr_group_product(dev, n, avg, nrhs, room):
@@ -49,6 +49,71 @@ def test_csr_group_product(dev, n, avg, nrhs, room):
     err = np.abs(Yb[:, :n].T.double().cpu().numpy() - ref)
     depth = np.diff(M.indptr)[:, None] + 8  # roundings of a row's sum
     assert (err <= 6e-8 * depth * mag + 1e-30).all()
+
+
+def hubs(n, avg, length, seed):
+    """Rows of about avg entries, three of them `length` long: first, last and in the middle of a wave's."""
+    rs = np.random.RandomState(seed)
+    lens = np.maximum(rs.poisson(avg, n), 1)
+    lens[[0, n // 2 + 5, n - 1]] = length
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    cols = rs.randint(0, n, ptr[-1]).astype(np.int32)  # several entries may share a column
+    return scipy.sparse.csr_matrix((rs.randn(ptr[-1]).astype(np.float32), cols, ptr), (n, n)), ptr, cols
+
+
+@pytest.mark.parametrize("n,avg,length", [(1001, 12, 127), (1001, 12, 129), (1001, 12, 257), (1001, 40, 300), (640, 12, 20001),
+                                          (1001, 100, 1025)])
+@pytest.mark.parametrize("nrhs", [1, 2, 4, 7])
+def test_csr_hub_rows(dev, n, avg, length, nrhs):
+    """Rows far longer than the average, with and without the x . Ax partials: right, and rounded like sums
+    shared by a wave.  A lane adds length / 64 products, in pairs and batches; random signs let the errors
+    of a sum grow like the root of its additions, so 2 sqrt(length / 64 + 8) units of sqrt(sum v^2 x^2)."""
+    M, ptr, cols = hubs(n, avg, length, length)
+    A = ca.Sparse.from_csr(*(torch.from_numpy(a).to(dev) for a in (ptr, cols, M.data)), (n, n))
+    X = torch.from_numpy(np.random.RandomState(nrhs).randn(n, nrhs).astype(np.float32)).to(dev)
+    X64 = X.double().cpu().numpy()
+    M64 = M.astype(np.float64)
+    err = (A @ X).double().cpu().numpy() - M64 @ X64
+    size = np.sqrt(M64.multiply(M64) @ X64**2)
+    for row in (0, n // 2 + 5, n - 1):
+        assert (np.abs(err[row]) <= 6e-8 * 2 * np.sqrt(length / 64 + 8) * size[row]).all()
+    assert (np.abs(err) <= 6e-8 * 12 * size).all() or length > 2000
+    S = scipy.sparse.diags(np.asarray(abs(M64).sum(1)).ravel() + np.asarray(abs(M64).sum(0)).ravel() + 1.0) - (
+        abs(M64) + abs(M64).T)
+    S = S.tocsr().astype(np.float32)  # CG takes p . Ap from the product
+    As = ca.Sparse.from_csr(*(torch.from_numpy(a).to(dev) for a in (S.indptr, S.indices, S.data)), (n, n))
+    x = inv(ca.PSD(As), HipCG(tol=1e-6, max_iters=400)) @ X
+    res = S.astype(np.float64) @ x.double().cpu().numpy() - X64
+    assert (np.linalg.norm(res, axis=0) <= 4e-6 * np.linalg.norm(X64, axis=0)).all()
+
+
+@pytest.mark.parametrize("avg,nrhs", [(40, 1), (90, 1), (120, 1), (120, 3), (120, 8)])
+def test_csr_rounds_like_a_wave_a_row(dev, avg, nrhs):
+    """The error of a whole product against that of 64 sums a row added as a tree (the mean over 20000 rows;
+    its spread over matrices is below 1 %).  A lane's plain chain gives 1.03 to 1.45."""
+    n, rs = 20000, np.random.RandomState(avg)
+    M, ptr, cols = hubs(n, avg, avg, avg)
+    A = ca.Sparse.from_csr(*(torch.from_numpy(a).to(dev) for a in (ptr, cols, M.data)), (n, n))
+    X = rs.randn(n, nrhs).astype(np.float32)
+    ref = M.astype(np.float64) @ X.astype(np.float64)
+    err = lambda Y: np.linalg.norm(Y - ref)  # noqa: E731
+    length = np.diff(ptr)
+    k = np.arange(192)
+    at = np.minimum(ptr[:-1, None] + k, ptr[1:, None] - 1)
+    v = np.where(k < length[:, None], M.data[at], 0).astype(np.float64)
+    assert length.max() <= 192
+    ours = (A @ torch.from_numpy(X).to(dev)).double().cpu().numpy()
+    wave = np.empty((n, nrhs))
+    for b in range(nrhs):
+        x = X[cols[at], b].astype(np.float64)
+        s = np.zeros((n, 64), np.float32)
+        for c in range(3):
+            s = (s + v[:, 64 * c:64 * c + 64] * x[:, 64 * c:64 * c + 64]).astype(np.float32)
+        while s.shape[1] > 1:
+            s = s[:, ::2] + s[:, 1::2]
+        wave[:, b] = s[:, 0]
+    print(avg, nrhs, err(ours) / err(wave), flush=True)
+    assert err(ours) < 1.025 * err(wave)
 
 
 def test_csr_group_ignores_other_columns_nonfinite(dev):
