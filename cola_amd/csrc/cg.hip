@@ -418,6 +418,10 @@ __global__ __launch_bounds__(256) void step_final_kernel(int nrhs, const float* 
 // already sees it set leaves p alone, which nothing reads once the loop has ended.
 // Latency bound: the two launches took 4.4 + 5.5 us of a step at 144000 x 8, 3.3 + 2.4 us at
 // 2500 x 4 and 4.6 + 4.9 us at 16384 x 8; joined, a step is 3.0, 4.0 and 2.5 us shorter.
+// Above kWavePartials the waves of a block share the partials: by themselves they read 16 KB of them at
+// n = 4 M for 12 KB of vectors.  Steps on a diagonal operator, two launches / joined by wave / by block:
+// 144000 x 1 15.0 / 12.4 / 12.8 us, 1 M x 8 81 / 79 / 78, 4 M x 8 310 / 314 / 301, 8 M x 1 75.7 / 75.1 / 72.6.
+constexpr int kWavePartials = 128;  // n = 524288
 template <bool V4, bool JOINED>
 __global__ __launch_bounds__(256) void update_p_kernel(int64_t n, const float* __restrict__ z, float* __restrict__ p,
                                                        int64_t ld, const float* __restrict__ part1,
@@ -445,7 +449,9 @@ __global__ __launch_bounds__(256) void update_p_kernel(int64_t n, const float* _
   float beta;
   if (JOINED) {
     const float den = step_den(v, nrhs)[b];
-    const double rz = column_total(precond ? part2 : part1, P, b);
+    __shared__ double dred[4];
+    const float* part = precond ? part2 : part1;
+    const double rz = P > kWavePartials ? column_total_block(part, P, b, dred) : column_total(part, P, b);
     beta = den == INFINITY ? 0.f : (float)safe_div(rz, (double)den);
   } else {
     beta = v.beta[b];

@@ -185,3 +185,21 @@ def test_scalar_shift_updated_in_place_between_solves(dev):
         x = inv(op, HipCG(tol=1e-7, max_iters=1000)) @ b.to(dev)
         xd = torch.linalg.solve(K.double() + value * torch.eye(n, dtype=torch.float64), b.double())
         assert rel(x, xd) < 2e-5, value
+
+
+@pytest.mark.parametrize("n,B", [(524288, 2), (524289, 2), (600000, 32), (600000, 33), (4500000, 1), (4500002, 2),
+                                 (4500003, 1), (2500, 32), (2501, 33)])
+@pytest.mark.parametrize("pre", [False, True])
+def test_cg_step_end_at_many_partials(dev, n, B, pre):
+    """The end of a step at the edges of its forms: up to 128 partials a wave totals them, above a block; up
+    to 32 columns it rides in the p update; above 4096 x 1024 entries a block's share is read in a loop.  A
+    diagonal of three values takes three steps, of fp32 sums of at most 5e6 terms in tiles of 4096 or 4395."""
+    g = torch.Generator(device=dev).manual_seed(B)
+    d = torch.randint(1, 4, (n, ), generator=g, device=dev).float()
+    b = torch.randn(n, B, generator=g, device=dev)
+    P = ca.Diagonal(torch.where(d < 3, 1.0, 2.0)) if pre else None  # P A: 1, 2 and 6
+    x, r, k, info = run_batched_cg(ca.Diagonal(d), b, None, 20, 1e-5, P)
+    assert k in (3, 4) and info["status"] == "ok"
+    err = (x * d[:, None] - b).norm(dim=0) / b.norm(dim=0)
+    assert float(err.max()) < 2e-5 + 5e-6
+    assert float((b - x * d[:, None] - r).norm() / b.norm()) < 5e-6
