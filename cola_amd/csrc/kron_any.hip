@@ -125,6 +125,9 @@ __global__ __launch_bounds__(256) void kron_any_pass_a(int slabs, int per, int n
 #pragma unroll
           for (int r = 0; r < C2; ++r) T[r] = mfma(a[r][e], k[e], T[r]);
       }
+      // rows past n2 are 0 times K3: zero for the second product also where K3 is not finite
+#pragma unroll
+      for (int q = 0; q < 4; ++q) T[C2 - 1][q] = 16 * (C2 - 1) + 4 * g + q < n2 ? T[C2 - 1][q] : 0.f;
       const float* p2 = L2 + li * kPitch + 4 * g;
 #pragma unroll
       for (int c = 0; c < C2; ++c) {

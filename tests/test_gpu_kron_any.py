@@ -57,6 +57,22 @@ def test_kron_any_product(dev, dims, nrhs):
     assert bool((Yb[:, n:] == -7.0).all())
 
 
+@pytest.mark.parametrize("dims,factor", [(d, f) for d in ((3, 20, 17), (20, 5, 4), (4, 3, 50), (33, 64, 20), (20, 7), (1, 60))
+                                         for f in range(len(d))])
+def test_kron_any_infinite_entry(dev, dims, factor):
+    """One infinite entry of a factor, everything else positive: infinite where it enters, finite elsewhere
+    (the padding to 16 is zeros times the other operand, whatever that holds)."""
+    g = torch.Generator().manual_seed(sum(dims))
+    fs = [torch.rand(d, d, generator=g) + 0.1 for d in dims]
+    at = dims[factor] - 1
+    fs[factor][at, 0] = float("inf")
+    X = torch.rand(torch.Size(dims).numel(), 2, generator=g) + 0.1
+    Y = (ca.Kronecker(*[ca.Dense(f.to(dev)) for f in fs]) @ X.to(dev)).cpu().reshape(*dims, 2)
+    hit = torch.zeros(*dims, 2, dtype=torch.bool)
+    hit.select(factor, at).fill_(True)
+    assert bool((torch.isposinf(Y) == hit).all()) and bool((torch.isfinite(Y) == ~hit).all())
+
+
 def test_kron_any_many_slabs(dev):
     """Enough slabs that a block walks several of them, the last block fewer."""
     dims, nrhs = (63, 18, 20), 53
