@@ -14,6 +14,8 @@
 //     (a workspace holds one partial per column slice, added in slice order).
 // Measured, 20000 points in 3-D, Matern 5/2, 4 rhs: 4242 us with one row per lane, 79 blocks and
 // the library's expf and sqrtf; now 210 us per call (the transposes and the host included).
+#include <type_traits>
+
 #include "common.hpp"
 #include "ops_internal.hpp"
 
@@ -21,6 +23,7 @@ using namespace ck;
 
 namespace {
 
+constexpr int kRbfCols = 4;     // columns at a time
 constexpr int kRbfTile = 256;   // columns staged per step
 constexpr int kRbfRows = 128;   // rows per block: two per lane
 constexpr int kRbfMaxDim = 8;
@@ -45,13 +48,25 @@ __device__ __forceinline__ float stationary(float d2, float ce, float ca) {
   return fmaf(a, fmaf(a, 1.f / 3.f, 1.f), 1.f) * e;
 }
 
+// The same where v_exp_f32 would return zero for a subnormal, or v_sqrt_f32 take one for zero.
+template <int FAMILY>
+__device__ __forceinline__ float stationary_far(float d2, float ce, float ca) {
+  const float r = FAMILY == 0 ? d2 : sqrtf(d2), arg = ce * r, a = ca * r;
+  const bool far = arg < -126.f;
+  const float e = __builtin_amdgcn_exp2f(far ? arg + 64.f : arg);
+  const float f = FAMILY == 0 || FAMILY == 1 ? e
+                  : FAMILY == 2              ? fmaf(a, e, e)
+                                             : fmaf(a, fmaf(a, 1.f / 3.f, 1.f), 1.f) * e;
+  return far ? f * 0x1p-64f : f;
+}
+
 // Column slice blockIdx.y of the rows 128 blockIdx.x ..: the finished rows when there is one slice
 // (part == nullptr), else part[(slice * NB + b) * n + row].
 template <int FAMILY, int DIM, int NB>
 __global__ __launch_bounds__(256) void rbf_kernel(int n, int dim, const float* __restrict__ P, int64_t ldp, float ce,
                                                   float ca, const float* __restrict__ X, int64_t ldx,
                                                   float* __restrict__ Y, int64_t ldy, int nbr, float scale,
-                                                  float shift, float* __restrict__ part,
+                                                  float shift, float far2, float* __restrict__ part,
                                                   const int* __restrict__ done) {
   if (done && *done) return;
   constexpr int W = (DIM + NB + 3) / 4 * 4;  // floats per staged column: its point, then its x
@@ -93,31 +108,53 @@ __global__ __launch_bounds__(256) void rbf_kernel(int n, int dim, const float* _
     const int left = n - t * kRbfTile - wave * 64;
     const int jn = left < 64 ? left : 64;
     const float4* col = tile + wave * 64 * (W / 4);
-#pragma unroll 4
-    for (int jj = 0; jj < jn; ++jj) {
-      float c[W];
+    // K columns from jj on; entries whose kernel value is subnormal go the long way, all K together
+    auto columns = [&](int jj, auto count) {
+      constexpr int K = decltype(count)::value;
+      float c[K][W], d0[K], d1[K], most = 0.f;
 #pragma unroll
-      for (int q = 0; q < W / 4; ++q) {
-        const float4 v = col[jj * (W / 4) + q];
-        c[4 * q] = v.x;
-        c[4 * q + 1] = v.y;
-        c[4 * q + 2] = v.z;
-        c[4 * q + 3] = v.w;
-      }
-      float d0 = 0.f, d1 = 0.f;
+      for (int k = 0; k < K; ++k) {
 #pragma unroll
-      for (int d = 0; d < DIM; ++d) {
-        const float e0 = p0[d] - c[d], e1 = p1[d] - c[d];
-        d0 = fmaf(e0, e0, d0);
-        d1 = fmaf(e1, e1, d1);
-      }
-      const float k0 = stationary<FAMILY>(d0, ce, ca), k1 = stationary<FAMILY>(d1, ce, ca);
+        for (int q = 0; q < W / 4; ++q) {
+          const float4 v = col[(jj + k) * (W / 4) + q];
+          c[k][4 * q] = v.x;
+          c[k][4 * q + 1] = v.y;
+          c[k][4 * q + 2] = v.z;
+          c[k][4 * q + 3] = v.w;
+        }
+        d0[k] = d1[k] = 0.f;
 #pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        acc0[b] = fmaf(k0, c[DIM + b], acc0[b]);
-        acc1[b] = fmaf(k1, c[DIM + b], acc1[b]);
+        for (int d = 0; d < DIM; ++d) {
+          const float e0 = p0[d] - c[k][d], e1 = p1[d] - c[k][d];
+          d0[k] = fmaf(e0, e0, d0[k]);
+          d1[k] = fmaf(e1, e1, d1[k]);
+        }
+        most = fmaxf(most, fmaxf(d0[k], d1[k]));
       }
-    }
+      if (__any(most > far2)) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          d0[k] = stationary_far<FAMILY>(d0[k], ce, ca);
+          d1[k] = stationary_far<FAMILY>(d1[k], ce, ca);
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          d0[k] = stationary<FAMILY>(d0[k], ce, ca);
+          d1[k] = stationary<FAMILY>(d1[k], ce, ca);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          acc0[b] = fmaf(d0[k], c[k][DIM + b], acc0[b]);
+          acc1[b] = fmaf(d1[k], c[k][DIM + b], acc1[b]);
+        }
+    };
+    int jj = 0;
+    for (; jj + kRbfCols <= jn; jj += kRbfCols) columns(jj, std::integral_constant<int, kRbfCols>());
+    for (; jj < jn; ++jj) columns(jj, std::integral_constant<int, 1>());
   }
   if (wave > 0) {
 #pragma unroll
@@ -176,11 +213,11 @@ inline int rbf_slices(int64_t n) {
 
 template <int FAMILY, int DIM>
 void rbf_launch(int nb_t, dim3 grid, hipStream_t s, int n, int dim, const float* P, int64_t ldp, float ce, float ca,
-                const float* X, int64_t ldx, float* Y, int64_t ldy, int nbr, float scale, float shift, float* part,
-                const int* done) {
+                const float* X, int64_t ldx, float* Y, int64_t ldy, int nbr, float scale, float shift, float far2,
+                float* part, const int* done) {
 #define CK_RBF(NB_)                                                                                                  \
   hipLaunchKernelGGL((rbf_kernel<FAMILY, DIM, NB_>), grid, dim3(256), 0, s, n, dim, P, ldp, ce, ca, X, ldx, Y, ldy, \
-                     nbr, scale, shift, part, done)
+                     nbr, scale, shift, far2, part, done)
   switch (nb_t) {
     case 1: CK_RBF(1); break;
     case 2: CK_RBF(2); break;
@@ -225,6 +262,9 @@ int rbf_apply(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, 
   const double l = (double)op->aux_f, log2e = 1.4426950408889634;
   const double root = fam == 2 ? sqrt(3.0) : fam == 3 ? sqrt(5.0) : 1.0;
   const float ce = (float)(fam == 0 ? -log2e / (2.0 * l * l) : -log2e * root / l), ca = (float)(root / l);
+  // squared distance from which on a kernel value is subnormal; none where the distances themselves may be
+  const double reach = fam == 0 ? sqrt(126.0 / -(double)ce) : 126.0 / -(double)ce;
+  const float far2 = reach < 1e-16 ? -1.f : (float)(reach * reach);
   const float* P = static_cast<const float*>(op->a);
   const int S = rbf_slices(n);
   for (int b0 = 0; b0 < nrhs; b0 += kRbfNB) {
@@ -238,19 +278,19 @@ int rbf_apply(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, 
     switch (fam) {
       case 0:
         rbf_family<0>(op->dim, nb_t, grid, s, n, (int)op->dim, P, op->lda, ce, ca, Xb, ldx, Yb, ldy, nb, op->scale,
-                      op->shift, part, done);
+                      op->shift, far2, part, done);
         break;
       case 1:
         rbf_family<1>(op->dim, nb_t, grid, s, n, (int)op->dim, P, op->lda, ce, ca, Xb, ldx, Yb, ldy, nb, op->scale,
-                      op->shift, part, done);
+                      op->shift, far2, part, done);
         break;
       case 2:
         rbf_family<2>(op->dim, nb_t, grid, s, n, (int)op->dim, P, op->lda, ce, ca, Xb, ldx, Yb, ldy, nb, op->scale,
-                      op->shift, part, done);
+                      op->shift, far2, part, done);
         break;
       default:
         rbf_family<3>(op->dim, nb_t, grid, s, n, (int)op->dim, P, op->lda, ce, ca, Xb, ldx, Yb, ldy, nb, op->scale,
-                      op->shift, part, done);
+                      op->shift, far2, part, done);
         break;
     }
     if (split)

@@ -61,3 +61,36 @@ def test_stationary_product_repeats_bitwise(dev):
     X, V = torch.rand(3000, 3, generator=g).to(dev), torch.randn(3000, 4, generator=g).to(dev)
     A = ca.ops.Kernel(X, X, ca.ops.matern52(0.3), 1024, 1024)
     assert torch.equal(A @ V, A @ V)
+
+
+@pytest.mark.parametrize("fam", [0, 1, 2, 3])
+@pytest.mark.parametrize("dim,nrhs,n", [(1, 1, 203), (3, 4, 203), (3, 4, 600)])
+def test_stationary_subnormal_entries(dev, fam, dim, nrhs, n):
+    """Columns of K itself, from 2^-100 down to the last subnormal: the exponent t is rounded a few times at
+    |t| <= 110 (1e-5 of an entry), a subnormal once or twice by 2^-149."""
+    ell = 0.4
+    t = torch.linspace(70.0, 108.0, n - 1, dtype=torch.float64)  # -log of the exponential
+    root = 3.0**0.5 if fam == 2 else 5.0**0.5 if fam == 3 else 1.0
+    r = ell * ((2 * t).sqrt() if fam == 0 else t / root)
+    pts = torch.zeros(n, dim)
+    pts[1:, dim - 1] = r.float()
+    V = torch.zeros(n, nrhs)
+    V[0] = 1.0
+    ref, _ = reference(fam, pts.double(), V.double(), float(torch.tensor(ell)))
+    fn = (ca.ops.rbf, ca.ops.matern12, ca.ops.matern32, ca.ops.matern52)[fam](ell)
+    Pd = pts.to(dev)
+    out = (ca.ops.Kernel(Pd, Pd, fn, 1024, 1024) @ V.to(dev)).cpu().double()
+    assert bool(((out - ref).abs() <= 2e-5 * ref + 3e-45).all())
+    assert float((out[1:, 0] > 0).double().mean()) > 0.9 * float((ref[1:, 0] > 1.5e-45).double().mean())
+
+
+@pytest.mark.parametrize("fam", [1, 2, 3])
+def test_stationary_subnormal_distances(dev, fam):
+    """Squared distances around 1e-39, with a lengthscale to match."""
+    g = torch.Generator().manual_seed(fam)
+    pts, V, ell = torch.rand(300, 2, generator=g) * 6e-20, torch.randn(300, 2, generator=g), 3e-20
+    ref, mag = reference(fam, pts.double(), V.double(), float(torch.tensor(ell)))
+    fn = (None, ca.ops.matern12, ca.ops.matern32, ca.ops.matern52)[fam](ell)
+    Pd = pts.to(dev)
+    out = (ca.ops.Kernel(Pd, Pd, fn, 1024, 1024) @ V.to(dev)).cpu().double()
+    assert bool(((out - ref).abs() <= 1e-3 * mag).all())
