@@ -412,7 +412,7 @@ def bench_dense_cg(args, dev):
     from cola_amd.linalg._engine import lower
     from cola_amd.linalg.cg import _fused_buffers
     aop = lower(op)
-    state, work, _, _ = _fused_buffers(dev, 1024, 1, 1000)
+    state, work, *_ = _fused_buffers(dev, 1024, 1, 1000)
     xr = torch.empty((2, 1024, 1), dtype=torch.float32, device=dev)
     t_kernel = time_kernel(lambda: N.call("ck_cg_fused", aop[0], None, 1, N.ptr(bd), bd.stride(0), bd.stride(1), None, 0,
                                           0, N.ptr(xr[0]), 1, 1, N.ptr(xr[1]), 1, 1, N.ptr(state), 1e-6, 1000,
