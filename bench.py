@@ -37,7 +37,7 @@ HBM_PEAK = 8000.0  # GB/s
 # WRITE_SIZE (x1.0), the factors a 1 GiB stream copy reads on the same counters (profiles/kron64_cg_64cubed_hbm_traffic.md)
 PASS_A_TRAFFIC_BYTES = (16651.2 + 16222.7) * 1024
 FP32_MFMA_PEAK = 157.3  # TFLOP/s
-# HBM bytes per dense_lds_kernel<8,4> launch (16384^2 fp32 matrix, 8 rhs): rocprofv3 --pmc FETCH_SIZE (x2.0)
+# HBM bytes per dense_f32_lds_kernel<8,4> launch (16384^2 fp32 matrix, 8 rhs): rocprofv3 --pmc FETCH_SIZE (x2.0)
 # plus WRITE_SIZE (x1.0), the factors a 1 GiB stream copy reads on the same counters
 # (profiles/dense_matvec_16384x8_hbm_traffic.md)
 DENSE8_TRAFFIC_BYTES = (526427.07 * 2.0 + 512.42) * 1024
@@ -54,7 +54,7 @@ def dense_product_roof(op, n, B, t):
     mat = 4 * n * (n + 128) // 2 if sym else 4 * n * n
     nbytes = mat + 2 * 4 * n * B
     kernel = (f"dense_sym_kernel<8> + dense_sym_reduce<8> (upper 128-column strips, {B} rhs)" if sym
-              else f"dense_lds_kernel<8,4> ({B} rhs)")
+              else f"dense_f32_lds_kernel<8,4> ({B} rhs)")
     traffic = DENSE8_SYM_TRAFFIC_BYTES if sym else DENSE8_TRAFFIC_BYTES
     return {"bound": "hbm", "kernel": kernel, "achieved": nbytes / t / 1e9, "peak": HBM_PEAK, "unit": "GB/s",
             "frac": nbytes / t / 1e9 / HBM_PEAK, "traffic": traffic, "launch_us": t * 1e6,
@@ -438,7 +438,7 @@ def bench_dense_cg(args, dev):
             "roofline": {"bound": "hbm", "kernel": "fused_cg_kernel<1, 4, 2, true> (whole solve, A rows held in registers)",
                          "achieved": ach, "peak": HBM_PEAK, "unit": "GB/s", "frac": ach / HBM_PEAK, "traffic": None,
                          "algorithmic_bytes_per_step": step_bytes,
-                         "note": "latency-bound: one grid-wide exchange per step; A is read from LDS, not HBM"},
+                         "note": "latency-bound: one grid-wide exchange per step; A stays in registers"},
             "cpu_baseline": {"value": 1 / dto, "unit": "solves/s", "cores": cpu_threads(), "kind": "port",
                              "sample": f"{reps} full solves of the oracle's CG (fp32 torch) in 2 s"}}
 

@@ -4,9 +4,10 @@
 // ABI header).  Every reduction is two-level with a fixed order: each block of
 // (rhs b, chunk) writes one partial, and whoever needs the column total adds
 // that column's partials in index order (fp64).  A block of the x/r update
-// recomputes its own column's p.Ap from the partials, so no grid-wide barrier
-// or atomic is needed; the cross-column decisions (k, done, errors) are made by
-// a one-block kernel at the end of each step.
+// recomputes its own column's p.Ap from the partials, one of the p update its
+// column's beta, so no grid-wide barrier or atomic is needed; the cross-column
+// decisions (k, done, errors) are made by one more block of the p update's
+// launch (above 32 columns by a one-block kernel before it).
 #include "cg_state.hpp"
 #include "common.hpp"
 #include "ops_internal.hpp"
@@ -26,7 +27,7 @@ __host__ __device__ inline CgView view(void* state, int nrhs) { return cg_view(s
 // columns as used ones: the beta array's hold, during a step, what each column's beta divides by --
 // gamma before the step, infinity for a column that has converged (written by the x/r update).
 constexpr int kJoinRhs = 32;
-__device__ inline float* step_den(const CgView& v, int nrhs) { return v.beta + kJoinRhs; }
+__device__ inline float* step_den(const CgView& v) { return v.beta + kJoinRhs; }
 
 inline int nparts_of(int64_t n) {
   int64_t p = cdiv(n, kChunk);
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(256) void update_xr_kernel(int64_t n, const float* 
   const float alpha = (float)a;
   if (blk == 0 && threadIdx.x == 0) {
     v.alpha[b] = alpha;
-    if (nrhs <= kJoinRhs) step_den(v, nrhs)[b] = frozen ? INFINITY : v.gamma[b];
+    if (nrhs <= kJoinRhs) step_den(v)[b] = frozen ? INFINITY : v.gamma[b];
     // the reference divides on regardless; the status records it (same value from every writer)
     if (!frozen && !(pap > 0.0) && v.ctrl->status == CK_OK) v.ctrl->status = CK_ERR_BREAKDOWN;
   }
@@ -429,7 +430,7 @@ __global__ __launch_bounds__(256) void update_p_kernel(int64_t n, const float* _
                                                        void* state, int nrhs) {
   CgView v = view(state, nrhs);
   if (JOINED && blockIdx.x == 0) {
-    if (blockIdx.y == 0 && !v.ctrl->done) step_scalars(v, nrhs, part1, part2, P, precond, step_den(v, nrhs));
+    if (blockIdx.y == 0 && !v.ctrl->done) step_scalars(v, nrhs, part1, part2, P, precond, step_den(v));
     return;
   }
   const int b = blockIdx.y;
@@ -448,7 +449,7 @@ __global__ __launch_bounds__(256) void update_p_kernel(int64_t n, const float* _
   }
   float beta;
   if (JOINED) {
-    const float den = step_den(v, nrhs)[b];
+    const float den = step_den(v)[b];
     __shared__ double dred[4];
     const float* part = precond ? part2 : part1;
     const double rz = P > kWavePartials ? column_total_block(part, P, b, dred) : column_total(part, P, b);
@@ -710,7 +711,7 @@ __global__ __launch_bounds__(256) void wbf_xr_kernel(int64_t n, int nrhs, const 
       alpha_s[b] = (float)a;
       if (tile == 0) {
         v.alpha[b] = (float)a;
-        if (nrhs <= kJoinRhs) step_den(v, nrhs)[b] = frozen ? INFINITY : v.gamma[b];
+        if (nrhs <= kJoinRhs) step_den(v)[b] = frozen ? INFINITY : v.gamma[b];
         if (!frozen && !(pap_b > 0.0) && v.ctrl->status == CK_OK) v.ctrl->status = CK_ERR_BREAKDOWN;
       }
     }
@@ -887,7 +888,7 @@ __global__ __launch_bounds__(256) void wbf_z_kernel(int64_t n, int nrhs, const f
   }
 }
 
-bool wb_fused_ok(const ck_op* A, const ck_op* P, int nrhs, const float* p, int64_t ld, size_t work_bytes) {
+bool wb_fused_ok(const ck_op* A, const ck_op* P, int nrhs, size_t work_bytes) {
   return P && A->kind == CK_OP_DENSE_F32 && P->kind == CK_OP_WOODBURY_INV && nrhs >= 3 && nrhs <= 8 &&
          P->rank >= 1 && P->rank <= 64 && P->lda >= P->rank && P->a && P->aux &&
          work_bytes >= wb_fused_bytes(A->n, nrhs, P->rank);
@@ -917,7 +918,7 @@ int cg_iterate(const ck_op* A, const ck_op* P, int32_t nrhs, float* x, float* r,
   const bool fuse_eig = P && P->kind == CK_OP_KRON_EIG_F32 && q.P == 64 && q.per == 4096 &&
                         kron64_eligible(P, r, ld, z, ld);
   // dense A with a Woodbury P: the fused step (dense_apply_xy, wbf_*) in P's workspace
-  const bool fuse_wb = !fuse_kron && wb_fused_ok(A, P, nrhs, p, ld, work_bytes);
+  const bool fuse_wb = !fuse_kron && wb_fused_ok(A, P, nrhs, work_bytes);
   const bool dense_xy = !fuse_kron && !fuse_wb && A->kind == CK_OP_DENSE_F32 && nrhs >= 3 && nrhs <= 8 && work &&
                         work_bytes >= dense_xy_bytes(n, nrhs);
   // CSR A: p.Ap partials from the SpMV's epilogue, into

@@ -1023,8 +1023,8 @@ constexpr int kF64NB = 8;  // rhs per pass
 // Every load is unconditional (rows and columns clamped, the extra terms multiplied by zero) and
 // the x chunk staged once per block for all of its rows: eight waves of four rows share one FP64 copy
 // of X[:, c0:c0+512) in LDS; A is streamed with non-temporal 16-byte loads, which need dword
-// alignment only, so odd orders and leading dimensions take the same path (12289 x 8: 1616 -> 164 us against one column per lane); the
-// last n % 4 columns are added one per lane.
+// alignment only, so odd orders and leading dimensions take the same path (12289 x 8: 1616 -> 164 us
+// against one column per lane); the last n % 4 columns are added one per lane.
 constexpr int kF64Chunk = 512;
 constexpr int kF64Waves = 8;
 typedef float f64acc_f4 __attribute__((ext_vector_type(4), aligned(4)));

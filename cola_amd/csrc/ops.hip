@@ -2,9 +2,10 @@
 //
 //   dense  : each wavefront owns ROWS rows; lanes stride the row in float4 chunks,
 //            one DPP wave reduction per (row, rhs).            [HBM / L2 bound]
-//   csr    : one lane per row, short rows batched into registers (short rows) or
-//            one wavefront per row (long rows);
-//            int32 column indices; coalesced rowptr/value streams. [HBM bound]
+//   csr    : by the average row: one lane per row up to 8 entries, 4 lanes (8 at eight rhs, 16
+//            at one rhs above 64) up to 128, a wave above; rows far longer than their group's
+//            share by the whole wave; int32 column indices. [HBM; bound by the gathers where
+//            columns scatter]
 //   kron   : factors of order <= 64, in kron.hip (64^3) and kron_any.hip.
 #include "common.hpp"
 #include "ops_internal.hpp"

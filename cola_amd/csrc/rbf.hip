@@ -7,13 +7,15 @@
 //   - dimension and rhs count are template parameters (nothing is padded to 8 of either);
 //   - exp is one v_exp_f32 on an argument scaled once: log2(e) and the lengthscale are folded
 //     into one constant in FP64, so the argument sees fewer roundings than l, 1/l, sqrt(k)/l * r
-//     and the exponential's own range reduction would give it; sqrt is one v_sqrt_f32 (1 ulp);
+//     and the exponential's own range reduction would give it; sqrt is one v_sqrt_f32 (1 ulp).
+//     Both take subnormals for zero: four columns at a time are looked over for entries that far
+//     out, which then go a longer way together (one maximum an entry, 0 to 5 % of the time);
 //   - a lane owns two rows, so a staged point and its x (one or two 16-byte LDS broadcasts) serve
 //     two entries; the four waves of a block share the rows and split each staged tile of 256
 //     columns, and the columns are also split over blockIdx.y until the grid fills the chip
 //     (a workspace holds one partial per column slice, added in slice order).
 // Measured, 20000 points in 3-D, Matern 5/2, 4 rhs: 4242 us with one row per lane, 79 blocks and
-// the library's expf and sqrtf; now 210 us per call (the transposes and the host included).
+// the library's expf and sqrtf; now 183 us per call (the transposes and the host included).
 #include <type_traits>
 
 #include "common.hpp"
@@ -30,8 +32,8 @@ constexpr int kRbfMaxDim = 8;
 constexpr int kRbfNB = 8;       // rhs per pass
 constexpr int kRbfMaxSlices = 32;
 // Blocks wanted: twice what the chip holds at once (256 CUs x 8 blocks of four waves), so that the
-// last wave of blocks is a small part of the run (case above: 512 blocks 262 us, 1024 240 us,
-// 2048 218 us, 4096 210 us with the host's share).
+// last wave of blocks is a small part of the run (case above by wall clock, an earlier form of
+// the kernel: 512 blocks 262 us, 1024 240 us, 2048 218 us, 4096 210 us).
 constexpr int kRbfBlocks = 4096;
 
 // The stationary kernel of the squared distance d2: FAMILY 0 exp(-d2 / (2 l^2)) (RBF), 1 exp(-r / l)
