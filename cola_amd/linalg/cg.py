@@ -8,7 +8,6 @@ to an engine kernel, otherwise step by step around ``A._matmat``) and reads
 the 8-byte control block once per chunk instead of syncing twice per step
 (cola/utils/torch_tqdm.py:42,88).
 """
-import contextlib
 import threading
 import time
 from dataclasses import dataclass
@@ -130,23 +129,21 @@ class _Workgroups:
     def __init__(self, total):
         self.total, self.used, self.changed = total, 0, threading.Condition()
 
-    @contextlib.contextmanager
-    def hold(self, count):
-        """Whether there was room: yields True with `count` workgroups held, else False."""
+    def take(self, count):
+        """Whether there was room: True with `count` more workgroups in use."""
         with self.changed:
-            held = self.changed.wait_for(lambda: self.used + count <= self.total, self.PATIENCE)
-            self.used += count if held else 0
-        try:
-            yield held
-        finally:
-            if held:
-                with self.changed:
-                    self.used -= count
-                    self.changed.notify_all()
+            room = self.used + count <= self.total or self.changed.wait_for(
+                lambda: self.used + count <= self.total, self.PATIENCE)
+            self.used += count if room else 0
+        return room
+
+    def give(self, count):
+        with self.changed:
+            self.used -= count
+            self.changed.notify_all()
 
 
 _WORKGROUPS = {}
-_ALONE = contextlib.nullcontext(True)  # one workgroup waits for nobody
 
 
 def _workgroups(dev):
@@ -183,16 +180,21 @@ def fused_solve(A, b, x0=None, max_iters=1000, tol=1e-6, P=None, nblocks=0, spin
         x0f = x0f if x0f.dtype == torch.float32 else x0f.float()
     t0 = time.time()
     stream = torch.cuda.current_stream(dev)
-    with lock, (gate.hold(count) if count > 1 else _ALONE) as held:
-        if not held:
+    with lock:
+        held = count if count > 1 else 0  # one workgroup waits for nobody
+        if held and not gate.take(held):
             return None
-        N.call("ck_cg_fused", aop[0], pop[0] if pop else None, B, N.ptr(bf), bf.stride(0), bf.stride(1), N.ptr(x0f),
-               x0f.stride(0) if x0f is not None else 0, x0f.stride(1) if x0f is not None else 0, N.ptr(x), x.stride(0),
-               x.stride(1), N.ptr(r), r.stride(0), r.stride(1), N.ptr(state), float(tol), int(max_iters), N.ptr(work),
-               work.numel() * 8, int(nblocks), int(spin_limit), int(wait_offset), int(bool(cooperative)),
-               N.stream_ptr(dev))
-        host.copy_(state, non_blocking=True)
-        stream.synchronize()
+        try:
+            N.call("ck_cg_fused", aop[0], pop[0] if pop else None, B, N.ptr(bf), bf.stride(0), bf.stride(1),
+                   N.ptr(x0f), x0f.stride(0) if x0f is not None else 0, x0f.stride(1) if x0f is not None else 0,
+                   N.ptr(x), x.stride(0), x.stride(1), N.ptr(r), r.stride(0), r.stride(1), N.ptr(state), float(tol),
+                   int(max_iters), N.ptr(work), work.numel() * 8, int(nblocks), int(spin_limit), int(wait_offset),
+                   int(bool(cooperative)), N.stream_ptr(dev))
+            host.copy_(state, non_blocking=True)
+            stream.synchronize()
+        finally:
+            if held:
+                gate.give(held)
         ctrl = host[:N.CTRL_BYTES].view(torch.int32)
         k, status = int(ctrl[0]), int(ctrl[5])
         if status == N.CK_ERR_TIMEOUT:

@@ -56,7 +56,8 @@ def engine(monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_stream", lambda dev=None: Stream())
     monkeypatch.setattr(N, "stream_ptr", lambda dev=None: None)
     monkeypatch.setattr(N, "call", call)
-    monkeypatch.setattr(N, "q", lambda name, *a: ENGINE["workgroups"] if name == "ck_cg_fused_workgroups" else query(name, *a))
+    monkeypatch.setattr(N, "q", lambda name, *a: ENGINE["workgroups"]
+                        if name == "ck_cg_fused_workgroups" else query(name, *a))
     monkeypatch.setattr(cgmod, "lower", lambda A: (None, ))
     monkeypatch.setattr(cgmod, "_WORKGROUPS", {None: cgmod._Workgroups(256)})
     ENGINE.update(workgroups=1, running=0, most=0)
