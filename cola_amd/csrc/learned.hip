@@ -1020,10 +1020,10 @@ __global__ __launch_bounds__(256) void rbf_dense_kernel(int n, int dim, const fl
 // ------------------------------------------------------- dense apply, fp64 vectors
 constexpr int kF64NB = 8;  // rhs per pass
 
-// Every load is unconditional (rows and columns clamped, the extra terms multiplied by zero) and
+// Every load is unconditional (rows and columns clamped, the extra terms left out) and
 // the x chunk staged once per block for all of its rows: eight waves of four rows share one FP64 copy
 // of X[:, c0:c0+512) in LDS; A is streamed with non-temporal 16-byte loads, which need dword
-// alignment only, so odd orders and leading dimensions take the same path (12289 x 8: 1616 -> 164 us
+// alignment only, so odd orders and leading dimensions take the same path (12289 x 8: 1616 -> 141 us
 // against one column per lane); the last n % 4 columns are added one per lane.
 constexpr int kF64Chunk = 512;
 constexpr int kF64Waves = 8;
@@ -1044,14 +1044,9 @@ __global__ __launch_bounds__(64 * kF64Waves) __attribute__((amdgpu_waves_per_eu(
   for (int r = 0; r < 4; ++r)
 #pragma unroll
     for (int b = 0; b < kF64NB; ++b) acc[r][b] = 0.0;
-  const float* arow[4];
-  float rmask[4];
+  const float* arow[4];  // rows past the last: its copy, never stored
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = row0 + r < n ? row0 + r : n - 1;
-    arow[r] = A + (int64_t)row * lda;
-    rmask[r] = row0 + r < n ? 1.f : 0.f;
-  }
+  for (int r = 0; r < 4; ++r) arow[r] = A + (int64_t)(row0 + r < n ? row0 + r : n - 1) * lda;
   const int n4 = n & ~3;
   for (int c0 = 0; c0 < n4; c0 += kF64Chunk) {
     const int cn = n4 - c0 < kF64Chunk ? n4 - c0 : kF64Chunk;  // a multiple of 4
@@ -1067,24 +1062,23 @@ __global__ __launch_bounds__(64 * kF64Waves) __attribute__((amdgpu_waves_per_eu(
     for (int q = 0; q < kF64Chunk / 256; ++q) {
       const int j = q * 256 + lane * 4;
       const int jc = j < cn ? j : cn - 4;  // clamped: the load stays unconditional
-      float4 a[4];
+      f64acc_f4 a[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const f64acc_f4 v = __builtin_nontemporal_load(reinterpret_cast<const f64acc_f4*>(arow[r] + c0 + jc));
-        const float m = j < cn ? rmask[r] : 0.f;
-        a[r] = make_float4(v.x * m, v.y * m, v.z * m, v.w * m);
-      }
+      for (int r = 0; r < 4; ++r) a[r] = __builtin_nontemporal_load(reinterpret_cast<const f64acc_f4*>(arow[r] + c0 + jc));
+      // no product with zero instead: the row's last entries, read again, need not be finite
+      if (j < cn) {
 #pragma unroll
-      for (int b = 0; b < kF64NB; ++b) {
-        const double2 x0 = xs[b][jc / 2], x1 = xs[b][jc / 2 + 1];
+        for (int b = 0; b < kF64NB; ++b) {
+          const double2 x0 = xs[b][j / 2], x1 = xs[b][j / 2 + 1];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          double t = acc[r][b];
-          t = fma((double)a[r].x, x0.x, t);
-          t = fma((double)a[r].y, x0.y, t);
-          t = fma((double)a[r].z, x1.x, t);
-          t = fma((double)a[r].w, x1.y, t);
-          acc[r][b] = t;
+          for (int r = 0; r < 4; ++r) {
+            double t = acc[r][b];
+            t = fma((double)a[r][0], x0.x, t);
+            t = fma((double)a[r][1], x0.y, t);
+            t = fma((double)a[r][2], x1.x, t);
+            t = fma((double)a[r][3], x1.y, t);
+            acc[r][b] = t;
+          }
         }
       }
     }

@@ -55,6 +55,28 @@ def test_dense_f64acc_any_alignment(dev, n, pad, off, nrhs):
     assert float((Yb[:, :n].T.cpu() - ref).norm() / ref.norm()) < 1e-14
 
 
+@pytest.mark.parametrize("n", [3, 131, 257, 513, 516, 1030])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_dense_products_infinite_entry(dev, n, dtype):
+    """An infinite entry in any column of its row, everything else positive: that row is infinite (and no NaN),
+    the others finite, at one and several rhs (lanes past a row's end may read its last entries again)."""
+    for col in {0, n - 1, n // 2, max(n - 4, 0), n - n % 4 - 1}:
+        A = torch.rand(n, n, device=dev) + 0.1
+        A[n - 2, col] = float("inf")
+        for nrhs in (1, 2, 5, 8):
+            X = torch.rand(n, nrhs, device=dev, dtype=dtype) + 0.1
+            if dtype == torch.float32:
+                Y = ca.Dense(A) @ X
+            else:
+                Xb, Yb = X.T.contiguous(), torch.empty(nrhs, n, device=dev, dtype=dtype)
+                N.call("ck_dense_apply_f64acc", n, N.ptr(A), n, 1.0, 0.0, nrhs, N.ptr(Xb), n, N.ptr(Yb), n,
+                       N.stream_ptr(dev))
+                Y = Yb.T
+            hit = torch.zeros_like(Y, dtype=torch.bool)
+            hit[n - 2] = True
+            assert bool((torch.isposinf(Y) == hit).all()) and bool((torch.isfinite(Y) == ~hit).all()), (col, nrhs)
+
+
 @pytest.mark.parametrize("n,nrhs", [(2047, 4), (2049, 3), (4099, 8), (8201, 5)])
 def test_cg_on_odd_orders(dev, n, nrhs):
     """Chained CG with p . Ap from the dense epilogue, and the fused Woodbury step of a refined solve."""
