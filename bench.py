@@ -40,10 +40,10 @@ FP32_MFMA_PEAK = 157.3  # TFLOP/s
 # HBM bytes per dense_f32_lds_kernel<8,4> launch (16384^2 fp32 matrix, 8 rhs): rocprofv3 --pmc FETCH_SIZE (x2.0)
 # plus WRITE_SIZE (x1.0), the factors a 1 GiB stream copy reads on the same counters
 # (profiles/dense_matvec_16384x8_hbm_traffic.md)
-DENSE8_TRAFFIC_BYTES = (526427.07 * 2.0 + 512.42) * 1024
+DENSE8_TRAFFIC_BYTES = (526424.10 * 2.0 + 512.13) * 1024
 # HBM bytes per symmetric 8-rhs product (dense_sym_kernel<8> + dense_sym_reduce<8>) on the same matrix,
 # same counters and factors (profiles/dense_sym_matvec_16384x8_hbm_traffic.md)
-DENSE8_SYM_TRAFFIC_BYTES = ((266583.10 + 19071.09) * 2.0 + (37650.49 + 512.0)) * 1024
+DENSE8_SYM_TRAFFIC_BYTES = ((266626.35 + 18589.0) * 2.0 + (36925.76 + 512.0)) * 1024
 
 
 def dense_product_roof(op, n, B, t):

@@ -107,7 +107,7 @@ __device__ __forceinline__ floatx4 load4(const float* __restrict__ p, int left) 
 // 64 made 16, and with 64 points on the matrix units larger sets run no faster either (16384 points 22.6
 // against 27.0 us, 131072 123 against 124: the weights a block reads come from L2).  The activations are
 // rolled loops over LDS: a launch runs its code once, from cold instruction caches.  1024 points: 40.4
-// us with 64 points per block on the vector units, now 8.8; 16384: 46.8 -> 22.6 us.
+// us with 64 points per block on the vector units, now 8.6; 16384: 46.8 -> 20.2 us.
 constexpr int kFwdRows = 16;
 
 template <bool SAVE>
