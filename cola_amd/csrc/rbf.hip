@@ -264,8 +264,9 @@ int rbf_apply(const ck_op* op, int nrhs, const float* X, int64_t ldx, float* Y, 
   const double l = (double)op->aux_f, log2e = 1.4426950408889634;
   const double root = fam == 2 ? sqrt(3.0) : fam == 3 ? sqrt(5.0) : 1.0;
   const float ce = (float)(fam == 0 ? -log2e / (2.0 * l * l) : -log2e * root / l), ca = (float)(root / l);
-  // squared distance from which on a kernel value is subnormal; none where the distances themselves may be
-  const double reach = fam == 0 ? sqrt(126.0 / -(double)ce) : 126.0 / -(double)ce;
+  // squared distance from which on an exponential may be subnormal (below 2^-126, and a margin for the
+  // rounding of either side); all where the distances themselves may be
+  const double reach = fam == 0 ? sqrt(125.5 / -(double)ce) : 125.5 / -(double)ce;
   const float far2 = reach < 1e-16 ? -1.f : (float)(reach * reach);
   const float* P = static_cast<const float*>(op->a);
   const int S = rbf_slices(n);

@@ -1,6 +1,8 @@
 """The on-the-fly stationary kernel product (CK_OP_RBF_F32) at the edges of its tiles: 128 rows per
 block, 256 columns per staged tile split over four waves, up to 8 rhs per pass, dimensions rounded
 up to a template size, with the columns split over blocks (workspace) and not (none)."""
+import math
+
 import pytest
 import torch
 
@@ -70,6 +72,7 @@ def test_stationary_subnormal_entries(dev, fam, dim, nrhs, n):
     |t| <= 110 (1e-5 of an entry), a subnormal once or twice by 2^-149."""
     ell = 0.4
     t = torch.linspace(70.0, 108.0, n - 1, dtype=torch.float64)  # -log of the exponential
+    t[:80] = 126 * math.log(2) * (1 + torch.linspace(-2e-6, 2e-6, 80, dtype=torch.float64))  # around the last normal one
     root = 3.0**0.5 if fam == 2 else 5.0**0.5 if fam == 3 else 1.0
     r = ell * ((2 * t).sqrt() if fam == 0 else t / root)
     pts = torch.zeros(n, dim)
@@ -81,6 +84,7 @@ def test_stationary_subnormal_entries(dev, fam, dim, nrhs, n):
     Pd = pts.to(dev)
     out = (ca.ops.Kernel(Pd, Pd, fn, 1024, 1024) @ V.to(dev)).cpu().double()
     assert bool(((out - ref).abs() <= 2e-5 * ref + 3e-45).all())
+    assert bool((out[1:81] > 0).all(dim=0)[0])
     assert float((out[1:, 0] > 0).double().mean()) > 0.9 * float((ref[1:, 0] > 1.5e-45).double().mean())
 
 
