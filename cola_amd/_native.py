@@ -130,6 +130,7 @@ _PROTOS = {
     "ck_cg_fused_workspace_bytes": (_sz, [_i64, _i32]),
     "ck_cg_fused_supported": (ctypes.c_int, [_op, _op, _i32]),
     "ck_cg_fused_workgroups": (_i32, [_op, _op, _i32, _i32, _i32]),
+    "ck_device_cus": (_i32, [_i32]),
     "ck_cg_fused_noalloc": (ctypes.c_int, [_op, _op, _i32, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _i64,
                                            _i64, _p, _f32, _i32, _i32, _i64, _i32, _i32, _p]),
     "ck_cg_fused_noalloc_max_bytes": (_sz, []),

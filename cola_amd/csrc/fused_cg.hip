@@ -972,6 +972,11 @@ int32_t ck_cg_fused_workgroups(const ck_op* A, const ck_op* P, int32_t nrhs, int
   return !p.ok ? 0 : one_workgroup(A->n, nrhs, nblocks, wait_offset) ? 1 : p.G;
 }
 
+int32_t ck_device_cus(int32_t device) {
+  int cus = 0;
+  return hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess ? cus : 0;
+}
+
 int ck_cg_fused(const ck_op* A, const ck_op* P, int32_t nrhs, const float* b, int64_t b_rs, int64_t b_cs,
                 const float* x0, int64_t x0_rs, int64_t x0_cs, float* x, int64_t x_rs, int64_t x_cs, float* r,
                 int64_t r_rs, int64_t r_cs, void* state, float tol, int32_t max_iters, void* work,

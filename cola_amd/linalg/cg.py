@@ -123,8 +123,9 @@ class _Workgroups:
     """Bound on the workgroups of persistent solves in flight on one device.  The workgroups of a solve
     wait for one another's words inside the kernel, so those of concurrent threads have to fit the
     device together, one per CU.  A solve that finds no room waits for others' solves (0.1 to some ms
-    each), but not for whatever else their streams were given first: after 20 ms it goes without."""
-    PATIENCE = 0.02
+    each, 5 for a process's first), but not for whatever else their streams were given first: after
+    50 ms it goes without."""
+    PATIENCE = 0.05
 
     def __init__(self, total):
         self.total, self.used, self.changed = total, 0, threading.Condition()
@@ -149,8 +150,7 @@ _WORKGROUPS = {}
 def _workgroups(dev):
     gate = _WORKGROUPS.get(dev.index)
     if gate is None:
-        cus = torch.cuda.get_device_properties(dev).multi_processor_count
-        gate = _WORKGROUPS.setdefault(dev.index, _Workgroups(cus))
+        gate = _WORKGROUPS.setdefault(dev.index, _Workgroups(N.q("ck_device_cus", dev.index)))
     return gate
 
 

@@ -325,6 +325,8 @@ int ck_cg_fused_supported(const ck_op* A, const ck_op* P, int32_t nrhs);
 /* Workgroups that such a call launches (0: not supported), for callers that keep concurrent solves
  * within the device.  No counterpart in the reference. */
 int32_t ck_cg_fused_workgroups(const ck_op* A, const ck_op* P, int32_t nrhs, int32_t nblocks, int32_t wait_offset);
+/* Compute units of a device (0: no such device). */
+int32_t ck_device_cus(int32_t device);
 int ck_cg_fused(const ck_op* A, const ck_op* P, int32_t nrhs, const float* b, int64_t b_rs, int64_t b_cs,
                 const float* x0, int64_t x0_rs, int64_t x0_cs, float* x, int64_t x_rs, int64_t x_cs, float* r,
                 int64_t r_rs, int64_t r_cs, void* state, float tol, int32_t max_iters, void* work,

@@ -123,6 +123,10 @@ def test_earlier_work_of_a_stream_holds_up_nobody(engine):
     assert done["busy"][0] - t0 >= 1.0 and done["busy"][1] and cgmod._WORKGROUPS[None].used == 0
 
 
+def test_devices_cus():
+    assert N.q("ck_device_cus", -1) == 0 and N.q("ck_device_cus", 1000) == 0
+
+
 def test_more_workgroups_than_the_device_has(engine):
     cgmod._WORKGROUPS[None] = cgmod._Workgroups(32)
     ENGINE["workgroups"] = 33

@@ -1,6 +1,7 @@
 """The persistent CG over several workgroups (rows in registers up to 3584 unknowns, read in every step
 above) at the edges of its chunks of 512 columns, 16 or 20 rows a workgroup and 1 / 4 / 8 columns,
 against FP64 and the chained launches; and concurrent solves of several threads."""
+import importlib
 import threading
 
 import pytest
@@ -72,6 +73,7 @@ def test_threads(dev):
     A, g = system(dev, n, 5)
     bs = [torch.randn(n, 2, generator=g, device=dev) for _ in range(8)]
     sol = torch.linalg.solve(A.double(), torch.cat(bs, 1).double())
+    importlib.import_module("cola_amd.linalg.cg")._WORKGROUPS.clear()  # all threads ask for the device's CUs at once
     torch.cuda.synchronize()
 
     def work(i):
