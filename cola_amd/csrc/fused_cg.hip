@@ -974,7 +974,9 @@ int32_t ck_cg_fused_workgroups(const ck_op* A, const ck_op* P, int32_t nrhs, int
 
 int32_t ck_device_cus(int32_t device) {
   int cus = 0;
-  return hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess ? cus : 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess) return cus;
+  (void)hipGetLastError();  // not the next launch's error
+  return 0;
 }
 
 int ck_cg_fused(const ck_op* A, const ck_op* P, int32_t nrhs, const float* b, int64_t b_rs, int64_t b_cs,
